@@ -390,7 +390,48 @@ void fft3d(Context& ctx, c2<T>* data, const Loader& load, int sign,
 
 // Pruning descriptor for an inverse transform whose input vanishes for
 // |k| >= k_hi (disabled when the band covers the whole kx range).
-Prune make_prune(const Geom& g, double k_hi);
+inline Prune make_prune(const Geom& g, double k_hi) {
+  Prune pr{};
+  pr.on = 0;
+  const double kcut2 = k_hi * k_hi * (1. + 1.e-9);
+  // Worth it only if the band leaves part of the (kx, ky) plane empty.
+  const double kx_max = (g.n[0] / 2) * g.dk[0];
+  const double ky_max = (g.n[1] / 2) * g.dk[1];
+  if (kx_max * kx_max + ky_max * ky_max < kcut2) return pr;
+  pr.on = 1;
+  pr.kcut2 = kcut2;
+  pr.dk0 = g.dk[0];
+  pr.dk1 = g.dk[1];
+  pr.n0 = g.n[0];
+  pr.n1 = g.n[1];
+  return pr;
+}
+
+// Shell fields of a real source field are real for m = 0 and even l (the
+// spectrum y_l0(k^) f(k) / W(k) is Hermitian).
+inline bool real_shells(int ell, int m) { return m == 0 && ell % 2 == 0; }
+
+// Shell fields of (ell, m) for `bins` and j_l-weighted shell fields (see
+// engine_fft.hpp).
+template <typename T>
+void shell_slab_ifft(Context& ctx, c2<T>* base, const double2* src,
+                     const trvg_binning& kb, const std::vector<int>& bins,
+                     const std::vector<int>& nmodes, int ell, int m, bool packed);
+template <typename T>
+void sjl_slab_ifft(Context& ctx, c2<T>* base, const double2* src, const Spline& sp,
+                   const std::vector<double>& r, const std::vector<int>& bins, int ell,
+                   int m, bool packed);
+
+// Batched transforms over work lists (engine_fft.hpp).
+template <typename T>
+void shell_slab_work(const Geom& g, const trvg_binning& kb, int nbins,
+                     int nfield_groups, bool packed, std::vector<ShellBand>& bands,
+                     std::vector<double>& kcut2, std::vector<int2>& wz,
+                     std::vector<int2>& wy, std::vector<int2>& wx);
+template <typename T, class BatchLoader>
+void fft3d_batch(Context& ctx, c2<T>* base, const BatchLoader& load, int sign,
+                 bool prune, const double* kcut2, const int2* wz, int nz,
+                 const int2* wy, int ny, const int2* wx, int nx);
 
 // Zero `mesh` and assign catalogue `c` with weight mode (WeightMode) and
 // scale through the production (tile-binned) path.

@@ -22,17 +22,6 @@
 
 namespace trvg {
 
-// Declared in engine_drivers.hip.
-template <typename T>
-void shell_slab_work(const Geom& g, const trvg_binning& kb, int nbins,
-                     int nfield_groups, bool packed, std::vector<ShellBand>& bands,
-                     std::vector<double>& kcut2, std::vector<int2>& wz,
-                     std::vector<int2>& wy, std::vector<int2>& wx);
-template <typename T, class BatchLoader>
-void fft3d_batch(Context& ctx, c2<T>* base, const BatchLoader& load, int sign,
-                 bool prune, const double* kcut2, const int2* wz, int nz,
-                 const int2* wy, int ny, const int2* wx, int nx);
-
 namespace {
 
 struct Term {

@@ -18,895 +18,9 @@
 #include <tuple>
 #include <type_traits>
 
-#include "batch_kernels.hpp"
-#include "diff_kernels.hpp"
 #include "engine.hpp"
 
 namespace trvg {
-
-// ---------------------------------------------------------------------------
-// FFT
-// ---------------------------------------------------------------------------
-
-template <typename T>
-static const c2<T>* twiddles(int n, int sign);
-
-// Twiddles of a transform in context ctx: borrowed tables where the context
-// has them, else the engine's cache.
-template <typename T>
-static const c2<T>* ctx_twiddles(const Context& ctx, int n, int sign) {
-  int lg = 0;
-  while ((1 << lg) < n) lg++;
-  const void* b = (lg < 11 && (1 << lg) == n) ? ctx.tw[sign > 0 ? 1 : 0][lg] : nullptr;
-  return b ? static_cast<const c2<T>*>(b) : twiddles<T>(n, sign);
-}
-
-template <typename T>
-static const c2<T>* twiddles(int n, int sign) {
-  static std::mutex mu;
-  static std::map<std::tuple<int, int, int>, c2<T>*> cache;
-  int dev = 0;
-  TRVG_HIP(hipGetDevice(&dev));
-  auto key = std::make_tuple(dev, n, sign);
-  std::lock_guard<std::mutex> lk(mu);
-  auto it = cache.find(key);
-  if (it != cache.end()) return it->second;
-  std::vector<c2<T>> h(n);
-  for (int m = 0; m < n; m++) {
-    double a = 2. * M_PI * double(m) / double(n);
-    h[m] = mk<T>(T(std::cos(a)), T(sign * std::sin(a)));
-  }
-  c2<T>* d = nullptr;
-  TRVG_HIP(hipMalloc(&d, n * sizeof(c2<T>)));
-  TRVG_HIP(hipMemcpy(d, h.data(), n * sizeof(c2<T>), hipMemcpyHostToDevice));
-  cache[key] = d;
-  return d;
-}
-
-
-template <typename T, int LOGN>
-static size_t fft_smem(bool row_flags) {
-  constexpr int N = 1 << LOGN;
-  constexpr int NL = FFT_THREADS * FftEpt<T>::v / N;
-  // Lines, twiddles, then (strided passes) one byte per row of pruning flags.
-  return size_t(NL * (N + 1) + N) * sizeof(c2<T>) + (row_flags ? N : 0);
-}
-
-// The register-resident z pass for FP32 meshes of 256 and 512 with loaders
-// that only read (the masked rows of shell transforms, plain transforms):
-// measured faster there.  FP64 passes and loaders with per-cell arithmetic
-// keep the LDS-staged pass, whose lower register use keeps more waves
-// resident.
-template <class Loader> struct ZRegLoader : std::false_type {};
-template <> struct ZRegLoader<LoadMaskedZBatch<float>> : std::true_type {};
-template <> struct ZRegLoader<LoadSame<float>> : std::true_type {};
-
-template <typename T, int LOGN, class Loader>
-constexpr bool use_zreg() {
-  return ZRegShape<LOGN>::ok && sizeof(T) == 4 && ZRegLoader<Loader>::value;
-}
-
-template <typename T, int LOGN, class Loader>
-static void launch_z(Context& ctx, c2<T>* data, const Loader& load, int sign,
-                     double read_bytes, double write_bytes, const Prune& pr) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const long long nblocks = ctx.g.nmesh / E;
-  const size_t smem = fft_smem<T, LOGN>(false);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, read_bytes + write_bytes);
-  if constexpr (use_zreg<T, LOGN, Loader>()) {
-    static_assert(E == zreg_block<T>(), "z pass block size");
-    hipLaunchKernelGGL((fft_pass_z_reg<T, LOGN, Loader>), dim3(unsigned(nblocks)),
-                       dim3(zreg_threads<T, LOGN>()), (zreg_smem<T, LOGN>()), ctx.stream, data,
-                       load, tw, ctx.g.n[1], sign, pr);
-  } else if (ctx.g.n[1] % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_z<T, LOGN, EPT, true, Loader>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, load, tw,
-                       ctx.g.n[1], sign, pr);
-  else
-    hipLaunchKernelGGL((fft_pass_z<T, LOGN, EPT, false, Loader>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, load, tw,
-                       ctx.g.n[1], sign, pr);
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T, int LOGN>
-static void launch_strided(Context& ctx, c2<T>* data, long long S,
-                           long long outer_stride, long long inner, int sign,
-                           const Prune& pr, int prune_mode, double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const long long nblocks = ctx.g.nmesh / E;
-  const size_t smem = fft_smem<T, LOGN>(true);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (inner % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_strided<T, LOGN, EPT, true>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, tw, S, outer_stride,
-                       inner, sign, pr, prune_mode);
-  else
-    hipLaunchKernelGGL((fft_pass_strided<T, LOGN, EPT, false>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, tw, S, outer_stride,
-                       inner, sign, pr, prune_mode);
-  TRVG_LAUNCH_CHECK();
-}
-
-static int ilog2(int n) {
-  int l = 0;
-  while ((1 << l) < n) l++;
-  return l;
-}
-
-#define TRVG_LOGN_SWITCH(lg, CALL)                               \
-  switch (lg) {                                                  \
-    case 3: { constexpr int LG = 3; CALL; } break;               \
-    case 4: { constexpr int LG = 4; CALL; } break;               \
-    case 5: { constexpr int LG = 5; CALL; } break;               \
-    case 6: { constexpr int LG = 6; CALL; } break;               \
-    case 7: { constexpr int LG = 7; CALL; } break;               \
-    case 8: { constexpr int LG = 8; CALL; } break;               \
-    case 9: { constexpr int LG = 9; CALL; } break;               \
-    case 10: { constexpr int LG = 10; CALL; } break;             \
-    default: throw Error(TRVG_ERR_PARAM, "Unsupported FFT size."); \
-  }
-
-// Axes of power-of-two length up to 1024 take the compile-time passes of
-// fft.hpp; other (even) lengths the mixed-radix passes of fft_gen.hpp.  Both
-// give a workgroup lines_per_block(n) lines (2048 / n for the former).
-static bool pow2_axis(int n) { return n >= 8 && n <= 1024 && (n & (n - 1)) == 0; }
-// The compile-time passes take whole blocks of 2048 elements: a power-of-two
-// axis of a mesh whose cell count is not a multiple of 2048 (other axes not
-// powers of two) goes through the mixed-radix passes too.
-static bool fast_axis(const Geom& g, int n) { return pow2_axis(n) && g.nmesh % 2048 == 0; }
-static int lines_per_block(int n) { return gen_lines_per_block(n); }
-static long long blocks_of(long long nlines, int nl) { return (nlines + nl - 1) / nl; }
-
-// Dynamic LDS above the default 64 KiB needs the kernel's attribute raised.
-template <class K>
-static void gen_lds(K kernel, size_t bytes) {
-  if (bytes > 64 * 1024)
-    TRVG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
-}
-
-template <typename T, class Loader>
-static void launch_z_gen(Context& ctx, c2<T>* data, const Loader& load, int sign,
-                         double bytes, const Prune& pr) {
-  const int N = ctx.g.n[2];
-  const GenPlan P = make_gen_plan(N);
-  const long long nlines = (long long)ctx.g.n[0] * ctx.g.n[1];
-  const size_t smem = gen_smem<T>(N, false);
-  auto kern = fft_pass_z_gen<T, Loader>;
-  gen_lds(kern, smem);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
-  hipLaunchKernelGGL(kern, dim3(unsigned(blocks_of(nlines, P.nl))), dim3(FFT_THREADS), smem,
-                     ctx.stream, data, load, ctx_twiddles<T>(ctx, N, sign), ctx.g.n[1],
-                     nlines, sign, pr, P);
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T>
-static void launch_strided_gen(Context& ctx, c2<T>* data, int N, long long S,
-                               long long outer_stride, long long inner, int sign,
-                               const Prune& pr, int prune_mode, double bytes) {
-  const GenPlan P = make_gen_plan(N);
-  const long long nlines = ctx.g.nmesh / N;
-  const size_t smem = gen_smem<T>(N, true);
-  auto kern = fft_pass_strided_gen<T>;
-  gen_lds(kern, smem);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  hipLaunchKernelGGL(kern, dim3(unsigned(blocks_of(nlines, P.nl))), dim3(FFT_THREADS), smem,
-                     ctx.stream, data, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
-                     nlines, pr, prune_mode, P);
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T, class BatchLoader>
-static void launch_z_batch_gen(Context& ctx, c2<T>* base, const BatchLoader& load, int sign,
-                               const Prune& pr, const double* kcut2, const int2* work,
-                               int nwork, double bytes) {
-  const int N = ctx.g.n[2];
-  const GenPlan P = make_gen_plan(N);
-  const long long nlines = (long long)ctx.g.n[0] * ctx.g.n[1];
-  const size_t smem = gen_smem<T>(N, false);
-  auto kern = fft_pass_z_batch_gen<T, BatchLoader>;
-  gen_lds(kern, smem);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
-  hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                     ctx.g.nmesh, load, ctx_twiddles<T>(ctx, N, sign), ctx.g.n[1], nlines,
-                     sign, pr, kcut2, work, P);
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T>
-static void launch_strided_batch_gen(Context& ctx, c2<T>* base, int N, long long S,
-                                     long long outer_stride, long long inner, int sign,
-                                     const Prune& pr, const double* kcut2, const int2* work,
-                                     int nwork, int prune_mode, double bytes) {
-  const GenPlan P = make_gen_plan(N);
-  const long long nlines = ctx.g.nmesh / N;
-  const size_t smem = gen_smem<T>(N, true);
-  auto kern = fft_pass_strided_batch_gen<T>;
-  gen_lds(kern, smem);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                     ctx.g.nmesh, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
-                     nlines, pr, kcut2, work, prune_mode, P);
-  TRVG_LAUNCH_CHECK();
-}
-
-Prune make_prune(const Geom& g, double k_hi) {
-  Prune pr{};
-  pr.on = 0;
-  const double kcut2 = k_hi * k_hi * (1. + 1.e-9);
-  // Worth it only if the band leaves part of the (kx, ky) plane empty.
-  const double kx_max = (g.n[0] / 2) * g.dk[0];
-  const double ky_max = (g.n[1] / 2) * g.dk[1];
-  if (kx_max * kx_max + ky_max * ky_max < kcut2) return pr;
-  pr.on = 1;
-  pr.kcut2 = kcut2;
-  pr.dk0 = g.dk[0];
-  pr.dk1 = g.dk[1];
-  pr.n0 = g.n[0];
-  pr.n1 = g.n[1];
-  return pr;
-}
-
-// ---------------------------------------------------------------------------
-// Batched shell transforms: one launch per pass for a whole slab of bins,
-// over only the blocks whose lines lie in each bin's band.
-// ---------------------------------------------------------------------------
-
-// Blocks of the z and y passes holding a line inside a pruning radius, for
-// one geometry (computed once per radius).  The host predicate carries a
-// relative margin over the kernels' exactly rounded one, so every block the
-// kernels would use is listed (a listed block with no needed line only
-// writes zeros that no later pass reads).
-struct PruneLists {
-  std::vector<int> zblocks, yblocks;
-  double d_lines = 0., slabs = 0.;   // needed z lines and y slabs
-};
-
-static const PruneLists& prune_lists(const Geom& g, double kcut2, int nl_z,
-                                     int nl_y) {
-  static std::mutex mu;
-  static std::map<std::vector<double>, std::unique_ptr<PruneLists>> cache;
-  std::vector<double> key = {double(g.n[0]), double(g.n[1]), double(g.n[2]),
-                             g.dk[0], g.dk[1], kcut2, double(nl_z), double(nl_y)};
-  std::lock_guard<std::mutex> lk(mu);
-  auto it = cache.find(key);
-  if (it != cache.end()) return *it->second;
-  auto pl = std::make_unique<PruneLists>();
-  const double kc = kcut2 * (1. + 1.e-12);
-  std::vector<char> slab_in(g.n[0]), line_in((size_t)g.n[0] * g.n[1]);
-  for (int i = 0; i < g.n[0]; i++) {
-    const double kx = shifted(i, g.n[0]) * g.dk[0];
-    slab_in[i] = kx * kx < kc;
-    pl->slabs += (kx * kx < kcut2);
-    for (int j = 0; j < g.n[1]; j++) {
-      const double ky = shifted(j, g.n[1]) * g.dk[1];
-      line_in[(size_t)i * g.n[1] + j] = kx * kx + ky * ky < kc;
-      pl->d_lines += (kx * kx + ky * ky < kcut2);
-    }
-  }
-  const long long nlines = (long long)g.n[0] * g.n[1];
-  for (long long b = 0; b * nl_z < nlines; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_z && !any; l++) any = line_in[b * nl_z + l];
-    if (any) pl->zblocks.push_back(int(b));
-  }
-  const long long ylines = (long long)g.n[0] * g.n[2];   // (i, k) lines
-  for (long long b = 0; b * nl_y < ylines; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_y && !any; l++) any = slab_in[(b * nl_y + l) / g.n[2]];
-    if (any) pl->yblocks.push_back(int(b));
-  }
-  return *(cache[key] = std::move(pl));
-}
-
-template <typename T, int LOGN, class BatchLoader>
-static void launch_z_batch(Context& ctx, c2<T>* base, const BatchLoader& load,
-                           int sign, const Prune& pr, const double* kcut2,
-                           const int2* work, int nwork, double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const size_t smem = fft_smem<T, LOGN>(false);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
-  bool reg = false;
-  if constexpr (use_zreg<T, LOGN, BatchLoader>()) {
-    static_assert(E == zreg_block<T>(), "z pass block size");
-    reg = !pr.on;   // the register pass takes every listed block
-    if (reg)
-      hipLaunchKernelGGL((fft_pass_z_batch_reg<T, LOGN, BatchLoader>),
-                         dim3(unsigned((nwork + 1) / 2)), dim3(zreg_threads<T, LOGN>()),
-                         (zreg_smem<T, LOGN>()), ctx.stream, base, ctx.g.nmesh, load, tw,
-                         ctx.g.n[1], sign, work, nwork);
-  }
-  if (!reg) {
-    if (ctx.g.n[1] % (E / N) == 0)
-      hipLaunchKernelGGL((fft_pass_z_batch<T, LOGN, EPT, true, BatchLoader>),
-                         dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream,
-                         base, ctx.g.nmesh, load, tw, ctx.g.n[1], sign, pr, kcut2, work);
-    else
-      hipLaunchKernelGGL((fft_pass_z_batch<T, LOGN, EPT, false, BatchLoader>),
-                         dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream,
-                         base, ctx.g.nmesh, load, tw, ctx.g.n[1], sign, pr, kcut2, work);
-  }
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T, int LOGN>
-static void launch_strided_batch(Context& ctx, c2<T>* base, long long S,
-                                 long long outer_stride, long long inner,
-                                 int sign, const Prune& pr, const double* kcut2,
-                                 const int2* work, int nwork, int prune_mode,
-                                 double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const size_t smem = fft_smem<T, LOGN>(true);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (inner % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_strided_batch<T, LOGN, EPT, true>), dim3(unsigned(nwork)),
-                       dim3(FFT_THREADS), smem, ctx.stream, base, ctx.g.nmesh, tw, S,
-                       outer_stride, inner, sign, pr, kcut2, work, prune_mode);
-  else
-    hipLaunchKernelGGL((fft_pass_strided_batch<T, LOGN, EPT, false>), dim3(unsigned(nwork)),
-                       dim3(FFT_THREADS), smem, ctx.stream, base, ctx.g.nmesh, tw, S,
-                       outer_stride, inner, sign, pr, kcut2, work, prune_mode);
-  TRVG_LAUNCH_CHECK();
-}
-
-// Transform of several fields in one launch per pass: field f of the work
-// lists lives at base + f * nmesh and loads through load.field(f); with
-// `prune`, kcut2[f] is field f's pruning radius and the lists hold only the
-// blocks that radius needs (z and y passes).
-template <typename T, class BatchLoader>
-void fft3d_batch(Context& ctx, c2<T>* base, const BatchLoader& load, int sign,
-                 bool prune, const double* kcut2, const int2* wz, int nz,
-                 const int2* wy, int ny, const int2* wx, int nx) {
-  const Geom& g = ctx.g;
-  Prune pr{};
-  pr.on = prune ? 1 : 0;
-  pr.dk0 = g.dk[0];
-  pr.dk1 = g.dk[1];
-  pr.n0 = g.n[0];
-  pr.n1 = g.n[1];
-  const double blk = double(FFT_THREADS * FftEpt<T>::v) * sizeof(c2<T>);
-  if (nz > 0) {
-    if (fast_axis(g, g.n[2])) {
-      TRVG_LOGN_SWITCH(ilog2(g.n[2]), (launch_z_batch<T, LG>(
-          ctx, base, load, sign, pr, kcut2, wz, nz, 2. * blk * nz)));
-    } else {
-      launch_z_batch_gen<T>(ctx, base, load, sign, pr, kcut2, wz, nz, 2. * blk * nz);
-    }
-  }
-  if (ny > 0) {
-    if (fast_axis(g, g.n[1])) {
-      TRVG_LOGN_SWITCH(ilog2(g.n[1]), (launch_strided_batch<T, LG>(
-          ctx, base, g.n[2], (long long)g.n[1] * g.n[2], g.n[2], sign, pr, kcut2, wy,
-          ny, 1, 2. * blk * ny)));
-    } else {
-      launch_strided_batch_gen<T>(ctx, base, g.n[1], g.n[2], (long long)g.n[1] * g.n[2],
-                                  g.n[2], sign, pr, kcut2, wy, ny, 1, 2. * blk * ny);
-    }
-  }
-  if (nx > 0) {
-    if (fast_axis(g, g.n[0])) {
-      TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_strided_batch<T, LG>(
-          ctx, base, (long long)g.n[1] * g.n[2], 0, (long long)g.n[1] * g.n[2], sign,
-          pr, kcut2, wx, nx, 2, 2. * blk * nx)));
-    } else {
-      launch_strided_batch_gen<T>(ctx, base, g.n[0], (long long)g.n[1] * g.n[2], 0,
-                                  (long long)g.n[1] * g.n[2], sign, pr, kcut2, wx, nx, 2,
-                                  2. * blk * nx);
-    }
-  }
-}
-
-// Work lists of a shell slab transform over `ngroups` groups of all
-// `nbins` bins: per group nt transforms (nbins, or (nbins + 1) / 2 when
-// packed, two real bins per transform), transform f = group * nt + t.
-// Returns the bins' bands (two per transform when packed, padded with an
-// empty band), each transform's pruning radius (+inf when the band covers
-// the whole plane), and the z / y / x blocks.
-template <typename T>
-void shell_slab_work(const Geom& g, const trvg_binning& kb, int nbins,
-                     int ngroups, bool packed, std::vector<ShellBand>& bands,
-                     std::vector<double>& kcut2, std::vector<int2>& wz,
-                     std::vector<int2>& wy, std::vector<int2>& wx) {
-  const int nl_z = lines_per_block(g.n[2]), nl_y = lines_per_block(g.n[1]);
-  const long long nblk = blocks_of((long long)g.n[1] * g.n[2], lines_per_block(g.n[0]));
-  const int per = packed ? 2 : 1;
-  const int nt = (nbins + per - 1) / per;
-  bands.assign((size_t)nt * per, ShellBand{HUGE_VAL, HUGE_VAL});
-  std::vector<double> kc(nt, 0.);
-  for (int q = 0; q < nbins; q++) {
-    bands[q] = shell_band(kb.bin_edges[q], kb.bin_edges[q + 1]);
-    Prune pq = make_prune(g, kb.bin_edges[q + 1]);
-    kc[q / per] = std::max(kc[q / per], pq.on ? pq.kcut2 : HUGE_VAL);
-  }
-  std::vector<const PruneLists*> pls(nt);
-  for (int t = 0; t < nt; t++) pls[t] = &prune_lists(g, kc[t], nl_z, nl_y);
-  kcut2.clear(); wz.clear(); wy.clear(); wx.clear();
-  for (int gi = 0; gi < ngroups; gi++)
-    for (int t = 0; t < nt; t++) {
-      const int f = gi * nt + t;
-      kcut2.push_back(kc[t]);
-      for (int w : pls[t]->zblocks) wz.push_back(make_int2(f, w));
-      for (int w : pls[t]->yblocks) wy.push_back(make_int2(f, w));
-      for (long long w = 0; w < nblk; w++) wx.push_back(make_int2(f, int(w)));
-    }
-}
-
-template void shell_slab_work<double>(const Geom&, const trvg_binning&, int, int,
-                                      bool, std::vector<ShellBand>&,
-                                      std::vector<double>&, std::vector<int2>&,
-                                      std::vector<int2>&, std::vector<int2>&);
-template void shell_slab_work<float>(const Geom&, const trvg_binning&, int, int,
-                                     bool, std::vector<ShellBand>&,
-                                     std::vector<double>&, std::vector<int2>&,
-                                     std::vector<int2>&, std::vector<int2>&);
-#define TRVG_FFT3D_BATCH_INST(T, L)                                             \
-  template void fft3d_batch<T, L>(Context&, c2<T>*, const L&, int, bool,        \
-                                  const double*, const int2*, int, const int2*, \
-                                  int, const int2*, int);
-TRVG_FFT3D_BATCH_INST(double, LoadScaleShiftMocks)
-TRVG_FFT3D_BATCH_INST(double, LoadTwoptMocks)
-TRVG_FFT3D_BATCH_INST(double, LoadShellMocks<double>)
-TRVG_FFT3D_BATCH_INST(float, LoadShellMocks<float>)
-TRVG_FFT3D_BATCH_INST(double, LoadShellPairMocks<double>)
-TRVG_FFT3D_BATCH_INST(float, LoadShellPairMocks<float>)
-TRVG_FFT3D_BATCH_INST(double, LoadDeconvMocks<double>)
-TRVG_FFT3D_BATCH_INST(float, LoadDeconvMocks<float>)
-#undef TRVG_FFT3D_BATCH_INST
-
-// Shell fields of a real source field are real for m = 0 and even l (the
-// spectrum y_l0(k^) f(k) / W(k) is Hermitian).
-static bool real_shells(int ell, int m) { return m == 0 && ell % 2 == 0; }
-
-// ---------------------------------------------------------------------------
-// Shell transforms, x-first: the x pass carries the shell loader (lines
-// along x at fixed (k_y, k_z), pruned on k_y^2 + k_z^2), the y pass is
-// pruned on k_z, and the last pass runs along the contiguous z lines, so
-// the full-size output of every field is written in whole 16 KiB blocks
-// rather than as short strided segments.
-// ---------------------------------------------------------------------------
-
-// Prune over the (z, y) axes: P2(k) tests k_z, P1(k, j) tests (k_z, k_y).
-static Prune prune_zy(const Geom& g) {
-  Prune pr{};
-  pr.on = 1;
-  pr.dk0 = g.dk[2];
-  pr.dk1 = g.dk[1];
-  pr.n0 = g.n[2];
-  pr.n1 = g.n[1];
-  return pr;
-}
-
-struct PruneListsXF {
-  std::vector<int> xblocks, yblocks;
-  double x_lines = 0., y_lines = 0.;   // needed x lines, written y lines
-};
-
-static const PruneListsXF& prune_lists_xfirst(const Geom& g, double kcut2, int nl_x,
-                                              int nl_y) {
-  static std::mutex mu;
-  static std::map<std::vector<double>, std::unique_ptr<PruneListsXF>> cache;
-  std::vector<double> key = {double(g.n[0]), double(g.n[1]), double(g.n[2]),
-                             g.dk[1], g.dk[2], kcut2, double(nl_x), double(nl_y)};
-  std::lock_guard<std::mutex> lk(mu);
-  auto it = cache.find(key);
-  if (it != cache.end()) return *it->second;
-  auto pl = std::make_unique<PruneListsXF>();
-  const double kc = kcut2 * (1. + 1.e-12);
-  const int n1 = g.n[1], n2 = g.n[2];
-  std::vector<char> kz_in(n2), line_in((size_t)n1 * n2);
-  double nkz = 0.;
-  for (int k = 0; k < n2; k++) {
-    const double kz = shifted(k, n2) * g.dk[2];
-    kz_in[k] = kz * kz < kc;
-    nkz += (kz * kz < kcut2);
-    for (int j = 0; j < n1; j++) {
-      const double ky = shifted(j, n1) * g.dk[1];
-      line_in[(size_t)j * n2 + k] = kz * kz + ky * ky < kc;
-      pl->x_lines += (kz * kz + ky * ky < kcut2);
-    }
-  }
-  pl->y_lines = nkz * g.n[0];
-  const long long xl = (long long)n1 * n2;
-  for (long long b = 0; b * nl_x < xl; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_x && !any; l++) any = line_in[b * nl_x + l];
-    if (any) pl->xblocks.push_back(int(b));
-  }
-  const long long yl = (long long)g.n[0] * n2;
-  for (long long b = 0; b * nl_y < yl; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_y && !any; l++) any = kz_in[(b * nl_y + l) % n2];
-    if (any) pl->yblocks.push_back(int(b));
-  }
-  return *(cache[key] = std::move(pl));
-}
-
-template <typename T, int LOGN, class BatchLoader>
-static void launch_x_load_batch(Context& ctx, c2<T>* base, const BatchLoader& load,
-                                const Prune& pr, const double* kcut2, const int2* work,
-                                int nwork, double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const size_t smem = fft_smem<T, LOGN>(false);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, +1);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (ctx.g.n[2] % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_x_load_batch<T, LOGN, EPT, true, BatchLoader>),
-                       dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                       ctx.g.nmesh, load, tw, ctx.g.n[1], ctx.g.n[2], +1, pr, kcut2, work);
-  else
-    hipLaunchKernelGGL((fft_pass_x_load_batch<T, LOGN, EPT, false, BatchLoader>),
-                       dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                       ctx.g.nmesh, load, tw, ctx.g.n[1], ctx.g.n[2], +1, pr, kcut2, work);
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T, class BatchLoader>
-static void launch_x_load_batch_gen(Context& ctx, c2<T>* base, const BatchLoader& load,
-                                    const Prune& pr, const double* kcut2, const int2* work,
-                                    int nwork, double bytes) {
-  const int N = ctx.g.n[0];
-  const GenPlan P = make_gen_plan(N);
-  const size_t smem = gen_smem<T>(N, false);
-  auto kern = fft_pass_x_load_batch_gen<T, BatchLoader>;
-  gen_lds(kern, smem);
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                     ctx.g.nmesh, load, ctx_twiddles<T>(ctx, N, +1), ctx.g.n[1], ctx.g.n[2],
-                     pr, kcut2, work, P);
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T>
-static void xfirst_yz(Context& ctx, c2<T>* base, const double* kcut2, const int2* wy, int ny,
-                      const int2* wz, int nz, double by, double bz);
-
-// The three passes of a batched x-first transform: field f of the work
-// lists lives at base + f * nmesh, loads through load.field(f) and is pruned
-// with radius kcut2[f] (+inf: no pruning); wz lists every block.
-template <typename T, class BatchLoader>
-static void xfirst_passes(Context& ctx, c2<T>* base, const BatchLoader& load,
-                          const double* kcut2, const int2* wx, int nx, const int2* wy,
-                          int ny, const int2* wz, int nz, double bx, double by, double bz) {
-  const Geom& g = ctx.g;
-  if (nx > 0) {
-    if (fast_axis(g, g.n[0])) {
-      TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_x_load_batch<T, LG>(
-          ctx, base, load, prune_zy(g), kcut2, wx, nx, bx)));
-    } else {
-      launch_x_load_batch_gen<T>(ctx, base, load, prune_zy(g), kcut2, wx, nx, bx);
-    }
-  }
-  xfirst_yz<T>(ctx, base, kcut2, wy, ny, wz, nz, by, bz);
-}
-
-// The y and z passes of a batched x-first transform.
-template <typename T>
-static void xfirst_yz(Context& ctx, c2<T>* base, const double* kcut2, const int2* wy, int ny,
-                      const int2* wz, int nz, double by, double bz) {
-  const Geom& g = ctx.g;
-  const Prune pr = prune_zy(g);
-  if (ny > 0) {
-    if (fast_axis(g, g.n[1])) {
-      TRVG_LOGN_SWITCH(ilog2(g.n[1]), (launch_strided_batch<T, LG>(
-          ctx, base, g.n[2], (long long)g.n[1] * g.n[2], g.n[2], +1, pr, kcut2, wy, ny, 3,
-          by)));
-    } else {
-      launch_strided_batch_gen<T>(ctx, base, g.n[1], g.n[2], (long long)g.n[1] * g.n[2],
-                                  g.n[2], +1, pr, kcut2, wy, ny, 3, by);
-    }
-  }
-  // z pass over every block, reading only the k_z rows the y pass wrote.
-  Prune off{};
-  off.on = 0;
-  LoadMaskedZBatch<T> lz{base, g.nmesh, kcut2, g.dk[2], g.n[2]};
-  if (nz > 0) {
-    if (fast_axis(g, g.n[2])) {
-      TRVG_LOGN_SWITCH(ilog2(g.n[2]), (launch_z_batch<T, LG>(
-          ctx, base, lz, +1, off, kcut2, wz, nz, bz)));
-    } else {
-      launch_z_batch_gen<T>(ctx, base, lz, +1, off, kcut2, wz, nz, bz);
-    }
-  }
-}
-
-// Shell fields of (ell, m) for `bins`: the backward transform of
-// y_lm(k^) src(k) / W(k) on each bin's shell, all bins per pass in one
-// launch.  Unpacked: field q at base + q * nmesh.  Packed (real shells:
-// real source, even l, m = 0): bins q = 2p, 2p + 1 are the real and
-// imaginary parts of base + p * nmesh.
-// Launch plan of a shell slab transform (bands, pruning radii, work lists
-// and profiler byte counts), a function of the geometry and the bins only:
-// built once per device and reused by every later call.
-struct ShellPlan {
-  DevArray<ShellBand> bands;
-  DevArray<double> kc;
-  DevArray<int2> w;
-  int nx = 0, ny = 0, nz = 0;
-  double bx = 0., by = 0., bz = 0.;
-};
-
-template <typename T>
-static std::shared_ptr<const ShellPlan> shell_plan(Context& ctx, const trvg_binning& kb,
-                                                   const std::vector<int>& bins,
-                                                   const std::vector<int>& nmodes,
-                                                   bool packed) {
-  const Geom& g = ctx.g;
-  const int nf = int(bins.size());
-  std::vector<double> key = {double(ctx.dev), double(sizeof(T)), double(packed)};
-  for (int a = 0; a < 3; a++) { key.push_back(g.n[a]); key.push_back(g.dk[a]); }
-  for (int b : bins) {
-    key.push_back(kb.bin_edges[b]);
-    key.push_back(kb.bin_edges[b + 1]);
-    key.push_back(nmodes[b]);
-  }
-  static std::mutex mu;
-  static std::map<std::vector<double>, std::shared_ptr<const ShellPlan>> cache;
-  {
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = cache.find(key);
-    if (it != cache.end()) return it->second;
-  }
-  const int nt = packed ? (nf + 1) / 2 : nf;
-  const int per = packed ? 2 : 1;
-  const int nl_x = lines_per_block(g.n[0]), nl_y = lines_per_block(g.n[1]);
-  const ShellBand none{HUGE_VAL, HUGE_VAL};
-  std::vector<ShellBand> bands((size_t)nt * per, none);
-  std::vector<double> kc(nt, 0.);
-  // z blocks: every (i, j) line of the last pass.
-  const long long nblk = blocks_of((long long)g.n[0] * g.n[1], lines_per_block(g.n[2]));
-  std::vector<int2> wx, wy, wz;
-  const double cb = sizeof(c2<T>);
-  auto pl = std::make_shared<ShellPlan>();
-  for (int q = 0; q < nf; q++) {
-    const int b = bins[q];
-    bands[q] = shell_band(kb.bin_edges[b], kb.bin_edges[b + 1]);
-    Prune pq = make_prune(g, kb.bin_edges[b + 1]);
-    kc[q / per] = std::max(kc[q / per], pq.on ? pq.kcut2 : HUGE_VAL);
-    pl->bx += double(nmodes[b]) * sizeof(double2);
-  }
-  for (int f = 0; f < nt; f++) {
-    const PruneListsXF& px = prune_lists_xfirst(g, kc[f], nl_x, nl_y);
-    for (int w : px.xblocks) wx.push_back(make_int2(f, w));
-    for (int w : px.yblocks) wy.push_back(make_int2(f, w));
-    for (long long w = 0; w < nblk; w++) wz.push_back(make_int2(f, int(w)));
-    const double xw = px.x_lines * g.n[0] * cb;
-    const double yw = px.y_lines * g.n[1] * cb;
-    pl->bx += xw;
-    pl->by += xw + yw;
-    pl->bz += yw + double(g.nmesh) * cb;
-  }
-  pl->nx = int(wx.size());
-  pl->ny = int(wy.size());
-  pl->nz = int(wz.size());
-  pl->bands.reset(bands.size());
-  pl->kc.reset(nt);
-  pl->w.reset(wx.size() + wy.size() + wz.size());
-  wx.insert(wx.end(), wy.begin(), wy.end());
-  wx.insert(wx.end(), wz.begin(), wz.end());
-  TRVG_HIP(hipMemcpyAsync(pl->bands.get(), bands.data(), bands.size() * sizeof(ShellBand),
-                          hipMemcpyHostToDevice, ctx.stream));
-  TRVG_HIP(hipMemcpyAsync(pl->kc.get(), kc.data(), nt * sizeof(double),
-                          hipMemcpyHostToDevice, ctx.stream));
-  TRVG_HIP(hipMemcpyAsync(pl->w.get(), wx.data(), wx.size() * sizeof(int2),
-                          hipMemcpyHostToDevice, ctx.stream));
-  TRVG_HIP(hipStreamSynchronize(ctx.stream));
-  std::lock_guard<std::mutex> lk(mu);
-  if (cache.size() >= 64) cache.clear();   // bounded; plans in use stay alive
-  cache[key] = pl;
-  return pl;
-}
-
-template <typename T>
-void shell_slab_ifft(Context& ctx, c2<T>* base, const double2* src,
-                     const trvg_binning& kb, const std::vector<int>& bins,
-                     const std::vector<int>& nmodes, int ell, int m, bool packed) {
-  const Geom& g = ctx.g;
-  if (bins.empty()) return;
-  const std::shared_ptr<const ShellPlan> pl = shell_plan<T>(ctx, kb, bins, nmodes, packed);
-  // The plan outlives the queued launches even if the cache drops it.
-  ctx.keep.push_back(std::const_pointer_cast<ShellPlan>(pl));
-  const int2* px = pl->w.get();
-  const int2* py = px + pl->nx;
-  const int2* pz = py + pl->ny;
-  if (packed) {
-    LoadShellPairBatch<T, double> ld{src, ctx.tab, g, pl->bands.get(), ell, m};
-    xfirst_passes<T>(ctx, base, ld, pl->kc.get(), px, pl->nx, py, pl->ny, pz, pl->nz,
-                     pl->bx, pl->by, pl->bz);
-  } else {
-    LoadShellBatch<T, double> ld{src, ctx.tab, g, pl->bands.get(), ell, m};
-    xfirst_passes<T>(ctx, base, ld, pl->kc.get(), px, pl->nx, py, pl->ny, pz, pl->nz,
-                     pl->bx, pl->by, pl->bz);
-  }
-}
-
-template <typename T, int LOGN>
-static void launch_x_sjl(Context& ctx, c2<T>* base, int nt, const double2* src,
-                         const Spline& sp, const double* r, int ell, int m, bool packed,
-                         double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const Geom& g = ctx.g;
-  const size_t smem = fft_smem<T, LOGN>(false);
-  const unsigned grid = unsigned((long long)g.n[1] * g.n[2] / (E / N));
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (packed)
-    hipLaunchKernelGGL((fft_x_sjl_multi<T, LOGN, EPT, true>), dim3(grid), dim3(FFT_THREADS),
-                       smem, ctx.stream, base, g.nmesh, nt, src, ctx.tab, g, sp.dev(), r, ell,
-                       m, ctx_twiddles<T>(ctx, N, +1));
-  else
-    hipLaunchKernelGGL((fft_x_sjl_multi<T, LOGN, EPT, false>), dim3(grid), dim3(FFT_THREADS),
-                       smem, ctx.stream, base, g.nmesh, nt, src, ctx.tab, g, sp.dev(), r, ell,
-                       m, ctx_twiddles<T>(ctx, N, +1));
-  TRVG_LAUNCH_CHECK();
-}
-
-template <typename T>
-static void launch_x_sjl_gen(Context& ctx, c2<T>* base, int nt, const double2* src,
-                             const Spline& sp, const double* r, int ell, int m, bool packed,
-                             double bytes) {
-  const Geom& g = ctx.g;
-  const int N = g.n[0];
-  const GenPlan P = make_gen_plan(N);
-  const size_t smem = gen_smem<T>(N, false);
-  const unsigned grid = unsigned(blocks_of((long long)g.n[1] * g.n[2], P.nl));
-  ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (packed) {
-    auto kern = fft_x_sjl_multi_gen<T, true>;
-    gen_lds(kern, smem);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(FFT_THREADS), smem, ctx.stream, base, g.nmesh,
-                       nt, src, ctx.tab, g, sp.dev(), r, ell, m,
-                       ctx_twiddles<T>(ctx, N, +1), P);
-  } else {
-    auto kern = fft_x_sjl_multi_gen<T, false>;
-    gen_lds(kern, smem);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(FFT_THREADS), smem, ctx.stream, base, g.nmesh,
-                       nt, src, ctx.tab, g, sp.dev(), r, ell, m,
-                       ctx_twiddles<T>(ctx, N, +1), P);
-  }
-  TRVG_LAUNCH_CHECK();
-}
-
-// j_l-weighted shell fields of (ell, m) for `bins` (3PCF,
-// inv_fourier_transform_sjl_ylm_wgtd_field, field.cpp:1908-2010), r the
-// bins' effective radii: x-first batched transforms over every block (no
-// band limit); layout and packing as shell_slab_ifft.
-template <typename T>
-void sjl_slab_ifft(Context& ctx, c2<T>* base, const double2* src, const Spline& sp,
-                   const std::vector<double>& r, const std::vector<int>& bins, int ell,
-                   int m, bool packed) {
-  const Geom& g = ctx.g;
-  const int nf = int(bins.size());
-  if (nf == 0) return;
-  const int nt = packed ? (nf + 1) / 2 : nf;
-  const int per = packed ? 2 : 1;
-  std::vector<double> rr((size_t)nt * per, -1.);
-  for (int q = 0; q < nf; q++) rr[q] = r[bins[q]];
-  DevArray<double> dr(rr.size());
-  ctx.upload(dr.get(), rr.data(), rr.size());
-  // Work lists (y blocks, then every z block, per transform) and the
-  // unpruned radii depend on the geometry and the transform count only:
-  // built once per device.
-  std::vector<double> key = {double(ctx.dev), double(sizeof(T)), double(nt)};
-  for (int a = 0; a < 3; a++) key.push_back(g.n[a]);
-  static std::mutex mu;
-  static std::map<std::vector<double>, std::shared_ptr<ShellPlan>> cache;
-  std::shared_ptr<ShellPlan> plan;
-  {
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = cache.find(key);
-    if (it != cache.end()) plan = it->second;
-  }
-  if (!plan) {
-    const PruneListsXF& pl = prune_lists_xfirst(g, HUGE_VAL, lines_per_block(g.n[0]),
-                                                lines_per_block(g.n[1]));
-    const long long nblk = blocks_of((long long)g.n[0] * g.n[1], lines_per_block(g.n[2]));
-    std::vector<double> kc(nt, HUGE_VAL);
-    std::vector<int2> w;   // y blocks, then z blocks
-    for (int f = 0; f < nt; f++)
-      for (int b : pl.yblocks) w.push_back(make_int2(f, b));
-    const size_t ny = w.size();
-    for (int f = 0; f < nt; f++)
-      for (long long b = 0; b < nblk; b++) w.push_back(make_int2(f, int(b)));
-    plan = std::make_shared<ShellPlan>();
-    plan->ny = int(ny);
-    plan->nz = int(w.size() - ny);
-    plan->kc.reset(nt);
-    plan->w.reset(w.size());
-    TRVG_HIP(hipMemcpyAsync(plan->kc.get(), kc.data(), nt * sizeof(double),
-                            hipMemcpyHostToDevice, ctx.stream));
-    TRVG_HIP(hipMemcpyAsync(plan->w.get(), w.data(), w.size() * sizeof(int2),
-                            hipMemcpyHostToDevice, ctx.stream));
-    TRVG_HIP(hipStreamSynchronize(ctx.stream));
-    std::lock_guard<std::mutex> lk(mu);
-    if (cache.size() >= 16) cache.clear();   // bounded; plans in use stay alive
-    cache[key] = plan;
-  }
-  ctx.keep.push_back(plan);
-  const size_t ny = size_t(plan->ny), nz = size_t(plan->nz);
-  const int2* dwp = plan->w.get();
-  // Algorithmic bytes: the source read once, then each pass writes (and the
-  // later ones read) every field.
-  const double fb = double(g.nmesh) * sizeof(c2<T>) * nt;
-  const double bx = double(g.nmesh) * sizeof(double2) + fb, by = 2. * fb, bz = 2. * fb;
-  if (fast_axis(g, g.n[0])) {
-    TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_x_sjl<T, LG>(ctx, base, nt, src, sp, dr.get(),
-                                                          ell, m, packed, bx)));
-  } else {
-    launch_x_sjl_gen<T>(ctx, base, nt, src, sp, dr.get(), ell, m, packed, bx);
-  }
-  // The radii stay owned until the stream is synchronised: returned to the
-  // shared pool now, another call could take and overwrite them while the
-  // x pass still reads them.
-  ctx.keep_until_flush(std::move(dr));
-  xfirst_yz<T>(ctx, base, plan->kc.get(), dwp, int(ny), dwp + ny, int(nz), by, bz);
-}
-
-template <typename T, class Loader>
-void fft3d(Context& ctx, c2<T>* data, const Loader& load, int sign,
-           double read_bytes, const Prune* prune) {
-  const Geom& g = ctx.g;
-  Prune pr{};
-  pr.on = 0;
-  if (prune) pr = *prune;
-  const double cb = sizeof(c2<T>);
-  // Lines / slabs each pass touches (for the profiler's algorithmic bytes).
-  double d_lines = double(g.n[0]) * g.n[1], slabs = g.n[0];
-  if (pr.on) {
-    d_lines = 0.;
-    slabs = 0.;
-    for (int i = 0; i < g.n[0]; i++) {
-      double kx = shifted(i, g.n[0]) * g.dk[0];
-      if (kx * kx < pr.kcut2) slabs += 1.;
-      for (int j = 0; j < g.n[1]; j++) {
-        double ky = shifted(j, g.n[1]) * g.dk[1];
-        if (kx * kx + ky * ky < pr.kcut2) d_lines += 1.;
-      }
-    }
-  }
-  if (read_bytes < 0.) read_bytes = double(g.nmesh) * cb;
-  const double zw = d_lines * g.n[2] * cb;
-  const double slab_vals = slabs * g.n[1] * g.n[2];
-  if (fast_axis(g, g.n[2])) {
-    TRVG_LOGN_SWITCH(ilog2(g.n[2]), (launch_z<T, LG, Loader>(
-        ctx, data, load, sign, read_bytes, zw, pr)));
-  } else {
-    launch_z_gen<T>(ctx, data, load, sign, read_bytes + zw, pr);
-  }
-  if (fast_axis(g, g.n[1])) {
-    TRVG_LOGN_SWITCH(ilog2(g.n[1]), (launch_strided<T, LG>(
-        ctx, data, g.n[2], (long long)g.n[1] * g.n[2], g.n[2], sign, pr, 1,
-        zw + slab_vals * cb)));
-  } else {
-    launch_strided_gen<T>(ctx, data, g.n[1], g.n[2], (long long)g.n[1] * g.n[2], g.n[2],
-                          sign, pr, 1, zw + slab_vals * cb);
-  }
-  if (fast_axis(g, g.n[0])) {
-    TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_strided<T, LG>(
-        ctx, data, (long long)g.n[1] * g.n[2], 0, (long long)g.n[1] * g.n[2], sign,
-        pr, 2, slab_vals * cb + double(g.nmesh) * cb)));
-  } else {
-    launch_strided_gen<T>(ctx, data, g.n[0], (long long)g.n[1] * g.n[2], 0,
-                          (long long)g.n[1] * g.n[2], sign, pr, 2,
-                          slab_vals * cb + double(g.nmesh) * cb);
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Small launch helpers
@@ -2332,34 +1446,5 @@ template Result run_3pcf<float>(Context&, const DeviceCatalogue&,
                                 const trvg_binning&, double, const Window3pcf*);
 template double run_mesh_norm<double>(Context&, const DeviceCatalogue&);
 template double run_mesh_norm<float>(Context&, const DeviceCatalogue&);
-template void fft3d<double, LoadSame<double>>(Context&, double2*,
-                                              const LoadSame<double>&, int,
-                                              double, const Prune*);
-template void fft3d<float, LoadSame<float>>(Context&, float2*,
-                                            const LoadSame<float>&, int, double,
-                                            const Prune*);
-
-// Loaders of the two-point path (engine_twopt.hip).
-template void fft3d<double, LoadScaleShift<double>>(Context&, double2*,
-                                                    const LoadScaleShift<double>&, int,
-                                                    double, const Prune*);
-template void fft3d<double, LoadTwopt<double, double>>(Context&, double2*,
-                                                       const LoadTwopt<double, double>&,
-                                                       int, double, const Prune*);
-
-// Loaders of the differentiable path (engine_diff.hip).
-#define TRVG_FFT3D_INST(T, L)                                                   \
-  template void fft3d<T, L>(Context&, c2<T>*, const L&, int, double, const Prune*);
-TRVG_FFT3D_INST(double, LoadReal<double>)
-TRVG_FFT3D_INST(float, LoadReal<float>)
-TRVG_FFT3D_INST(double, LoadShellCotangent<double>)
-TRVG_FFT3D_INST(float, LoadShellCotangent<float>)
-#define TRVG_COMMA ,
-TRVG_FFT3D_INST(double, LoadDeconv<double TRVG_COMMA double>)
-TRVG_FFT3D_INST(float, LoadDeconv<float TRVG_COMMA float>)
-TRVG_FFT3D_INST(double, LoadShell<double TRVG_COMMA double>)
-TRVG_FFT3D_INST(float, LoadShell<float TRVG_COMMA float>)
-#undef TRVG_COMMA
-#undef TRVG_FFT3D_INST
 
 }  // namespace trvg
