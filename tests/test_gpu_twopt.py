@@ -131,6 +131,36 @@ def test_engine_twopt_matches_oracle(case):
                                    out[1]['_norm_factors'][i], rtol=1e-12)
 
 
+@pytest.mark.parametrize('scheme', ['ngp', 'cic', 'tsc', 'pcs'])
+@pytest.mark.parametrize('ng', [(32, 32, 32), (20, 36, 8)])
+def test_interlaced_assignment_at_the_box_edges(scheme, ng):
+    """The shadow pass at the first and last cells of an axis (its base cell
+    wraps, sits exactly on index n, and order 3 keeps the reference's rule
+    for the last two cells), against the oracle; meshes of whole and partial
+    8-cell tiles."""
+    from triumvirate_amd import twopt as T
+    from triumvirate_amd.catalogue import ParticleCatalogue
+    from triumvirate_amd.dataobjs import Binning
+    print(f"interlaced edges {scheme} {ng}", flush=True)
+    g = np.random.default_rng(11)
+    cell, L = 31.25, tuple(31.25 * n for n in ng)     # exact in binary
+    pos = []
+    for n in ng:
+        edge = np.array([0.25, 0.5, 0.75, 1.25, 1.5, n - 1.5, n - 1.25, n - 0.75,
+                         n - 0.5, n - 0.25])
+        c = np.concatenate([g.choice(edge, 1500), g.uniform(0.25, n - 0.25, 500)])
+        c[:2] = 0.25, n - 0.25                        # extents: no shift
+        pos.append(c * cell)
+    b = Binning('fourier', 'lin', bin_min=0.01, bin_max=0.09, num_bins=5)
+    out = []
+    for backend in (_engine(), _oracle()):
+        cat = ParticleCatalogue(*pos, nz=len(pos[0]) / np.prod(L))
+        out.append(T._compute_2pt_stats_sim_like(
+            backend, 'powspec', cat, paramset=_paramset(ng, L, scheme, 'on', 0),
+            degree=0, binning=b))
+    _compare(out[0], out[1], 'powspec')
+
+
 def test_public_twopt_api():
     """The public functions run end to end with the reference's argument
     names and return the reference's keys."""

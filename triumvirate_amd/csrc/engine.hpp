@@ -439,10 +439,11 @@ template <typename T>
 void assign_field(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c, int mode,
                   int ell, int m, double scale);
 
-// Add catalogue `c` with weight mode and scale into `mesh` (no zeroing).
+// Add catalogue `c` with weight mode and scale into `mesh` (no zeroing);
+// shadow: the half-cell-shifted pass of interlacing.
 template <typename T>
 void assign_add(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c, int mode,
-                int ell, int m, double scale);
+                int ell, int m, double scale, bool shadow = false);
 
 // Two-point statistics (engine_twopt.hip).  Binned values of one
 // power-spectrum or correlation-function multipole.

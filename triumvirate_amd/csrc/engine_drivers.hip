@@ -138,12 +138,15 @@ static unsigned tile_grid(const TiledView& tv) {
 template <typename T, int ORDER>
 static void assign_order(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c,
                          const TiledView& tv, int mode, int ell, int m, double scale,
-                         int cplx_w) {
+                         int cplx_w, bool shadow) {
   DevParticles sv = c.view();
   if (tile_grid(tv) > 0) {
-    hipLaunchKernelGGL((k_assign_tiled<T, ORDER>), dim3(tile_grid(tv)), dim3(256), 0,
-                       ctx.stream, mesh, sv, ctx.g, tv.tg, tv.work.get(), tv.meta.get(),
-                       mode, ell, m, scale, cplx_w);
+    auto kern = cplx_w == 1 ? (shadow ? k_assign_tiled<T, ORDER, true, true>
+                                      : k_assign_tiled<T, ORDER, true, false>)
+                            : (shadow ? k_assign_tiled<T, ORDER, false, true>
+                                      : k_assign_tiled<T, ORDER, false, false>);
+    hipLaunchKernelGGL(kern, dim3(tile_grid(tv)), dim3(256), 0, ctx.stream, mesh, sv, ctx.g,
+                       tv.tg, tv.work.get(), tv.meta.get(), mode, ell, m, scale, cplx_w);
     TRVG_LAUNCH_CHECK();
   }
   // Stragglers [meta[1], n) keep the reference's flattened-index rule.
@@ -152,16 +155,18 @@ static void assign_order(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c,
                                                       ? grid_for(ctx, tv.nstraggle, 16)
                                                       : 64u),
                        dim3(256), 0, ctx.stream, mesh, sv, ctx.g, mode, ell, m, scale,
-                       cplx_w, 0, tv.meta.get() + 1);
+                       cplx_w, int(shadow), tv.meta.get() + 1);
     TRVG_LAUNCH_CHECK();
   }
 }
 
 // imag: a real weight (m = 0 or a unit/scalar mode) goes into the
-// imaginary parts of the mesh instead of the real parts.
+// imaginary parts of the mesh instead of the real parts.  shadow: the
+// half-cell-shifted pass of interlacing.
 template <typename T>
 static void assign(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c,
-                   int mode, int ell, int m, double scale, bool imag = false) {
+                   int mode, int ell, int m, double scale, bool imag = false,
+                   bool shadow = false) {
   // y_l0 is real (its imaginary part is a signed zero): m = 0 fields take
   // real parts only.
   int cplx_w = ((mode == WM_YLM_W || mode == WM_YLMC_W2) && m != 0);
@@ -178,10 +183,10 @@ static void assign(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c,
                   ((mode == WM_YLM_W || mode == WM_YLMC_W2) ? 24. : 0.);
   ProfScope ps(ctx, KC_ASSIGN, c.n * pbytes + double(ctx.g.nmesh) * sizeof(c2<T>));
   switch (ctx.p.assignment_order) {
-    case 1: assign_order<T, 1>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w); break;
-    case 2: assign_order<T, 2>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w); break;
-    case 3: assign_order<T, 3>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w); break;
-    default: assign_order<T, 4>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w); break;
+    case 1: assign_order<T, 1>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w, shadow); break;
+    case 2: assign_order<T, 2>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w, shadow); break;
+    case 3: assign_order<T, 3>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w, shadow); break;
+    default: assign_order<T, 4>(ctx, mesh, c, tv, mode, ell, m, scale, cplx_w, shadow); break;
   }
 }
 
@@ -241,11 +246,11 @@ static void assign_dual(Context& ctx, T* ra, T* rb, const DeviceCatalogue& c, in
 
 template <typename T>
 void assign_add(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c, int mode,
-                int ell, int m, double scale) {
-  assign<T>(ctx, mesh, c, mode, ell, m, scale);
+                int ell, int m, double scale, bool shadow) {
+  assign<T>(ctx, mesh, c, mode, ell, m, scale, false, shadow);
 }
 template void assign_add<double>(Context&, double2*, const DeviceCatalogue&, int, int,
-                                 int, double);
+                                 int, double, bool);
 
 template <typename T>
 void assign_field(Context& ctx, c2<T>* mesh, const DeviceCatalogue& c, int mode,

@@ -63,30 +63,6 @@ void zero_mesh(Context& ctx, double2* f) {
   TRVG_LAUNCH_CHECK();
 }
 
-// The half-cell-shifted pass of field.cpp's interlacing, added into fs.
-template <int ORDER>
-void shadow_order(Context& ctx, double2* fs, const DeviceCatalogue& c, int mode, int ell,
-                  int m, double scale) {
-  const int cplx_w = (mode == WM_YLM_W && m != 0) ? 1 : 0;
-  hipLaunchKernelGGL((k_assign<double, ORDER>), dim3(grid_for(ctx, c.n, 16)), dim3(256), 0,
-                     ctx.stream, fs, c.view(), ctx.g, mode, ell, m, scale, cplx_w, 1,
-                     nullptr);
-  TRVG_LAUNCH_CHECK();
-}
-
-void shadow_add(Context& ctx, double2* fs, const DeviceCatalogue& c, int mode, int ell,
-                int m, double scale) {
-  if (mode == WM_YLM_W && c.los.get() == nullptr)
-    throw Error(TRVG_ERR_DATA, "Lines of sight are required for survey-type fields.");
-  ProfScope ps(ctx, KC_ASSIGN, double(c.n) * 56. + double(ctx.g.nmesh) * 16.);
-  switch (ctx.p.assignment_order) {
-    case 1: shadow_order<1>(ctx, fs, c, mode, ell, m, scale); break;
-    case 2: shadow_order<2>(ctx, fs, c, mode, ell, m, scale); break;
-    case 3: shadow_order<3>(ctx, fs, c, mode, ell, m, scale); break;
-    default: shadow_order<4>(ctx, fs, c, mode, ell, m, scale); break;
-  }
-}
-
 // Which field a two-point call builds.
 enum FieldKind {
   FK_PAIR,     // sum_d y w - alpha sum_r y w       (field.cpp:1246-1323)
@@ -115,12 +91,12 @@ void twopt_field(Context& ctx, double2* f, double2* fs, FieldKind kind,
   if (!il) return;
   zero_mesh(ctx, fs);
   if (kind == FK_PAIR) {
-    shadow_add(ctx, fs, *d, WM_YLM_W, ell, m, 1.);
-    shadow_add(ctx, fs, r, WM_YLM_W, ell, m, -alpha);
+    assign_add<double>(ctx, fs, *d, WM_YLM_W, ell, m, 1., true);
+    assign_add<double>(ctx, fs, r, WM_YLM_W, ell, m, -alpha, true);
   } else if (kind == FK_SINGLE) {
-    shadow_add(ctx, fs, r, WM_YLM_W, ell, m, 1.);
+    assign_add<double>(ctx, fs, r, WM_YLM_W, ell, m, 1., true);
   } else {
-    shadow_add(ctx, fs, r, WM_UNIT, 0, 0, 1.);
+    assign_add<double>(ctx, fs, r, WM_UNIT, 0, 0, 1., true);
   }
   fft3d<double>(ctx, fs, LoadScaleShift<double>{fs, 0., ctx.g.vol_cell}, -1);
   ProfScope ps(ctx, KC_MISC, 3. * double(ctx.g.nmesh) * 16.);

@@ -47,12 +47,102 @@ __device__ __forceinline__ double2 particle_weight(const DevParticles& p,
   return dmk(y.x * w2, -y.y * w2);
 }
 
-// Mesh assignment (field.cpp:569-1112): window weights and periodic index
-// rules per scheme; cell value += w * W_x W_y W_z / V_cell (times `scale`,
-// e.g. -alpha for randoms).  `shadow` selects the half-cell-shifted pass
-// used for interlacing.  Particles [*first, n) (all of them when `first` is
-// null) are assigned.  Hardware FP64/FP32 atomics on the coarse-grained
-// mesh.
+// Mesh assignment of one particle of weight (wre, wim) (field.cpp:569-1112):
+// window weights and periodic index rules per scheme; cell value +=
+// w W_x W_y W_z.  `shadow` selects the half-cell-shifted pass used for
+// interlacing.  Hardware FP64/FP32 atomics on the coarse-grained mesh.
+template <typename T, int ORDER>
+__device__ __forceinline__ void assign_particle(c2<T>* __restrict__ mesh, const double pos[3],
+                                                double wre, double wim, const Geom& g,
+                                                int cplx_w, int shadow) {
+  int ijk[ORDER][3];
+  double win[ORDER][3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const int ng = g.n[a];
+    double loc = __ddiv_rn(__dmul_rn(double(ng), pos[a]), g.L[a]);
+    if (shadow) {
+      loc = __dadd_rn(loc, 0.5);
+      if (loc > ng) loc = __dadd_rn(loc, -double(ng));
+    }
+    int idx = int(loc);
+    double s = __dadd_rn(loc, -double(idx));
+    if (ORDER == 1) {
+      if (s >= 0.5) idx = (idx == ng - 1) ? 0 : idx + 1;
+      ijk[0][a] = idx;
+      win[0][a] = 1.;
+    } else if (ORDER == 2) {
+      ijk[0][a] = idx;
+      ijk[1][a] = (idx == ng - 1) ? 0 : idx + 1;
+      win[0][a] = 1. - s;
+      win[1][a] = s;
+    } else if (ORDER == 3) {
+      if (s < 0.5) {
+        ijk[0][a] = (idx == 0) ? ng - 1 : idx - 1;
+        ijk[1][a] = idx;
+        ijk[2][a] = (idx == ng - 1) ? 0 : idx + 1;
+        win[0][a] = 0.5 * (0.5 - s) * (0.5 - s);
+        win[1][a] = 0.75 - s * s;
+        win[2][a] = 0.5 * (0.5 + s) * (0.5 + s);
+      } else if (!shadow) {
+        ijk[0][a] = idx;
+        ijk[1][a] = (idx == ng - 1) ? 0 : idx + 1;
+        ijk[2][a] = (ijk[1][a] == ng - 1) ? 0 : ijk[1][a] + 1;
+        double sp = 1. - s;
+        win[0][a] = 0.5 * (0.5 + sp) * (0.5 + sp);
+        win[1][a] = 0.75 - sp * sp;
+        win[2][a] = 0.5 * (0.5 - sp) * (0.5 - sp);
+      } else {
+        // The reference's shadow pass tests the base index for the last
+        // cell too (field.cpp:944-950): kept for identical fields.
+        ijk[0][a] = idx;
+        ijk[1][a] = (idx == ng - 1) ? 0 : idx + 1;
+        ijk[2][a] = (idx == ng - 1) ? 0 : ijk[1][a] + 1;
+        double sp = 1. - s;
+        win[0][a] = 0.5 * (0.5 + sp) * (0.5 + sp);
+        win[1][a] = 0.75 - sp * sp;
+        win[2][a] = 0.5 * (0.5 - sp) * (0.5 - sp);
+      }
+    } else {
+      ijk[0][a] = (idx == 0) ? ng - 1 : idx - 1;
+      ijk[1][a] = idx;
+      ijk[2][a] = (idx == ng - 1) ? 0 : idx + 1;
+      ijk[3][a] = (ijk[2][a] == ng - 1) ? 0 : ijk[2][a] + 1;
+      double sm = 1. - s;
+      win[0][a] = 1. / 6 * sm * sm * sm;
+      win[1][a] = 1. / 6 * (4. - 6. * s * s + 3. * s * s * s);
+      win[2][a] = 1. / 6 * (4. - 6. * sm * sm + 3. * sm * sm * sm);
+      win[3][a] = 1. / 6 * s * s * s;
+    }
+  }
+#pragma unroll
+  for (int il = 0; il < ORDER; il++) {
+#pragma unroll
+    for (int jl = 0; jl < ORDER; jl++) {
+      const long long row =
+          ((long long)ijk[il][0] * g.n[1] + ijk[jl][1]) * g.n[2];
+      const double wij = win[il][0] * win[jl][1];
+#pragma unroll
+      for (int kl = 0; kl < ORDER; kl++) {
+        const long long gid = row + ijk[kl][2];
+        // Same guard as the reference: only the flattened index is
+        // checked (a particle at x = L lands in a neighbouring row).
+        if (gid < 0 || gid >= g.nmesh) continue;
+        const double wv = wij * win[kl][2];
+        T* cell = reinterpret_cast<T*>(mesh + gid);
+        if (cplx_w == 2) {           // real weight into the imaginary part
+          unsafeAtomicAdd(cell + 1, T(wre * wv));
+          continue;
+        }
+        unsafeAtomicAdd(cell, T(wre * wv));
+        if (cplx_w) unsafeAtomicAdd(cell + 1, T(wim * wv));
+      }
+    }
+  }
+}
+
+// Particles [*first, n) (all of them when `first` is null), weights divided
+// by V_cell and multiplied by `scale` (e.g. -alpha for randoms).
 template <typename T, int ORDER>
 __global__ void __launch_bounds__(256)
 k_assign(c2<T>* __restrict__ mesh, DevParticles p, Geom g, int mode, int ell,
@@ -63,93 +153,9 @@ k_assign(c2<T>* __restrict__ mesh, DevParticles p, Geom g, int mode, int ell,
   for (long long pid = p0 + blockIdx.x * (long long)blockDim.x + threadIdx.x;
        pid < p.n; pid += (long long)gridDim.x * blockDim.x) {
     const double pos[3] = {p.x[pid], p.y[pid], p.z[pid]};
-    int ijk[ORDER][3];
-    double win[ORDER][3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      const int ng = g.n[a];
-      double loc = __ddiv_rn(__dmul_rn(double(ng), pos[a]), g.L[a]);
-      if (shadow) {
-        loc = __dadd_rn(loc, 0.5);
-        if (loc > ng) loc = __dadd_rn(loc, -double(ng));
-      }
-      int idx = int(loc);
-      double s = __dadd_rn(loc, -double(idx));
-      if (ORDER == 1) {
-        if (s >= 0.5) idx = (idx == ng - 1) ? 0 : idx + 1;
-        ijk[0][a] = idx;
-        win[0][a] = 1.;
-      } else if (ORDER == 2) {
-        ijk[0][a] = idx;
-        ijk[1][a] = (idx == ng - 1) ? 0 : idx + 1;
-        win[0][a] = 1. - s;
-        win[1][a] = s;
-      } else if (ORDER == 3) {
-        if (s < 0.5) {
-          ijk[0][a] = (idx == 0) ? ng - 1 : idx - 1;
-          ijk[1][a] = idx;
-          ijk[2][a] = (idx == ng - 1) ? 0 : idx + 1;
-          win[0][a] = 0.5 * (0.5 - s) * (0.5 - s);
-          win[1][a] = 0.75 - s * s;
-          win[2][a] = 0.5 * (0.5 + s) * (0.5 + s);
-        } else if (!shadow) {
-          ijk[0][a] = idx;
-          ijk[1][a] = (idx == ng - 1) ? 0 : idx + 1;
-          ijk[2][a] = (ijk[1][a] == ng - 1) ? 0 : ijk[1][a] + 1;
-          double sp = 1. - s;
-          win[0][a] = 0.5 * (0.5 + sp) * (0.5 + sp);
-          win[1][a] = 0.75 - sp * sp;
-          win[2][a] = 0.5 * (0.5 - sp) * (0.5 - sp);
-        } else {
-          // The reference's shadow pass tests the base index for the last
-          // cell too (field.cpp:944-950): kept for identical fields.
-          ijk[0][a] = idx;
-          ijk[1][a] = (idx == ng - 1) ? 0 : idx + 1;
-          ijk[2][a] = (idx == ng - 1) ? 0 : ijk[1][a] + 1;
-          double sp = 1. - s;
-          win[0][a] = 0.5 * (0.5 + sp) * (0.5 + sp);
-          win[1][a] = 0.75 - sp * sp;
-          win[2][a] = 0.5 * (0.5 - sp) * (0.5 - sp);
-        }
-      } else {
-        ijk[0][a] = (idx == 0) ? ng - 1 : idx - 1;
-        ijk[1][a] = idx;
-        ijk[2][a] = (idx == ng - 1) ? 0 : idx + 1;
-        ijk[3][a] = (ijk[2][a] == ng - 1) ? 0 : ijk[2][a] + 1;
-        double sm = 1. - s;
-        win[0][a] = 1. / 6 * sm * sm * sm;
-        win[1][a] = 1. / 6 * (4. - 6. * s * s + 3. * s * s * s);
-        win[2][a] = 1. / 6 * (4. - 6. * sm * sm + 3. * sm * sm * sm);
-        win[3][a] = 1. / 6 * s * s * s;
-      }
-    }
-    double2 wt = particle_weight(p, pid, mode, ell, m);
-    double wre = inv_vol_cell * wt.x * scale;
-    double wim = inv_vol_cell * wt.y * scale;
-#pragma unroll
-    for (int il = 0; il < ORDER; il++) {
-#pragma unroll
-      for (int jl = 0; jl < ORDER; jl++) {
-        const long long row =
-            ((long long)ijk[il][0] * g.n[1] + ijk[jl][1]) * g.n[2];
-        const double wij = win[il][0] * win[jl][1];
-#pragma unroll
-        for (int kl = 0; kl < ORDER; kl++) {
-          const long long gid = row + ijk[kl][2];
-          // Same guard as the reference: only the flattened index is
-          // checked (a particle at x = L lands in a neighbouring row).
-          if (gid < 0 || gid >= g.nmesh) continue;
-          const double wv = wij * win[kl][2];
-          T* cell = reinterpret_cast<T*>(mesh + gid);
-          if (cplx_w == 2) {           // real weight into the imaginary part
-            unsafeAtomicAdd(cell + 1, T(wre * wv));
-            continue;
-          }
-          unsafeAtomicAdd(cell, T(wre * wv));
-          if (cplx_w) unsafeAtomicAdd(cell + 1, T(wim * wv));
-        }
-      }
-    }
+    const double2 wt = particle_weight(p, pid, mode, ell, m);
+    assign_particle<T, ORDER>(mesh, pos, inv_vol_cell * wt.x * scale,
+                              inv_vol_cell * wt.y * scale, g, cplx_w, shadow);
   }
 }
 
@@ -1312,14 +1318,35 @@ k_tile_work(const unsigned int* __restrict__ offs, const unsigned int* __restric
 }
 
 // Window weights of a particle along the three axes and the tile-local
-// index (halo origin o0) of the first covered cell per axis.
-template <int ORDER>
-__device__ __forceinline__ void tile_stencil(const Geom& g, const int o0[3],
+// index (halo origin o0) of the first covered cell per axis.  SHADOW: the
+// half-cell-shifted position of interlacing, whose base cell is the
+// particle's own or the next one.  False for a particle whose cells are not
+// (index + offset) mod n there (k_assign's rules at the last cells: a base
+// index n, and the order-3 shadow rule of the last two cells), which the
+// caller assigns through assign_particle.
+template <int ORDER, bool SHADOW = false>
+__device__ __forceinline__ bool tile_stencil(const Geom& g, const int o0[3],
                                              double x, double y, double z,
                                              int lo[3], double win[ORDER][3]) {
   int idx[3];
   double s[3];
-  base_cell(g, x, y, z, idx, s);
+  bool regular = true;
+  if (SHADOW) {
+    const double pos[3] = {x, y, z};
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int ng = g.n[a];
+      double loc = __dadd_rn(__ddiv_rn(__dmul_rn(double(ng), pos[a]), g.L[a]), 0.5);
+      const bool wrap = loc > ng;
+      if (wrap) loc = __dadd_rn(loc, -double(ng));
+      idx[a] = int(loc);
+      s[a] = __dadd_rn(loc, -double(idx[a]));
+      regular = regular && idx[a] < ng && !(ORDER == 3 && s[a] >= 0.5 && idx[a] >= ng - 2);
+      if (wrap) idx[a] += ng;   // next to the particle's own cell n - 1
+    }
+  } else {
+    base_cell(g, x, y, z, idx, s);
+  }
 #pragma unroll
   for (int a = 0; a < 3; a++) {
     const double sa = s[a];
@@ -1352,6 +1379,7 @@ __device__ __forceinline__ void tile_stencil(const Geom& g, const int o0[3],
     }
     lo[a] = first - o0[a];
   }
+  return regular;
 }
 
 // Tile halo origin of work item wk.
@@ -1364,28 +1392,37 @@ __device__ __forceinline__ void tile_origin(const TileGeom& tg, int t, int o0[3]
   o0[2] = tz * TILE - 1;
 }
 
-// Periodic mesh cell of tile-local cell c.
+// Periodic mesh cell of tile-local cell c of a block of H cells per side.
+// Only cells that a particle of the tile touches are asked for: they lie
+// within [-1, n + 3] per axis, so one wrap is enough.
+template <int H = TILE_H>
 __device__ __forceinline__ long long tile_cell(const Geom& g, const int o0[3], int c) {
-  const int lz = c % TILE_H, ly = (c / TILE_H) % TILE_H, lx = c / (TILE_H * TILE_H);
+  const int lz = c % H, ly = (c / H) % H, lx = c / (H * H);
   int gx = o0[0] + lx, gy = o0[1] + ly, gz = o0[2] + lz;
-  gx = (gx % g.n[0] + g.n[0]) % g.n[0];
-  gy = (gy % g.n[1] + g.n[1]) % g.n[1];
-  gz = (gz % g.n[2] + g.n[2]) % g.n[2];
+  gx += gx < 0 ? g.n[0] : (gx >= g.n[0] ? -g.n[0] : 0);
+  gy += gy < 0 ? g.n[1] : (gy >= g.n[1] ? -g.n[1] : 0);
+  gz += gz < 0 ? g.n[2] : (gz >= g.n[2] ? -g.n[2] : 0);
   return ((long long)gx * g.n[1] + gy) * g.n[2] + gz;
 }
 
-template <typename T, int ORDER>
+// CPLX: complex weights (a second LDS block); SHADOW: the half-cell-shifted
+// pass of interlacing (stencils reach one cell further: a 12^3 block).  The
+// shadow pass used to go straight to the mesh, ORDER^3 global atomics per
+// particle (PCS on 256^3: 15 ms per 2e6 particles, 67 ms of the 111 ms of an
+// interlaced quadrupole); binned like the main pass it takes 0.23 ms.
+template <typename T, int ORDER, bool CPLX, bool SHADOW>
 __global__ void __launch_bounds__(256)
 k_assign_tiled(c2<T>* __restrict__ mesh, DevParticles p, Geom g, TileGeom tg,
                const TileWork* __restrict__ work, const unsigned int* __restrict__ meta,
                int mode, int ell, int m, double scale, int cplx_w) {
-  __shared__ double acc_re[TILE_CELLS];
-  __shared__ double acc_im[TILE_CELLS];
+  constexpr int H = TILE_H + (SHADOW ? 1 : 0), CELLS = H * H * H;
+  __shared__ double acc_re[CELLS];
+  __shared__ double acc_im[CPLX ? CELLS : 1];
   if (blockIdx.x >= meta[0]) return;   // grid sized by a bound
   const TileWork wk = work[blockIdx.x];
-  for (int c = threadIdx.x; c < TILE_CELLS; c += blockDim.x) {
+  for (int c = threadIdx.x; c < CELLS; c += blockDim.x) {
     acc_re[c] = 0.;
-    acc_im[c] = 0.;
+    if (CPLX) acc_im[c] = 0.;
   }
   int o0[3];
   tile_origin(tg, wk.tile, o0);
@@ -1395,36 +1432,42 @@ k_assign_tiled(c2<T>* __restrict__ mesh, DevParticles p, Geom g, TileGeom tg,
     const long long pid = wk.start + q;
     int lo[3];
     double win[ORDER][3];
-    tile_stencil<ORDER>(g, o0, p.x[pid], p.y[pid], p.z[pid], lo, win);
-    double2 wt = particle_weight(p, pid, mode, ell, m);
+    const bool regular =
+        tile_stencil<ORDER, SHADOW>(g, o0, p.x[pid], p.y[pid], p.z[pid], lo, win);
+    const double2 wt = particle_weight(p, pid, mode, ell, m);
     const double wre = inv_vol_cell * wt.x * scale;
     const double wim = inv_vol_cell * wt.y * scale;
+    if (SHADOW && !regular) {
+      const double pos[3] = {p.x[pid], p.y[pid], p.z[pid]};
+      assign_particle<T, ORDER>(mesh, pos, wre, wim, g, cplx_w, 1);
+      continue;
+    }
 #pragma unroll
     for (int il = 0; il < ORDER; il++) {
 #pragma unroll
       for (int jl = 0; jl < ORDER; jl++) {
-        const int row = ((lo[0] + il) * TILE_H + (lo[1] + jl)) * TILE_H + lo[2];
+        const int row = ((lo[0] + il) * H + (lo[1] + jl)) * H + lo[2];
         const double wij = win[il][0] * win[jl][1];
 #pragma unroll
         for (int kl = 0; kl < ORDER; kl++) {
           const double wv = wij * win[kl][2];
           atomicAdd(&acc_re[row + kl], wre * wv);
-          if (cplx_w == 1) atomicAdd(&acc_im[row + kl], wim * wv);
+          if (CPLX) atomicAdd(&acc_im[row + kl], wim * wv);
         }
       }
     }
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < TILE_CELLS; c += blockDim.x) {
-    const double vr = acc_re[c], vi = acc_im[c];
+  for (int c = threadIdx.x; c < CELLS; c += blockDim.x) {
+    const double vr = acc_re[c], vi = CPLX ? acc_im[c] : 0.;
     if (vr == 0. && vi == 0.) continue;
-    T* cell = reinterpret_cast<T*>(mesh + tile_cell(g, o0, c));
-    if (cplx_w == 2) {             // real weight into the imaginary part
+    T* cell = reinterpret_cast<T*>(mesh + tile_cell<H>(g, o0, c));
+    if (!CPLX && cplx_w == 2) {    // real weight into the imaginary part
       unsafeAtomicAdd(cell + 1, T(vr));
       continue;
     }
     unsafeAtomicAdd(cell, T(vr));
-    if (cplx_w) unsafeAtomicAdd(cell + 1, T(vi));
+    if (CPLX) unsafeAtomicAdd(cell + 1, T(vi));
   }
 }
 
