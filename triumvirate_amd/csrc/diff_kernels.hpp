@@ -166,22 +166,6 @@ struct LoadReal {
   }
 };
 
-// First-pass loader of FFT[2 a F G]: reads the shell field F and G(x)
-// (real parts), returns (2 a F G, 0) and adds a F^2 to gG (each cell is
-// loaded exactly once per transform, so the update is race-free).
-template <typename T>
-struct LoadShellCotangent {
-  const c2<T>* F;
-  const c2<T>* G;
-  T* gG;
-  double a;
-  __device__ c2<T> operator()(long long g, int, int, int) const {
-    const double f = double(F[g].x), gg = double(G[g].x);
-    gG[g] = T(double(gG[g]) + a * f * f);
-    return mk<T>(T(2. * a * f * gg), T(0));
-  }
-};
-
 // sum_x Re F(x)^2 Re G(x), per-block FP64 partials.
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
@@ -203,41 +187,104 @@ k_f2g_partials(const c2<T>* __restrict__ F, const c2<T>* __restrict__ G,
   if (threadIdx.x == 0) part[(long long)blockIdx.x * stride] = red[0];
 }
 
-// acc(k) += t(k) / W(k) on the shell of `band` (the predicate of LoadShell).
+// sum_x F_b(x)^2 Re G(x) of the two real fields of mesh blockIdx.y of a
+// packed slab: per-block FP64 partials part[blockIdx.x][2 gridDim.y].
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
-k_adj_shell_acc(c2<T>* __restrict__ acc, const c2<T>* __restrict__ t, Geom g,
-                AxisTables tab, ShellBand band) {
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-       c < g.nmesh; c += (long long)gridDim.x * blockDim.x) {
-    const int k = int(c % g.n[2]);
-    const long long ij = c / g.n[2];
-    const int j = int(ij % g.n[1]), i = int(ij / g.n[1]);
-    const double kx = grid_coord(i, g.n[0], g.dk[0]);
-    const double ky = grid_coord(j, g.n[1], g.dk[1]);
-    const double kz = grid_coord(k, g.n[2], g.dk[2]);
-    if (!band.contains(mag2_exact(kx, ky, kz))) continue;
-    const double iw = 1. / window_at(tab, i, j, k);
-    c2<T> a = acc[c], v = t[c];
-    acc[c] = mk<T>(T(double(a.x) + double(v.x) * iw),
-                   T(double(a.y) + double(v.y) * iw));
+k_f2g_packed(const c2<T>* __restrict__ F, const c2<T>* __restrict__ G, long long n,
+             double* __restrict__ part) {
+  __shared__ double red[2][RED_THREADS];
+  const c2<T>* f = F + blockIdx.y * n;
+  double s0 = 0., s1 = 0.;
+  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < n;
+       c += (long long)gridDim.x * blockDim.x) {
+    const c2<T> v = f[c];
+    const double g = double(G[c].x), x = double(v.x), y = double(v.y);
+    s0 += x * x * g;
+    s1 += y * y * g;
+  }
+  red[0][threadIdx.x] = s0;
+  red[1][threadIdx.x] = s1;
+  __syncthreads();
+  for (int h = RED_THREADS / 2; h > 0; h >>= 1) {
+    if (threadIdx.x < h) {
+      red[0][threadIdx.x] += red[0][threadIdx.x + h];
+      red[1][threadIdx.x] += red[1][threadIdx.x + h];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < 2)
+    part[((long long)blockIdx.x * gridDim.y + blockIdx.y) * 2 + threadIdx.x] =
+        red[threadIdx.x][0];
+}
+
+// Cotangents of the shell fields and of G: mesh p of the packed slab F
+// becomes 2 (a_2p F_2p + i a_2p+1 F_2p+1) G, and mesh nt sum_b a_b F_b^2.
+template <typename T>
+__global__ void __launch_bounds__(RED_THREADS)
+k_cotangents(c2<T>* __restrict__ F, const c2<T>* __restrict__ G, long long n, int nt,
+             const double* __restrict__ a) {
+  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < n;
+       c += (long long)gridDim.x * blockDim.x) {
+    const double g = double(G[c].x);
+    double s = 0.;
+    for (int p = 0; p < nt; p++) {
+      const c2<T> f = F[(long long)p * n + c];
+      const double x = double(f.x), y = double(f.y), a0 = a[2 * p], a1 = a[2 * p + 1];
+      s += a0 * x * x + a1 * y * y;
+      F[(long long)p * n + c] = mk<T>(T(2. * a0 * x * g), T(2. * a1 * y * g));
+    }
+    F[(long long)nt * n + c] = mk<T>(T(s), T(0));
   }
 }
 
-// acc(k) += t(k) s / W(k) on every mode.
+// acc(k) += [the spectrum of the cotangent of the bin holding k, + scale
+// times that of G's cotangent] / W(k), from the transformed slab of
+// k_cotangents on the mesh `c` to the full mesh `g` (window tables of g).
+// Bin b of the group is real field slot[b] of the slab (-1: not in it):
+// with P = FFT[u + i v], u(k) = (P(k) + P(-k)^*) / 2 and v(k) = (P(k) -
+// P(-k)^*) / 2i.  Each cell of c is one cell of g, so the update is
+// race-free.
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
-k_adj_all_acc(c2<T>* __restrict__ acc, const c2<T>* __restrict__ t, Geom g,
-              AxisTables tab, double s) {
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-       c < g.nmesh; c += (long long)gridDim.x * blockDim.x) {
-    const int k = int(c % g.n[2]);
-    const long long ij = c / g.n[2];
-    const int j = int(ij % g.n[1]), i = int(ij / g.n[1]);
-    const double f = s / window_at(tab, i, j, k);
-    c2<T> a = acc[c], v = t[c];
-    acc[c] = mk<T>(T(double(a.x) + double(v.x) * f),
-                   T(double(a.y) + double(v.y) * f));
+k_adj_acc(c2<T>* __restrict__ acc, const c2<T>* __restrict__ P, int nt, Geom g, Geom c,
+          AxisTables tab, const double* __restrict__ edge, int nb,
+          const int* __restrict__ slot, double scale) {
+  for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < c.nmesh;
+       q += (long long)gridDim.x * blockDim.x) {
+    const long long ij = q / c.n[2];
+    const int ix[3] = {int(ij / c.n[1]), int(ij % c.n[1]), int(q % c.n[2])};
+    int f[3], r[3];
+    double k[3];
+    bool edge_mode = false;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int m = shifted(ix[a], c.n[a]);
+      edge_mode |= c.n[a] < g.n[a] && ix[a] == c.n[a] / 2;
+      f[a] = m < 0 ? m + g.n[a] : m;
+      r[a] = ix[a] == 0 ? 0 : c.n[a] - ix[a];
+      k[a] = grid_coord(ix[a], c.n[a], c.dk[a]);
+    }
+    if (edge_mode) continue;   // beyond the products of any bin
+    const c2<T> t = P[(long long)nt * c.nmesh + q];
+    double re = scale * double(t.x), im = scale * double(t.y);
+    const int b = find_bin(edge, nb, mag2_exact(k[0], k[1], k[2]));
+    const int s = b < 0 ? -1 : slot[b];
+    if (s >= 0) {
+      const c2<T>* p = P + (long long)(s / 2) * c.nmesh;
+      const c2<T> u = p[q];
+      const c2<T> v = p[((long long)r[0] * c.n[1] + r[1]) * c.n[2] + r[2]];
+      if (s % 2 == 0) {
+        re += 0.5 * (double(u.x) + double(v.x));
+        im += 0.5 * (double(u.y) - double(v.y));
+      } else {
+        re += 0.5 * (double(u.y) + double(v.y));
+        im -= 0.5 * (double(u.x) - double(v.x));
+      }
+    }
+    const double iw = 1. / window_at(tab, f[0], f[1], f[2]);
+    c2<T>* o = acc + ((long long)f[0] * g.n[1] + f[1]) * g.n[2] + f[2];
+    *o = mk<T>(T(double(o->x) + re * iw), T(double(o->y) + im * iw));
   }
 }
 

@@ -260,6 +260,183 @@ void Context::flush() {
   for (auto& f : d) f();
 }
 
+// ---------------------------------------------------------------------------
+// Smaller meshes for band-limited pair sums
+// ---------------------------------------------------------------------------
+
+Geom mesh_of(const Geom& g, const int n[3]) {
+  Geom c = g;
+  for (int a = 0; a < 3; a++) {
+    c.n[a] = n[a];
+    c.dr[a] = g.L[a] / n[a];
+  }
+  c.nmesh = (long long)n[0] * n[1] * n[2];
+  c.vol_cell = c.vol / double(c.nmesh);
+  return c;
+}
+
+namespace {
+
+constexpr int ONES_MAX = 2048;
+
+// A table of ones per device, as long as the longest mesh axis.
+const double* ones_table(int dev) {
+  static std::mutex mu;
+  static std::map<int, std::unique_ptr<DevArray<double>>> cache;
+  std::lock_guard<std::mutex> lk(mu);
+  auto& t = cache[dev];
+  if (!t) {
+    auto d = std::make_unique<DevArray<double>>(ONES_MAX);
+    const std::vector<double> h(ONES_MAX, 1.);
+    TRVG_HIP(hipMemcpy(d->get(), h.data(), ONES_MAX * sizeof(double), hipMemcpyHostToDevice));
+    t = std::move(d);
+  }
+  return t->get();
+}
+
+bool pow2(int n) { return (n & (n - 1)) == 0; }
+
+// Cost of a pass along an axis relative to one of power-of-two length: the
+// mixed-radix passes of other lengths move a cell at about a quarter of
+// the rate (FP64, 200^3 against 256^3: 27 against 6 ps per cell).
+double axis_cost(int n) { return pow2(n) && n <= 1024 ? 1. : 4.; }
+
+// The cheapest mesh with m >= 2 K + 2 per axis (none longer than the full
+// mesh's): per axis the next power of two, the next even length with no
+// prime factor above 5, or the full length.
+void group_mesh(const Geom& g, const int K[3], int n[3], double& cells) {
+  int opt[3][3], no[3];
+  for (int a = 0; a < 3; a++) {
+    const int need = 2 * K[a] + 2;
+    no[a] = 0;
+    opt[a][no[a]++] = g.n[a];
+    int p = 16;
+    while (p < need) p *= 2;
+    if (p < g.n[a]) opt[a][no[a]++] = p;
+    for (int m = std::max(need + need % 2, 16); m < g.n[a] && m < p; m += 2) {
+      int r = m;
+      for (int q : {2, 3, 5})
+        while (r % q == 0) r /= q;
+      if (r == 1) { opt[a][no[a]++] = m; break; }
+    }
+  }
+  double best = HUGE_VAL;
+  for (int i = 0; i < no[0]; i++)
+    for (int j = 0; j < no[1]; j++)
+      for (int k = 0; k < no[2]; k++) {
+        const int m[3] = {opt[0][i], opt[1][j], opt[2][k]};
+        const double c = double(m[0]) * m[1] * m[2] *
+                         (axis_cost(m[0]) + axis_cost(m[1]) + axis_cost(m[2])) / 3.;
+        if (c < best) {
+          best = c;
+          for (int a = 0; a < 3; a++) n[a] = m[a];
+        }
+      }
+  cells = best;
+}
+
+}  // namespace
+
+std::vector<MeshGroup> plan_mesh_groups(const Geom& g, const trvg_binning& kb,
+                                        const std::vector<int>& ra,
+                                        const std::vector<int>& cb, bool split,
+                                        size_t cell_bytes) {
+  const int P = int(ra.size());
+  // Largest |index| along each axis of a mode below a bin's upper edge.
+  auto reach = [&](int b, int a) {
+    const double h = std::floor(kb.bin_edges[b + 1] / g.dk[a] * (1. + 1.e-9));
+    return h < g.n[a] / 2 ? int(std::max(h, 0.)) : g.n[a] / 2;
+  };
+  std::vector<int> order(P);
+  for (int d = 0; d < P; d++) order[d] = d;
+  auto top = [&](int d) { return kb.bin_edges[ra[d] + 1] + kb.bin_edges[cb[d] + 1]; };
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return top(x) < top(y); });
+  // Mesh of the pairs up to position j of that order.
+  std::vector<MeshGroup> upto(P);
+  std::vector<double> cells(P);
+  int K[3] = {0, 0, 0};
+  for (int j = 0; j < P; j++) {
+    for (int a = 0; a < 3; a++)
+      K[a] = std::max(K[a], reach(ra[order[j]], a) + reach(cb[order[j]], a));
+    if (!split && j + 1 < P) continue;
+    group_mesh(g, K, upto[j].n, cells[j]);
+    upto[j].coarse = false;
+    for (int a = 0; a < 3; a++) upto[j].coarse |= upto[j].n[a] < g.n[a];
+  }
+  // Cost in microseconds of pairs i..j on one mesh: about twelve launches
+  // (two more to truncate the sources), then six traversals per transformed
+  // field (three passes, the pair sum) and per G, at 4.5 TB/s.
+  auto cost = [&](int i, int j) {
+    return 60. + (upto[j].coarse ? 12. : 0.) +
+           cells[j] * double(cell_bytes) * (6. * (j - i + 1) + 8.) / 4.5e6;
+  };
+  std::vector<MeshGroup> out;
+  if (P == 0) return out;
+  std::vector<double> best(P + 1, HUGE_VAL);
+  std::vector<int> from(P + 1, 0);
+  best[0] = 0.;
+  for (int j = 0; j < P; j++) {
+    if (!split && j + 1 < P) continue;
+    for (int i = split ? 0 : j - P + 1; i <= (split ? j : 0); i++) {
+      const double c = best[i] + cost(i, j);
+      if (c < best[j + 1]) { best[j + 1] = c; from[j + 1] = i; }
+    }
+  }
+  for (int j = P; j > 0; j = from[j]) {
+    MeshGroup gr = upto[j - 1];
+    gr.pairs.assign(order.begin() + from[j], order.begin() + j);
+    std::sort(gr.pairs.begin(), gr.pairs.end());
+    out.push_back(std::move(gr));
+  }
+  return out;
+}
+
+MeshScope::MeshScope(Context& ctx, const Geom& g) : ctx_(ctx), g_(ctx.g), tab_(ctx.tab) {
+  const double* one = ones_table(ctx.dev);
+  ctx.g = g;
+  ctx.tab = AxisTables{{one, one, one}, {one, one, one}, {one, one, one}, 1, 0};
+}
+
+namespace {
+
+template <typename T>
+__global__ void __launch_bounds__(RED_THREADS)
+k_truncate_modes(const c2<T>* __restrict__ src, Geom g, AxisTables tab, Geom c,
+                 c2<T>* __restrict__ out) {
+  for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < c.nmesh;
+       q += (long long)gridDim.x * blockDim.x) {
+    const long long ij = q / c.n[2];
+    const int ix[3] = {int(ij / c.n[1]), int(ij % c.n[1]), int(q % c.n[2])};
+    int f[3];
+    bool edge = false;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int m = shifted(ix[a], c.n[a]);
+      edge |= c.n[a] < g.n[a] && ix[a] == c.n[a] / 2;
+      f[a] = m < 0 ? m + g.n[a] : m;
+    }
+    if (edge) {
+      out[q] = mk<T>(T(0), T(0));
+      continue;
+    }
+    const c2<T> v = src[((long long)f[0] * g.n[1] + f[1]) * g.n[2] + f[2]];
+    const double iw = 1. / window_at(tab, f[0], f[1], f[2]);
+    out[q] = mk<T>(T(double(v.x) * iw), T(double(v.y) * iw));
+  }
+}
+
+}  // namespace
+
+template <typename T>
+void truncate_modes(Context& ctx, const c2<T>* src, const Geom& c, c2<T>* out) {
+  ProfScope ps(ctx, KC_MISC, 2. * double(c.nmesh) * sizeof(c2<T>));
+  hipLaunchKernelGGL((k_truncate_modes<T>), dim3(grid_for(ctx, c.nmesh)), dim3(RED_THREADS), 0,
+                     ctx.stream, src, ctx.g, ctx.tab, c, out);
+  TRVG_LAUNCH_CHECK();
+}
+template void truncate_modes<double>(Context&, const double2*, const Geom&, double2*);
+template void truncate_modes<float>(Context&, const float2*, const Geom&, float2*);
+
 Context::Context(const trvg_params& params) : p(params) {
   if (p.device >= 0) TRVG_HIP(hipSetDevice(p.device));
   g = make_geom(p);

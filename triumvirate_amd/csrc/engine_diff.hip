@@ -6,7 +6,9 @@
 // real mesh delta(x) (the unweighted field fluctuation of
 // field.cpp:1235-1243 when delta comes from trvg_diff_assign minus the
 // mean).  Shell fields are recomputed in the backward pass instead of being
-// stored.  Device pointers in, host vectors of per-bin values out.
+// stored.  Bins whose products fit a smaller mesh run there (MeshGroup), two
+// real shells per transform.  Device pointers in, host vectors of per-bin
+// values out.
 #include <cmath>
 #include <vector>
 
@@ -15,95 +17,150 @@
 
 namespace trvg {
 
+namespace {
+
+// The bins that share one mesh (every bin pairs with itself only) and their
+// fields there: G(x) and the real shell fields F_b, two per complex mesh
+// (bin bins[2p + c] is component c of mesh p).  The slab has one more mesh,
+// for the cotangent of G in the backward pass.
 template <typename T>
-static void diff_common_fields(Context& ctx, const T* mesh, c2<T>* D, c2<T>* G) {
-  const Geom& g = ctx.g;
-  fft3d<T>(ctx, D, LoadReal<T>{mesh, T(g.vol_cell)}, -1,
-           double(g.nmesh) * sizeof(T));
-  fft3d<T>(ctx, G, LoadDeconv<T, T>{D, ctx.tab, 1. / g.vol}, +1);
+struct DiffGroup {
+  std::vector<int> bins;
+  Geom g;
+  bool coarse;
+  int nt;
+  DevArray<c2<T>> D, G, F;
+};
+
+// D(k) of the mesh, then per group G and the shells.
+template <typename T>
+std::vector<DiffGroup<T>> diff_groups(Context& ctx, const trvg_binning& kb, const T* mesh,
+                                      const std::vector<int>& nmodes) {
+  const Geom g = ctx.g;
+  std::vector<int> all(kb.num_bins);
+  for (int b = 0; b < kb.num_bins; b++) all[b] = b;
+  DevArray<c2<T>> D(g.nmesh);
+  fft3d<T>(ctx, D.get(), LoadReal<T>{mesh, T(g.vol_cell)}, -1, double(g.nmesh) * sizeof(T));
+  std::vector<DiffGroup<T>> out;
+  for (const MeshGroup& gr : plan_mesh_groups(g, kb, all, all, true, sizeof(c2<T>))) {
+    DiffGroup<T> d;
+    d.bins = gr.pairs;   // pair b is bin b with itself
+    d.coarse = gr.coarse;
+    d.g = gr.coarse ? mesh_of(g, gr.n) : g;
+    d.nt = (int(d.bins.size()) + 1) / 2;
+    const c2<T>* src = D.get();
+    if (gr.coarse) {
+      d.D.reset(d.g.nmesh);
+      truncate_modes<T>(ctx, D.get(), d.g, d.D.get());
+      src = d.D.get();
+    }
+    std::unique_ptr<MeshScope> scope;
+    if (gr.coarse) scope = std::make_unique<MeshScope>(ctx, d.g);
+    d.G.reset(d.g.nmesh);
+    fft3d<T>(ctx, d.G.get(), LoadDeconv<T, T>{src, ctx.tab, 1. / g.vol}, +1);
+    d.F.reset(size_t(d.nt + 1) * d.g.nmesh);
+    shell_slab_ifft<T, T>(ctx, d.F.get(), src, kb, d.bins, nmodes, 0, 0, true);
+    out.push_back(std::move(d));
+  }
+  ctx.keep_until_flush(std::move(D));
+  return out;
 }
 
-template <typename T>
-static void diff_shell(Context& ctx, const c2<T>* D, c2<T>* F,
-                       const trvg_binning& kb, int b, int nmodes) {
-  LoadShell<T, T> ls{D, ctx.tab, ctx.g,
-                     shell_band(kb.bin_edges[b], kb.bin_edges[b + 1]), 0, 0};
-  Prune pr = make_prune(ctx.g, kb.bin_edges[b + 1]);
-  fft3d<T>(ctx, F, ls, +1, double(nmodes) * sizeof(c2<T>), &pr);
-}
+}  // namespace
 
 template <typename T>
 std::vector<double> diff_bispec_forward(Context& ctx, const trvg_binning& kb,
                                         double norm, const T* mesh,
                                         std::vector<int>& nmodes) {
-  const Geom& g = ctx.g;
-  const long long nm = g.nmesh;
-  const int nb = kb.num_bins;
   ShellStats ss = shell_stats(ctx, kb);
   nmodes = ss.nmodes;
-  DevArray<c2<T>> D(nm), G(nm), F(nm);
-  diff_common_fields<T>(ctx, mesh, D.get(), G.get());
-  const unsigned grid = grid_for(ctx, nm, 4);
-  DevArray<double> part((size_t)grid * nb), sums(nb);   // [grid][nb]
-  for (int b = 0; b < nb; b++) {
-    diff_shell<T>(ctx, D.get(), F.get(), kb, b, ss.nmodes[b]);
-    ProfScope ps(ctx, KC_PAIR_REDUCE, 2. * double(nm) * sizeof(c2<T>));
-    hipLaunchKernelGGL((k_f2g_partials<T>), dim3(grid), dim3(RED_THREADS), 0,
-                       ctx.stream, F.get(), G.get(), nm, part.get() + b, nb);
+  std::vector<DiffGroup<T>> groups = diff_groups<T>(ctx, kb, mesh, ss.nmodes);
+  std::vector<const double*> h;
+  for (DiffGroup<T>& d : groups) {
+    const int nv = 2 * d.nt;
+    const unsigned grid = grid_for(ctx, d.g.nmesh, 4);
+    DevArray<double> part((size_t)grid * nv), sums(nv);   // [grid][nv]
+    ProfScope ps(ctx, KC_PAIR_REDUCE, double(d.nt + 1) * double(d.g.nmesh) * sizeof(c2<T>));
+    hipLaunchKernelGGL((k_f2g_packed<T>), dim3(grid, unsigned(d.nt)), dim3(RED_THREADS), 0,
+                       ctx.stream, d.F.get(), d.G.get(), d.g.nmesh, part.get());
     TRVG_LAUNCH_CHECK();
+    reduce_cols(ctx, part.get(), int(grid), nv, sums.get());
+    h.push_back(ctx.download(sums.get(), nv));
+    ctx.keep_until_flush(std::move(part));
+    ctx.keep_until_flush(std::move(sums));
   }
-  reduce_cols(ctx, part.get(), int(grid), nb, sums.get());
-  std::vector<double> h(nb);
-  TRVG_HIP(hipMemcpyAsync(h.data(), sums.get(), nb * 8, hipMemcpyDeviceToHost, ctx.stream));
-  TRVG_HIP(hipStreamSynchronize(ctx.stream));
-  std::vector<double> out(nb);
-  for (int b = 0; b < nb; b++) {
-    const double n = double(ss.nmodes[b]);
-    out[b] = norm * g.vol_cell * h[b] / (n * n);   // NaN for an empty bin
-  }
+  ctx.flush();
+  std::vector<double> out(kb.num_bins);
+  for (size_t q = 0; q < groups.size(); q++)
+    for (size_t i = 0; i < groups[q].bins.size(); i++) {
+      const int b = groups[q].bins[i];
+      const double n = double(ss.nmodes[b]);
+      out[b] = norm * groups[q].g.vol_cell * h[q][i] / (n * n);   // NaN for an empty bin
+    }
   return out;
 }
 
 template <typename T>
 void diff_bispec_backward(Context& ctx, const trvg_binning& kb, double norm,
                           const T* mesh, const double* grad_bk, T* grad_mesh) {
-  const Geom& g = ctx.g;
+  const Geom g = ctx.g;
   const long long nm = g.nmesh;
   const int nb = kb.num_bins;
   ShellStats ss = shell_stats(ctx, kb);
-  DevArray<c2<T>> D(nm), G(nm), F(nm), acc(nm);
-  DevArray<T> gG(nm);
-  diff_common_fields<T>(ctx, mesh, D.get(), G.get());
+  std::vector<DiffGroup<T>> groups = diff_groups<T>(ctx, kb, mesh, ss.nmodes);
+  DevArray<c2<T>> acc(nm);
   const unsigned grid = grid_for(ctx, nm);
   hipLaunchKernelGGL((k_zero<T>), dim3(grid), dim3(RED_THREADS), 0, ctx.stream,
                      acc.get(), nm);
   TRVG_LAUNCH_CHECK();
-  hipLaunchKernelGGL((k_zero_real<T>), dim3(grid), dim3(RED_THREADS), 0,
-                     ctx.stream, gG.get(), nm);
-  TRVG_LAUNCH_CHECK();
-  for (int b = 0; b < nb; b++) {
-    const double n = double(ss.nmodes[b]);
-    if (grad_bk[b] == 0. || ss.nmodes[b] == 0) continue;
-    const double a = grad_bk[b] * norm * g.vol_cell / (n * n);
-    diff_shell<T>(ctx, D.get(), F.get(), kb, b, ss.nmodes[b]);
-    // In place: F <- FFT[2 a F G]; gG += a F^2.
-    fft3d<T>(ctx, F.get(), LoadShellCotangent<T>{F.get(), G.get(), gG.get(), a}, -1,
-             double(nm) * (2. * sizeof(c2<T>) + 2. * sizeof(T)));
-    ProfScope ps(ctx, KC_MISC, 3. * double(nm) * sizeof(c2<T>));
-    hipLaunchKernelGGL((k_adj_shell_acc<T>), dim3(grid), dim3(RED_THREADS), 0,
-                       ctx.stream, acc.get(), F.get(), g, ctx.tab,
-                       shell_band(kb.bin_edges[b], kb.bin_edges[b + 1]));
+  // Thresholds of |k|^2 between the bins (bin b: [edge[b], edge[b + 1])).
+  std::vector<double> edge(nb + 1);
+  for (int b = 0; b <= nb; b++) edge[b] = sq_threshold(kb.bin_edges[b]);
+  DevArray<double> dedge(nb + 1);
+  ctx.upload(dedge.get(), edge.data(), nb + 1);
+  bool all_coarse = true;
+  for (DiffGroup<T>& d : groups) {
+    all_coarse = all_coarse && d.coarse;
+    std::vector<double> a(2 * d.nt, 0.);
+    std::vector<int> slot(nb, -1);
+    for (size_t i = 0; i < d.bins.size(); i++) {
+      const int b = d.bins[i];
+      const double n = double(ss.nmodes[b]);
+      if (grad_bk[b] == 0. || ss.nmodes[b] == 0) continue;
+      a[i] = grad_bk[b] * norm * d.g.vol_cell / (n * n);
+      slot[b] = int(i);
+    }
+    DevArray<double> da(a.size());
+    DevArray<int> dslot(nb);
+    ctx.upload(da.get(), a.data(), a.size());
+    ctx.upload(dslot.get(), slot.data(), nb);
+    {
+      ProfScope ps(ctx, KC_MISC, (2. * d.nt + 2.) * double(d.g.nmesh) * sizeof(c2<T>));
+      hipLaunchKernelGGL((k_cotangents<T>), dim3(grid_for(ctx, d.g.nmesh)), dim3(RED_THREADS),
+                         0, ctx.stream, d.F.get(), d.G.get(), d.g.nmesh, d.nt, da.get());
+      TRVG_LAUNCH_CHECK();
+    }
+    {
+      std::unique_ptr<MeshScope> scope;
+      if (d.coarse) scope = std::make_unique<MeshScope>(ctx, d.g);
+      slab_fft<T>(ctx, d.F.get(), d.nt + 1);
+    }
+    ProfScope ps(ctx, KC_MISC, 3. * double(d.g.nmesh) * sizeof(c2<T>));
+    hipLaunchKernelGGL((k_adj_acc<T>), dim3(grid_for(ctx, d.g.nmesh)), dim3(RED_THREADS), 0,
+                       ctx.stream, acc.get(), d.F.get(), d.nt, g, d.g, ctx.tab, dedge.get(),
+                       nb, dslot.get(), 1. / g.vol);
     TRVG_LAUNCH_CHECK();
+    ctx.keep_until_flush(std::move(da));
+    ctx.keep_until_flush(std::move(dslot));
   }
-  fft3d<T>(ctx, F.get(), LoadReal<T>{gG.get(), T(1)}, -1, double(nm) * sizeof(T));
-  hipLaunchKernelGGL((k_adj_all_acc<T>), dim3(grid), dim3(RED_THREADS), 0,
-                     ctx.stream, acc.get(), F.get(), g, ctx.tab, 1. / g.vol);
-  TRVG_LAUNCH_CHECK();
-  fft3d<T>(ctx, acc.get(), LoadSame<T>{acc.get()}, +1);
+  // The products F_b^2 reach twice the highest bin edge.
+  Prune pr{};
+  if (all_coarse) pr = make_prune(g, 2. * kb.bin_edges[nb]);
+  fft3d<T>(ctx, acc.get(), LoadSame<T>{acc.get()}, +1, -1., &pr);
   hipLaunchKernelGGL((k_real_part<T>), dim3(grid), dim3(RED_THREADS), 0,
                      ctx.stream, grad_mesh, acc.get(), nm, g.vol_cell);
   TRVG_LAUNCH_CHECK();
-  TRVG_HIP(hipStreamSynchronize(ctx.stream));
+  ctx.flush();
 }
 
 template <typename T, int ORDER>

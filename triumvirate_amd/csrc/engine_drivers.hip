@@ -972,12 +972,13 @@ static cplx ipow(int n) {
 template <typename T>
 struct ShellSlab {
   int ell = -1, m = 0;
+  int n[3] = {0, 0, 0};     // mesh
   std::vector<int> index;   // bin -> field index in `data`, -1 if absent
   int nfields = 0;
   bool packed = false;      // real fields, two per complex mesh
   DevArray<c2<T>> data;
-  bool covers(int l, int mm, const std::vector<int>& bins) const {
-    if (ell != l || m != mm) return false;
+  bool covers(const Geom& g, int l, int mm, const std::vector<int>& bins) const {
+    if (ell != l || m != mm || n[0] != g.n[0] || n[1] != g.n[1] || n[2] != g.n[2]) return false;
     for (int b : bins)
       if (b >= int(index.size()) || index[b] < 0) return false;
     return true;
@@ -997,7 +998,7 @@ class SlabCache {
   ShellSlab<T>* get(Context& ctx, int l, int m, const std::vector<int>& bins,
                     int nb, const ShellSlab<T>* keep, bool packed, Make&& make) {
     for (size_t i = 0; i < entries_.size(); i++)
-      if (entries_[i]->covers(l, m, bins)) {
+      if (entries_[i]->covers(ctx.g, l, m, bins)) {
         auto e = std::move(entries_[i]);      // move to the back (MRU)
         entries_.erase(entries_.begin() + i);
         entries_.push_back(std::move(e));
@@ -1013,6 +1014,7 @@ class SlabCache {
     auto e = std::make_unique<ShellSlab<T>>();
     e->ell = l;
     e->m = m;
+    for (int a = 0; a < 3; a++) e->n[a] = ctx.g.n[a];
     e->index.assign(nb, -1);
     e->nfields = int(bins.size());
     e->packed = packed;
@@ -1068,7 +1070,7 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
                                      const trvg_binning& kb,
                                      const std::vector<Multipole>& mps,
                                      SurveyPrefill* pre) {
-  const Geom& g = ctx.g;
+  const Geom g = ctx.g;   // a copy: the pair sums may run on another mesh
   const long long nm = g.nmesh;
   const double alpha = survey ? d.wstotal / r->wstotal : 1.;
   const int nb = kb.num_bins;
@@ -1117,11 +1119,25 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
   // multipole.
   int t_ell = -2, t_m = 0;
   cplx t_sbar(0., 0.);
-  SlabCache<T> slabs(mps.size() > 1 ? 3 : 2);
-  auto make_shell = [&](int l, int mm) {
-    return [&, l, mm](c2<T>* base, const std::vector<int>& bins) {
-      shell_slab_ifft<T>(ctx, base, dn00.get(), kb, bins, ss.nmodes, l, mm,
-                         real_shells(l, mm));
+  // Meshes of each multipole's pair sums, and dn00(k) / W(k) on them.
+  std::vector<std::vector<MeshGroup>> plans;
+  size_t ngroups = 1;
+  long long nm_coarse = 0;
+  for (const Multipole& mp : mps) {
+    std::vector<int> ra, cb;
+    pair_bins(mp.shape, nb, mp.idx_bin, ra, cb);
+    const bool split = mp.shape != TRVG_SHAPE_FULL && mp.shape != TRVG_SHAPE_TRIU;
+    plans.push_back(plan_mesh_groups(g, kb, ra, cb, split, sizeof(c2<T>)));
+    ngroups = std::max(ngroups, plans.back().size());
+    for (const MeshGroup& gr : plans.back())
+      if (gr.coarse) nm_coarse = std::max(nm_coarse, mesh_of(g, gr.n).nmesh);
+  }
+  std::map<std::vector<int>, DevArray<double2>> coarse00;
+  DevArray<double2> coarseLM;
+  SlabCache<T> slabs((mps.size() > 1 ? 3 : 2) * ngroups);
+  auto make_shell = [&](const double2* src, int l, int mm) {
+    return [&, src, l, mm](c2<T>* base, const std::vector<int>& bins) {
+      shell_slab_ifft<T, double>(ctx, base, src, kb, bins, ss.nmodes, l, mm, real_shells(l, mm));
     };
   };
 
@@ -1146,7 +1162,7 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
     std::vector<int> ra, cb;
     pair_bins(p.shape, nb, p.idx_bin, ra, cb);
     const int dim = int(ra.size());
-    std::vector<int> rows = distinct(ra), cols = distinct(cb);
+    const std::vector<MeshGroup>& plan = plans[results.size()];
 
     Result out;
     out.dim = dim;
@@ -1183,33 +1199,59 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
         NLMp = NLM.get();
       }
 
-      // G_LM(x): compensated, inverse-transformed (threept.cpp:452-459).
-      LoadDeconv<T, double> ldg{dnLMp, ctx.tab, 1. / g.vol};
-      fft3d<T>(ctx, G.get(), ldg, +1, double(nm) * sizeof(double2));
-
       // G_LM is real for M = 0 (real weights Y_L0) and in a periodic box.
       const bool g_real = !survey || tm.M == 0;
-      // Shell fields F_a (l1, m1) for the row bins, F_b (l2, m2) for columns.
-      ShellSlab<T>* A = slabs.get(ctx, p.ell1, tm.m1, rows, nb, nullptr,
-                                  real_shells(p.ell1, tm.m1), make_shell(p.ell1, tm.m1));
-      ShellSlab<T>* B = slabs.get(ctx, p.ell2, tm.m2, cols, nb, A,
-                                  real_shells(p.ell2, tm.m2), make_shell(p.ell2, tm.m2));
-      std::vector<int2> pairs(dim);
-      for (int dv = 0; dv < dim; dv++)
-        pairs[dv] = make_int2(A->index[ra[dv]], B->index[cb[dv]]);
-      // Results arrive at the flush after the last term (the sinks add
-      // into `out`, which outlives them).
       const double coupling = tm.coupling, f_mirror = tm.f_mirror;
-      pair_reduce<T>(ctx, A->data.get(), A->nfields, A->packed, B->data.get(),
-                     B->nfields, B->packed, G.get(), g_real, pairs,
-                     [&out, &ra, &cb, &ss, dim, coupling, f_mirror,
-                      vc = g.vol_cell](std::vector<cplx>&& S) {
-                       for (int dv = 0; dv < dim; dv++) {
-                         cplx sv = S[dv] / (double(ss.nmodes[ra[dv]]) *
-                                            double(ss.nmodes[cb[dv]]));
-                         out.raw[dv] += coupling * vc * (sv + f_mirror * std::conj(sv));
-                       }
-                     });
+      for (const MeshGroup& gr : plan) {
+        const double2 *src00 = dn00.get(), *srcLM = dnLMp;
+        const Geom gc = gr.coarse ? mesh_of(g, gr.n) : g;
+        if (gr.coarse) {
+          DevArray<double2>& c00 = coarse00[{gr.n[0], gr.n[1], gr.n[2]}];
+          if (!c00.get()) {
+            c00.reset(gc.nmesh);
+            truncate_modes<double>(ctx, dn00.get(), gc, c00.get());
+          }
+          src00 = srcLM = c00.get();
+          if (dnLMp != dn00.get()) {
+            if (!coarseLM.get()) coarseLM.reset(nm_coarse);
+            truncate_modes<double>(ctx, dnLMp, gc, coarseLM.get());
+            srcLM = coarseLM.get();
+          }
+        }
+        std::unique_ptr<MeshScope> scope;
+        if (gr.coarse) scope = std::make_unique<MeshScope>(ctx, gc);
+        std::vector<int> gra, gcb;
+        for (int dv : gr.pairs) { gra.push_back(ra[dv]); gcb.push_back(cb[dv]); }
+        const std::vector<int> rows = distinct(gra), cols = distinct(gcb);
+
+        // G_LM(x): compensated, inverse-transformed (threept.cpp:452-459).
+        LoadDeconv<T, double> ldg{srcLM, ctx.tab, 1. / g.vol};
+        fft3d<T>(ctx, G.get(), ldg, +1, double(gc.nmesh) * sizeof(double2));
+
+        // Shell fields F_a (l1, m1) for the row bins, F_b (l2, m2) for columns.
+        ShellSlab<T>* A =
+            slabs.get(ctx, p.ell1, tm.m1, rows, nb, nullptr, real_shells(p.ell1, tm.m1),
+                      make_shell(src00, p.ell1, tm.m1));
+        ShellSlab<T>* B =
+            slabs.get(ctx, p.ell2, tm.m2, cols, nb, A, real_shells(p.ell2, tm.m2),
+                      make_shell(src00, p.ell2, tm.m2));
+        std::vector<int2> pairs(gra.size());
+        for (size_t d = 0; d < gra.size(); d++)
+          pairs[d] = make_int2(A->index[gra[d]], B->index[gcb[d]]);
+        // Results arrive at the flush after the last term (the sinks add
+        // into `out`, which outlives them).
+        pair_reduce<T>(ctx, A->data.get(), A->nfields, A->packed, B->data.get(),
+                       B->nfields, B->packed, G.get(), g_real, pairs,
+                       [&out, &ra, &cb, &ss, dvs = gr.pairs, coupling, f_mirror,
+                        vc = gc.vol_cell](std::vector<cplx>&& S) {
+                         for (size_t d = 0; d < dvs.size(); d++) {
+                           const int dv = dvs[d];
+                           cplx sv = S[d] / (double(ss.nmodes[ra[dv]]) *
+                                             double(ss.nmodes[cb[dv]]));
+                           out.raw[dv] += coupling * vc * (sv + f_mirror * std::conj(sv));
+                         }
+                       });
+      }
 
       // Shot noise (threept.cpp:771-966).
       const cplx Sbar = survey ? sbar.at({p.ELL, tm.M}) : cplx(double(d.n), 0.);

@@ -71,6 +71,7 @@ static size_t fft_smem(bool row_flags) {
 template <class Loader> struct ZRegLoader : std::false_type {};
 template <> struct ZRegLoader<LoadMaskedZBatch<float>> : std::true_type {};
 template <> struct ZRegLoader<LoadSame<float>> : std::true_type {};
+template <> struct ZRegLoader<LoadSameBatch<float>> : std::true_type {};
 
 template <typename T, int LOGN, class Loader>
 constexpr bool use_zreg() {
@@ -660,8 +661,8 @@ static std::shared_ptr<const ShellPlan> shell_plan(Context& ctx, const trvg_binn
   return pl;
 }
 
-template <typename T>
-void shell_slab_ifft(Context& ctx, c2<T>* base, const double2* src,
+template <typename T, typename S>
+void shell_slab_ifft(Context& ctx, c2<T>* base, const c2<S>* src,
                      const trvg_binning& kb, const std::vector<int>& bins,
                      const std::vector<int>& nmodes, int ell, int m, bool packed) {
   const Geom& g = ctx.g;
@@ -673,14 +674,59 @@ void shell_slab_ifft(Context& ctx, c2<T>* base, const double2* src,
   const int2* py = px + pl->nx;
   const int2* pz = py + pl->ny;
   if (packed) {
-    LoadShellPairBatch<T, double> ld{src, ctx.tab, g, pl->bands.get(), ell, m};
+    LoadShellPairBatch<T, S> ld{src, ctx.tab, g, pl->bands.get(), ell, m};
     xfirst_passes<T>(ctx, base, ld, pl->kc.get(), px, pl->nx, py, pl->ny, pz, pl->nz,
                      pl->bx, pl->by, pl->bz);
   } else {
-    LoadShellBatch<T, double> ld{src, ctx.tab, g, pl->bands.get(), ell, m};
+    LoadShellBatch<T, S> ld{src, ctx.tab, g, pl->bands.get(), ell, m};
     xfirst_passes<T>(ctx, base, ld, pl->kc.get(), px, pl->nx, py, pl->ny, pz, pl->nz,
                      pl->bx, pl->by, pl->bz);
   }
+}
+
+// Forward transforms in place of the nf meshes at `base`, all of them per
+// pass in one launch (work lists cached per device, geometry and nf).
+template <typename T>
+void slab_fft(Context& ctx, c2<T>* base, int nf) {
+  const Geom& g = ctx.g;
+  std::vector<double> key = {double(ctx.dev), double(sizeof(T)), double(nf)};
+  for (int a = 0; a < 3; a++) key.push_back(g.n[a]);
+  static std::mutex mu;
+  static std::map<std::vector<double>, std::shared_ptr<ShellPlan>> cache;
+  std::shared_ptr<ShellPlan> plan;
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = cache.find(key);
+    if (it != cache.end()) plan = it->second;
+  }
+  if (!plan) {
+    std::vector<int2> w;
+    plan = std::make_shared<ShellPlan>();
+    int* count[3] = {&plan->nx, &plan->ny, &plan->nz};
+    for (int a = 0; a < 3; a++) {
+      const long long nb = blocks_of(g.nmesh / g.n[a], lines_per_block(g.n[a]));
+      for (int f = 0; f < nf; f++)
+        for (long long b = 0; b < nb; b++) w.push_back(make_int2(f, int(b)));
+      *count[a] = int(nb) * nf;
+    }
+    const std::vector<double> kc(nf, HUGE_VAL);
+    plan->kc.reset(nf);
+    plan->w.reset(w.size());
+    TRVG_HIP(hipMemcpyAsync(plan->kc.get(), kc.data(), nf * sizeof(double),
+                            hipMemcpyHostToDevice, ctx.stream));
+    TRVG_HIP(hipMemcpyAsync(plan->w.get(), w.data(), w.size() * sizeof(int2),
+                            hipMemcpyHostToDevice, ctx.stream));
+    TRVG_HIP(hipStreamSynchronize(ctx.stream));
+    std::lock_guard<std::mutex> lk(mu);
+    if (cache.size() >= 16) cache.clear();   // bounded; plans in use stay alive
+    cache[key] = plan;
+  }
+  ctx.keep.push_back(plan);
+  const int2* wx = plan->w.get();
+  const int2* wy = wx + plan->nx;
+  const int2* wz = wy + plan->ny;
+  fft3d_batch<T>(ctx, base, LoadSameBatch<T>{base, g.nmesh}, -1, false, plan->kc.get(), wz,
+                 plan->nz, wy, plan->ny, wx, plan->nx);
 }
 
 template <typename T, int LOGN>

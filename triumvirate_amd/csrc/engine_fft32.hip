@@ -12,7 +12,6 @@ TRVG_FFT3D_INST(LoadDeconv<float TRVG_COMMA double>)
 // Loaders of the differentiable path (engine_diff.hip).
 TRVG_FFT3D_INST(LoadReal<float>)
 TRVG_FFT3D_INST(LoadDeconv<float TRVG_COMMA float>)
-TRVG_FFT3D_INST(LoadShellCotangent<float>)
 TRVG_FFT3D_INST(LoadShell<float TRVG_COMMA float>)
 #undef TRVG_FFT3D_INST
 
@@ -20,9 +19,13 @@ template void shell_slab_work<float>(const Geom&, const trvg_binning&, int, int,
                                    std::vector<ShellBand>&, std::vector<double>&,
                                    std::vector<int2>&, std::vector<int2>&,
                                    std::vector<int2>&);
-template void shell_slab_ifft<float>(Context&, c2<float>*, const double2*, const trvg_binning&,
-                                   const std::vector<int>&, const std::vector<int>&, int, int,
-                                   bool);
+template void shell_slab_ifft<float, double>(Context&, c2<float>*, const double2*,
+                                           const trvg_binning&, const std::vector<int>&,
+                                           const std::vector<int>&, int, int, bool);
+template void shell_slab_ifft<float, float>(Context&, float2*, const float2*,
+                                            const trvg_binning&, const std::vector<int>&,
+                                            const std::vector<int>&, int, int, bool);
+template void slab_fft<float>(Context&, c2<float>*, int);
 template void sjl_slab_ifft<float>(Context&, c2<float>*, const double2*, const Spline&,
                                  const std::vector<double>&, const std::vector<int>&, int, int,
                                  bool);

@@ -13,7 +13,6 @@ TRVG_FFT3D_INST(LoadTwopt<double TRVG_COMMA double>)
 TRVG_FFT3D_INST(LoadDeconv<double TRVG_COMMA double>)
 // Loaders of the differentiable path (engine_diff.hip).
 TRVG_FFT3D_INST(LoadReal<double>)
-TRVG_FFT3D_INST(LoadShellCotangent<double>)
 TRVG_FFT3D_INST(LoadShell<double TRVG_COMMA double>)
 #undef TRVG_FFT3D_INST
 
@@ -21,9 +20,10 @@ template void shell_slab_work<double>(const Geom&, const trvg_binning&, int, int
                                    std::vector<ShellBand>&, std::vector<double>&,
                                    std::vector<int2>&, std::vector<int2>&,
                                    std::vector<int2>&);
-template void shell_slab_ifft<double>(Context&, c2<double>*, const double2*, const trvg_binning&,
-                                   const std::vector<int>&, const std::vector<int>&, int, int,
-                                   bool);
+template void shell_slab_ifft<double, double>(Context&, c2<double>*, const double2*,
+                                           const trvg_binning&, const std::vector<int>&,
+                                           const std::vector<int>&, int, int, bool);
+template void slab_fft<double>(Context&, c2<double>*, int);
 template void sjl_slab_ifft<double>(Context&, c2<double>*, const double2*, const Spline&,
                                  const std::vector<double>&, const std::vector<int>&, int, int,
                                  bool);

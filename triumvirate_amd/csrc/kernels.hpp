@@ -280,6 +280,16 @@ struct LoadMaskedZBatch {
   }
 };
 
+// Identity loader over the fields of a slab.
+template <typename T>
+struct LoadSameBatch {
+  const c2<T>* base;
+  long long fstride;
+  __device__ LoadSame<T> field(int f) const {
+    return LoadSame<T>{base + (long long)f * fstride};
+  }
+};
+
 // LoadShell for field q of a batched slab transform (band of bin q).
 template <typename T, typename S = T>
 struct LoadShellBatch {
