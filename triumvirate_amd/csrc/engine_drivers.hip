@@ -481,24 +481,103 @@ static void launch_pair_lds(Context& ctx, unsigned grid, size_t smem, const c2<T
   TRVG_LAUNCH_CHECK();
 }
 
-// S_p = sum_x F_a(x) F_b(x) G(x) for pairs p = (a, b) of logical fields,
-// handed to `sink` at the next ctx.flush() (the launches are only queued).
-// A side / B side packed: real fields stored two per complex mesh (logical
-// field 2q + c is component c of mesh q); g_real: G is real.
-template <typename T>
-static void pair_reduce(Context& ctx, const c2<T>* FA, int na, bool a_packed,
-                        const c2<T>* FB, int nbf, bool b_packed, const c2<T>* G,
-                        bool g_real, const std::vector<int2>& pairs,
-                        std::function<void(std::vector<cplx>&&)> sink) {
-  if (a_packed && !b_packed) {
-    // The product is symmetric in (a, b): put the packed side second.
-    std::vector<int2> sw(pairs.size());
-    for (size_t d = 0; d < pairs.size(); d++) sw[d] = make_int2(pairs[d].y, pairs[d].x);
-    pair_reduce<T>(ctx, FB, nbf, false, FA, na, true, G, g_real, sw, std::move(sink));
-    return;
+// What a term uses of its pair sums S: it adds S + f conj(S), twice the
+// real part (f = 1) or the imaginary part (f = -1) of a term counted with its
+// mirror, or S itself (f = 0, the term of m1 = m2 = M = 0).
+enum PairPart { PAIR_FULL, PAIR_REAL, PAIR_IMAG };
+static PairPart wanted(double f_mirror) {
+  return f_mirror > 0. ? PAIR_REAL : (f_mirror < 0. ? PAIR_IMAG : PAIR_FULL);
+}
+
+template <int MODE, bool FULL, int NTA>
+static auto pair_mfma_kernel(int ntb) {
+  return ntb == 1 ? k_pair_mfma<MODE, FULL, NTA, 1> : k_pair_mfma<MODE, FULL, NTA, 2>;
+}
+
+template <int MODE, bool FULL>
+static void launch_pair_mfma(Context& ctx, unsigned grid, size_t smem, const float2* fa,
+                             int nas, const float2* fb, int nbs, const float2* G,
+                             long long nm, int nta, int ntb, unsigned mask, bool same,
+                             bool rot, double* part) {
+  auto kern = nta == 1 ? pair_mfma_kernel<MODE, FULL, 1>(ntb) : pair_mfma_kernel<MODE, FULL, 2>(ntb);
+  if (smem > 64 * 1024)
+    TRVG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(smem)));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), smem, ctx.stream, fa, nas, fb, nbs, G, nm,
+                     mask, int(same), int(rot), part);
+  TRVG_LAUNCH_CHECK();
+}
+
+// pair_reduce of FP32 fields with a complex A side on the matrix cores
+// (k_pair_mfma).
+static void pair_reduce_mfma(Context& ctx, const float2* FA, int na, const float2* FB, int nbf, bool b_packed, const float2* G,
+                             PairPart want, const std::vector<int2>& pairs,
+                             std::function<void(std::vector<cplx>&&)> sink) {
+  const int mode = b_packed ? 1 : 0;
+  const bool full = want == PAIR_FULL;
+  const long long nm = ctx.g.nmesh;
+  constexpr int SIDE = PM_TILE * PM_NT;   // fields a side of one launch
+  struct Group {
+    int a0, b0, nta, ntb;
+    const double* h;
+  };
+  std::vector<Group> groups;
+  const long long nchunks = nm / PairLds<float>::LDC;
+  for (int b0 = 0; b0 < nbf; b0 += SIDE) {
+    for (int a0 = 0; a0 < na; a0 += SIDE) {
+      const int nas = std::min(SIDE, na - a0), nbs = std::min(SIDE, nbf - b0);
+      const int nta = (nas + PM_TILE - 1) / PM_TILE, ntb = (nbs + PM_TILE - 1) / PM_TILE;
+      unsigned mask = 0u;
+      for (const int2& pr : pairs)
+        if (pr.x >= a0 && pr.x < a0 + nas && pr.y >= b0 && pr.y < b0 + nbs)
+          mask |= 1u << ((pr.x - a0) / PM_TILE * ntb + (pr.y - b0) / PM_TILE);
+      if (mask == 0u) continue;
+      const bool same = FA == FB && !b_packed && a0 == b0 && nas == nbs;
+      const int ma = pair_rows_a(mode, nas), mb = same ? 0 : pair_rows_b(mode, nbs);
+      const size_t smem = pair_mfma_smem(ma + mb + 1, nta * ntb, full);
+      const int per_cu = std::max(1, std::min(8, int((160 * 1024) / smem)));
+      const unsigned grid =
+          unsigned(std::max<long long>(1, std::min<long long>(nchunks, (long long)ctx.sm_count * per_cu)));
+      const int width = nta * ntb * PM_TILE * PM_TILE * (full ? 2 : 1);
+      DevArray<double> part((size_t)grid * width), sum(width);
+      {
+        // A packed side holds two fields per mesh (group starts are even).
+        const float2* fa = FA + (long long)a0 * nm;
+        const float2* fb = FB + (long long)(mode >= 1 ? b0 / 2 : b0) * nm;
+        ProfScope ps(ctx, KC_PAIR_REDUCE, (ma + mb + 1.) * double(nm) * sizeof(float2));
+        const bool rot = want == PAIR_IMAG;
+        auto go = mode == 1 ? (full ? launch_pair_mfma<1, true> : launch_pair_mfma<1, false>)
+                            : (full ? launch_pair_mfma<0, true> : launch_pair_mfma<0, false>);
+        go(ctx, grid, smem, fa, nas, fb, nbs, G, nm, nta, ntb, mask, same, rot, part.get());
+      }
+      reduce_cols(ctx, part.get(), int(grid), width, sum.get());
+      groups.push_back(Group{a0, b0, nta, ntb, ctx.download(sum.get(), width)});
+      ctx.keep_until_flush(std::move(part));
+      ctx.keep_until_flush(std::move(sum));
+    }
   }
-  if (a_packed && !g_real)
-    throw Error(TRVG_ERR_INTERNAL, "Real shell pairs need a real G field.");
+  ctx.defer([groups = std::move(groups), pairs, full, want, sink = std::move(sink)]() {
+    std::vector<cplx> out(pairs.size());
+    for (const Group& gr : groups)
+      for (size_t d = 0; d < pairs.size(); d++) {
+        const int a = pairs[d].x - gr.a0, b = pairs[d].y - gr.b0;
+        if (a < 0 || b < 0 || a >= gr.nta * PM_TILE || b >= gr.ntb * PM_TILE) continue;
+        const int tile = a / PM_TILE * gr.ntb + b / PM_TILE;
+        const double* h = gr.h + tile * 256 + a % PM_TILE * 16 + b % PM_TILE;
+        out[d] = full ? cplx(h[0], h[gr.nta * gr.ntb * 256])
+                      : (want == PAIR_IMAG ? cplx(0., h[0]) : cplx(h[0], 0.));
+      }
+    sink(std::move(out));
+  });
+}
+
+// pair_reduce on the vector units (k_pair_lds): FP64 fields and two real
+// sides.
+template <typename T>
+static void pair_reduce_lds(Context& ctx, const c2<T>* FA, int na, bool a_packed,
+                            const c2<T>* FB, int nbf, bool b_packed, const c2<T>* G,
+                            const std::vector<int2>& pairs,
+                            std::function<void(std::vector<cplx>&&)> sink) {
   const int mode = (a_packed && b_packed) ? 2 : (b_packed ? 1 : 0);
   const long long nm = ctx.g.nmesh;
   const int rbn = (na + 3) / 4, cbn = (nbf + 3) / 4;
@@ -550,8 +629,8 @@ static void pair_reduce(Context& ctx, const c2<T>* FA, int na, bool a_packed,
         switch (kmode) {
           case 3: launch_pair_lds<T, 3>(ctx, grid, smem, fa, nas, fb, nbs, G, nm, dt.get(), nt, part.get()); break;
           case 2: launch_pair_lds<T, 2>(ctx, grid, smem, fa, nas, fb, nbs, G, nm, dt.get(), nt, part.get()); break;
-          case 1: launch_pair_lds<T, 1>(ctx, grid, smem, fa, nas, fb, nbs, G, nm, dt.get(), nt, part.get()); break;
-          default: launch_pair_lds<T, 0>(ctx, grid, smem, fa, nas, fb, nbs, G, nm, dt.get(), nt, part.get()); break;
+          case 1: if constexpr (sizeof(T) == 8) launch_pair_lds<T, 1>(ctx, grid, smem, fa, nas, fb, nbs, G, nm, dt.get(), nt, part.get()); break;
+          default: if constexpr (sizeof(T) == 8) launch_pair_lds<T, 0>(ctx, grid, smem, fa, nas, fb, nbs, G, nm, dt.get(), nt, part.get()); break;
         }
         TRVG_LAUNCH_CHECK();
       }
@@ -580,6 +659,34 @@ static void pair_reduce(Context& ctx, const c2<T>* FA, int na, bool a_packed,
       out[d] = full[(size_t)pairs[d].x * nbf + pairs[d].y];
     sink(std::move(out));
   });
+}
+
+// S_p = sum_x F_a(x) F_b(x) G(x) for pairs p = (a, b) of logical fields,
+// handed to `sink` at the next ctx.flush() (the launches are only queued).
+// A side / B side packed: real fields stored two per complex mesh (logical
+// field 2q + c is component c of mesh q); g_real: G is real.  `want`: what
+// the caller uses of S (the rest may come back as zero).
+template <typename T>
+static void pair_reduce(Context& ctx, const c2<T>* FA, int na, bool a_packed,
+                        const c2<T>* FB, int nbf, bool b_packed, const c2<T>* G,
+                        bool g_real, PairPart want, const std::vector<int2>& pairs,
+                        std::function<void(std::vector<cplx>&&)> sink) {
+  if (a_packed && !b_packed) {
+    // The product is symmetric in (a, b): put the packed side second.
+    std::vector<int2> sw(pairs.size());
+    for (size_t d = 0; d < pairs.size(); d++) sw[d] = make_int2(pairs[d].y, pairs[d].x);
+    pair_reduce<T>(ctx, FB, nbf, false, FA, na, true, G, g_real, want, sw, std::move(sink));
+    return;
+  }
+  if (a_packed && !g_real)
+    throw Error(TRVG_ERR_INTERNAL, "Real shell pairs need a real G field.");
+  if constexpr (sizeof(T) == 4) {
+    if (!a_packed) {
+      pair_reduce_mfma(ctx, FA, na, FB, nbf, b_packed, G, want, pairs, std::move(sink));
+      return;
+    }
+  }
+  pair_reduce_lds<T>(ctx, FA, na, a_packed, FB, nbf, b_packed, G, pairs, std::move(sink));
 }
 
 struct TwoPt {
@@ -1241,7 +1348,7 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
         // Results arrive at the flush after the last term (the sinks add
         // into `out`, which outlives them).
         pair_reduce<T>(ctx, A->data.get(), A->nfields, A->packed, B->data.get(),
-                       B->nfields, B->packed, G.get(), g_real, pairs,
+                       B->nfields, B->packed, G.get(), g_real, wanted(f_mirror), pairs,
                        [&out, &ra, &cb, &ss, dvs = gr.pairs, coupling, f_mirror,
                         vc = gc.vol_cell](std::vector<cplx>&& S) {
                          for (size_t d = 0; d < dvs.size(); d++) {
@@ -1438,7 +1545,7 @@ Result run_3pcf(Context& ctx, const DeviceCatalogue& d,
     // G_LM is real for M = 0 (real weights Y_L0) and in a periodic box.
     const bool g_real = !survey || tm.M == 0;
     pair_reduce<T>(ctx, A->data.get(), A->nfields, A->packed, B->data.get(), B->nfields,
-                   B->packed, G.get(), g_real, pairs,
+                   B->packed, G.get(), g_real, wanted(tm.f_mirror), pairs,
                    [&out, dim, c = tm.coupling * g.vol_cell * factor_phase,
                     fm = tm.f_mirror](std::vector<cplx>&& S) {
                      for (int dv = 0; dv < dim; dv++)

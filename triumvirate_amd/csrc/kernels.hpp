@@ -2089,3 +2089,236 @@ k_pair_lds(const c2<T>* __restrict__ FA, int na, const c2<T>* __restrict__ FB, i
 }
 
 }  // namespace trvg
+
+namespace trvg {
+
+// ---------------------------------------------------------------------------
+// FP32 pair product-reduction on the matrix cores:
+//   S[ia][ib] = sum_x FA[ia](x) FB[ib](x) G(x)
+// as a contraction over the cells with v_mfma_f32_16x16x4_f32 (FP32 products
+// and sums, as the vector kernel), 16 x 16 pairs per tile, NTA x NTB tiles.
+// Staging as k_pair_lds: chunks of LDC cells, one row per mesh and one for G,
+// direct to LDS and double buffered.  Each of the four waves takes a quarter
+// of a chunk's cells and every tile; lane (i = lane % 16, k = lane / 16)
+// reads field i of a tile at two cells per 16-byte access, which feed two
+// matrix instructions.  Sums of one chunk (32 cells) stay in FP32 and are
+// then added in FP64.
+//
+// MODE 0: complex sides; 1: B side real, two per mesh.  FULL: complex sums;
+// else real parts only (of the sums, or with `rot` of -i times them), half
+// the products.  `same`: both sides are the same fields, staged once.  Bit
+// a * NTB + b of `mask` is set for the tiles with pairs.
+//
+// What bounds it: HBM (4.5-5 TB/s), where the vector kernel spent several
+// times the issue slots of that on products and LDS reads.  Complex sides,
+// 30 + 30 fields of 512^3: 27.7 -> 14.4 ms (real parts); the same 30 fields
+// on both sides, complex sums: 27.7 -> 10.1 ms; 20 complex with 20 real
+// fields of 256^3: 1.01 -> 0.84 ms.  Two real sides stay on the vector
+// kernel: one product per pair and cell there fills the units as well (20
+// with 20 fields of 256^3: 0.57 ms against 0.54, one side 0.37 against 0.54).
+// ---------------------------------------------------------------------------
+
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+
+// Pairs per tile side and most tiles a side of one launch.
+constexpr int PM_TILE = 16;
+constexpr int PM_NT = 2;
+
+inline size_t pair_mfma_smem(int rows, int tiles, bool full) {
+  const size_t buf = 2 * size_t(rows) * PairLds<float>::ROWB;
+  const size_t red = size_t(tiles) * PM_TILE * PM_TILE * (full ? 2 : 1) * sizeof(double);
+  return buf > red ? buf : red;
+}
+
+template <int MODE, bool FULL, int NTA, int NTB>
+__global__ void __launch_bounds__(256)
+k_pair_mfma(const float2* __restrict__ FA, int na, const float2* __restrict__ FB, int nbf,
+            const float2* __restrict__ G, long long nmesh, unsigned mask, int same, int rot,
+            double* __restrict__ part) {
+  using L = PairLds<float>;
+  constexpr int NC = FULL ? 2 : 1;              // sums per pair
+  constexpr int SUMS = NTA * NTB * PM_TILE * PM_TILE;
+  extern __shared__ __attribute__((aligned(16))) char smp_raw[];
+  const int MA = pair_rows_a(MODE, na);
+  const int MB = same ? 0 : pair_rows_b(MODE, nbf);
+  const int R = MA + MB + 1;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int li = lane % 16, lk = lane / 16;
+  // Byte offsets of this lane's rows (clamped to existing fields; the host
+  // discards pairs past na / nbf) and component of a packed field.
+  int ra[NTA], rb[NTB];
+#pragma unroll
+  for (int t = 0; t < NTA; t++) {
+    const int f = min(t * PM_TILE + li, na - 1);
+    ra[t] = f * L::ROWB;
+  }
+#pragma unroll
+  for (int t = 0; t < NTB; t++) {
+    const int f = min(t * PM_TILE + li, nbf - 1);
+    rb[t] = ((MODE >= 1 ? f / 2 : f) + (same ? 0 : MA)) * L::ROWB;
+  }
+  // Odd fields of a packed pair sit in the imaginary part (a clamped field's
+  // parity may be wrong, which only discarded pairs see).
+  const bool odd = li & 1;
+
+  const long long nchunks = nmesh / L::LDC;
+  auto src = [&](int r) {
+    return r < MA ? FA + (long long)r * nmesh
+                  : (r < MA + MB ? FB + (long long)(r - MA) * nmesh : G);
+  };
+  auto issue = [&](long long ch, int b) {
+    char* base = smp_raw + (size_t)b * R * L::ROWB;
+    const long long off = ch * L::LDC + (long long)lane * L::PER_LANE;
+    for (int r = wave; r < R; r += 4)
+      __builtin_amdgcn_global_load_lds(
+          (const void*)(src(r) + off),
+          (__attribute__((address_space(3))) void*)(
+              (__attribute__((address_space(3))) char*)(base + (size_t)r * L::ROWB)),
+          16, 0, 0);
+  };
+
+  double sum[NC][NTA][NTB][4];
+#pragma unroll
+  for (int n = 0; n < NC; n++)
+#pragma unroll
+    for (int a = 0; a < NTA; a++)
+#pragma unroll
+      for (int b = 0; b < NTB; b++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) sum[n][a][b][r] = 0.;
+
+  // This wave's quarter of the chunk in `buf`.
+  auto reduce = [&](const char* buf) {
+    f32x4 acc[NC][NTA][NTB];
+#pragma unroll
+    for (int n = 0; n < NC; n++)
+#pragma unroll
+      for (int a = 0; a < NTA; a++)
+#pragma unroll
+        for (int b = 0; b < NTB; b++) acc[n][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const char* gbuf = buf + (size_t)(MA + MB) * L::ROWB;
+#pragma unroll
+    for (int c8 = 0; c8 < L::LDC / 4; c8 += 8) {
+      const int cell = wave * (L::LDC / 4) + c8 + 2 * lk;
+      // Two cells per access, as values (a selection between members of a
+      // struct would go through scratch).
+      auto cells = [cell](const char* row) {
+        const float4 w = *reinterpret_cast<const float4*>(row + cell * sizeof(float2));
+        return f32x4{w.x, w.y, w.z, w.w};
+      };
+      const f32x4 g = cells(gbuf);
+      float gx[2], gy[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        // -i g with rot: Re(-i z) = Im(z).
+        gx[u] = rot ? g[2 * u + 1] : g[2 * u];
+        gy[u] = rot ? -g[2 * u] : g[2 * u + 1];
+      }
+      // Left operands: F_a, or F_a G where only A is complex.
+      float ax[NTA][2], ay[NTA][2];
+#pragma unroll
+      for (int t = 0; t < NTA; t++) {
+        const f32x4 v = cells(buf + ra[t]);
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const float x = v[2 * u], y = v[2 * u + 1];
+          if (MODE == 1) {
+            ax[t][u] = x * gx[u] - y * gy[u];
+            if (FULL) ay[t][u] = x * gy[u] + y * gx[u];
+          } else {
+            ax[t][u] = x;
+            ay[t][u] = y;
+          }
+        }
+      }
+      // Right operands: F_b G, or F_b where A carries G.
+#pragma unroll
+      for (int b = 0; b < NTB; b++) {
+        const f32x4 v = cells(buf + rb[b]);
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const float x = v[2 * u], y = v[2 * u + 1];
+          float hx, hy = 0.f;
+          if (MODE == 1) {
+            hx = odd ? y : x;
+          } else {
+            hx = x * gx[u] - y * gy[u];
+            hy = x * gy[u] + y * gx[u];
+          }
+#pragma unroll
+          for (int a = 0; a < NTA; a++) {
+            if (!((mask >> (a * NTB + b)) & 1u)) continue;   // uniform
+            f32x4& re = acc[0][a][b];
+            re = __builtin_amdgcn_mfma_f32_16x16x4f32(ax[a][u], hx, re, 0, 0, 0);
+            if (MODE == 0)
+              re = __builtin_amdgcn_mfma_f32_16x16x4f32(ay[a][u], -hy, re, 0, 0, 0);
+            if constexpr (FULL) {
+              f32x4& im = acc[NC - 1][a][b];
+              im = __builtin_amdgcn_mfma_f32_16x16x4f32(ay[a][u], hx, im, 0, 0, 0);
+              if (MODE == 0)
+                im = __builtin_amdgcn_mfma_f32_16x16x4f32(ax[a][u], hy, im, 0, 0, 0);
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NC; n++)
+#pragma unroll
+      for (int a = 0; a < NTA; a++)
+#pragma unroll
+        for (int b = 0; b < NTB; b++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) sum[n][a][b][r] += double(acc[n][a][b][r]);
+  };
+
+  int cur = 0;
+  long long ch = blockIdx.x;
+  if (ch < nchunks) issue(ch, 0);
+  for (; ch < nchunks; ch += gridDim.x) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (ch + gridDim.x < nchunks) issue(ch + gridDim.x, cur ^ 1);
+    reduce(smp_raw + (size_t)cur * R * L::ROWB);
+    cur ^= 1;
+  }
+  __syncthreads();
+  // Cells past the last whole chunk: one more, filled up with zeros, by the
+  // block next in turn.
+  if (nchunks * L::LDC < nmesh && blockIdx.x == nchunks % gridDim.x) {
+    for (int r = wave; r < R; r += 4) {
+      const float2* s = src(r);
+      float2* d = reinterpret_cast<float2*>(smp_raw + (size_t)r * L::ROWB);
+      for (int c = lane; c < L::LDC; c += 64) {
+        const long long q = nchunks * L::LDC + c;
+        d[c] = q < nmesh ? s[q] : make_float2(0.f, 0.f);
+      }
+    }
+    __syncthreads();
+    reduce(smp_raw);
+    __syncthreads();
+  }
+  // Sums of the four waves, in their order; entry (i, j) of a tile is
+  // register i % 4 of lane 16 (i / 4) + j.
+  double* red = reinterpret_cast<double*>(smp_raw);
+  for (int w = 0; w < 4; w++) {
+    if (wave == w) {
+#pragma unroll
+      for (int n = 0; n < NC; n++)
+#pragma unroll
+        for (int a = 0; a < NTA; a++)
+#pragma unroll
+          for (int b = 0; b < NTB; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              double* p = red + n * SUMS + (a * NTB + b) * 256 + (4 * lk + r) * 16 + li;
+              *p = (w ? *p : 0.) + sum[n][a][b][r];
+            }
+    }
+    __syncthreads();
+  }
+  for (int q = threadIdx.x; q < NC * SUMS; q += 256)
+    part[(long long)blockIdx.x * NC * SUMS + q] = red[q];
+}
+
+}  // namespace trvg
