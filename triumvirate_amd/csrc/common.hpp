@@ -350,8 +350,10 @@ struct SplineDev {
     return i;
   }
 
+  // FAR = false: the caller knows x < split.
+  template <bool FAR = true>
   __device__ double eval(double x) const {
-    if (x >= split) return sph_bessel_dev(ell, x);
+    if (FAR && x >= split) return sph_bessel_dev(ell, x);
     const int i = interval(x);
     const double delx = x - __dmul_rn(step, double(i));
     const double4 q = cf[i];
@@ -361,8 +363,9 @@ struct SplineDev {
   // FP32 evaluation (FP32 fields): the interval from the FP64 argument, the
   // cubic in FP32.  At an interval edge the neighbouring cubic is used,
   // which the spline's continuity makes equivalent to FP32 rounding.
+  template <bool FAR = true>
   __device__ float eval32(double x) const {
-    if (x >= split) return float(sph_bessel_dev(ell, x));
+    if (FAR && x >= split) return float(sph_bessel_dev(ell, x));
     int i = int(x * inv_step);
     if (i > n - 2) i = n - 2;
     if (i < 0) i = 0;

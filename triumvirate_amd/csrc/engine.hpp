@@ -479,6 +479,9 @@ void slab_fft(Context& ctx, c2<T>* base, int nf);
 
 // Batched transforms over work lists (engine_fft.hpp).
 template <typename T>
+void full_work(const Geom& g, int nf, std::vector<int2>& wz, std::vector<int2>& wy,
+               std::vector<int2>& wx);
+template <typename T>
 void shell_slab_work(const Geom& g, const trvg_binning& kb, int nbins,
                      int nfield_groups, bool packed, std::vector<ShellBand>& bands,
                      std::vector<double>& kcut2, std::vector<int2>& wz,

@@ -148,7 +148,8 @@ class BatchPlan : public BatchPlanBase {
 
     // Work lists: unpruned passes over B fields, and the shell slabs
     // (complex and packed real).
-    full_lists(B_, wfull_);
+    full_lists<double>(B_, wfull_);
+    full_lists<T>(B_, wfullT_);
     for (int pk = 0; pk < 2; pk++) {
       SlabWork& sw = swork_[pk];
       std::vector<ShellBand> bands;
@@ -352,23 +353,19 @@ class BatchPlan : public BatchPlanBase {
                               hipMemcpyHostToDevice, ctx_.stream));
   }
 
+  // Every block of each catalogue's mesh, per pass (z, y, x).
+  struct FullWork {
+    DevArray<int2> w[3];
+    int n[3];
+  };
   template <typename U>
-  void full_lists(int nfields, std::vector<int2>& w) {
-    constexpr int E = FFT_THREADS * FftEpt<U>::v;
-    const long long nblk = nm_ / E;
-    w.clear();
-    for (int f = 0; f < nfields; f++)
-      for (long long k = 0; k < nblk; k++) w.push_back(make_int2(f, int(k)));
-  }
-  void full_lists(int nfields, DevArray<int2>& d64) {
-    std::vector<int2> w;
-    full_lists<double>(nfields, w);
-    upload(d64, w);
-    nfull64_ = int(w.size());
-    std::vector<int2> w32;
-    full_lists<T>(nfields, w32);
-    upload(wfullT_, w32);
-    nfullT_ = int(w32.size());
+  void full_lists(int nfields, FullWork& f) {
+    std::vector<int2> w[3];
+    full_work<U>(ctx_.g, nfields, w[0], w[1], w[2]);
+    for (int q = 0; q < 3; q++) {
+      upload(f.w[q], w[q]);
+      f.n[q] = int(w[q].size());
+    }
   }
 
   int slab_index(int l, int m) {
@@ -459,8 +456,8 @@ class BatchPlan : public BatchPlanBase {
     launch_assign();
     LoadScaleShiftMocks ls{D_.get(), nm_, d_nmock_.get(), g.vol, g.vol_cell};
     fft3d_batch<double>(ctx_, D_.get(), ls, -1, false, swork_[0].kcut2.get(),
-                        wfull_.get(), nfull64_, wfull_.get(), nfull64_,
-                        wfull_.get(), nfull64_);
+                        wfull_.w[0].get(), wfull_.n[0], wfull_.w[1].get(), wfull_.n[1],
+                        wfull_.w[2].get(), wfull_.n[2]);
     // Shell slabs (all bins of every mock per pass).
     for (size_t i = 0; i < slabs_.size(); i++) {
       const SlabWork& sw = swork_[slab_packed_[i] ? 1 : 0];
@@ -479,14 +476,15 @@ class BatchPlan : public BatchPlanBase {
     }
     // G(x) = IFFT[dn00 / (W V)] (every periodic-box term uses dn00).
     LoadDeconvMocks<T> ld{D_.get(), nm_, ctx_.tab, 1. / g.vol};
-    fft3d_batch<T>(ctx_, G_.get(), ld, +1, false, swork_[0].kcut2.get(), wfullT_.get(),
-                   nfullT_, wfullT_.get(), nfullT_, wfullT_.get(), nfullT_);
+    fft3d_batch<T>(ctx_, G_.get(), ld, +1, false, swork_[0].kcut2.get(),
+                   wfullT_.w[0].get(), wfullT_.n[0], wfullT_.w[1].get(), wfullT_.n[1],
+                   wfullT_.w[2].get(), wfullT_.n[2]);
     // Shot-noise field t(x) = IFFT[(dn00 N00^* - N) / C1] / V: the same for
     // every term and multipole of a periodic box (threept.cpp:950-964).
     LoadTwoptMocks lt{D_.get(), D_.get(), nm_, ctx_.tab, d_nmock_.get(), 1. / g.vol};
     fft3d_batch<double>(ctx_, tfield_.get(), lt, +1, false, swork_[0].kcut2.get(),
-                        wfull_.get(), nfull64_, wfull_.get(), nfull64_,
-                        wfull_.get(), nfull64_);
+                        wfull_.w[0].get(), wfull_.n[0], wfull_.w[1].get(), wfull_.n[1],
+                        wfull_.w[2].get(), wfull_.n[2]);
     for (auto& P : mps_) run_multipole(*P);
   }
 
@@ -766,8 +764,7 @@ class BatchPlan : public BatchPlanBase {
     DevArray<int2> work;   // z, then y, then x blocks
     int nz = 0, ny = 0, nx = 0;
   } swork_[2];
-  DevArray<int2> wfull_, wfullT_;
-  int nfull64_ = 0, nfullT_ = 0;
+  FullWork wfull_, wfullT_;
   std::vector<std::pair<int, int>> slabs_;
   std::vector<bool> slab_packed_;
   std::vector<DevArray<c2<T>>> slab_data_;

@@ -7,7 +7,6 @@
 #include <algorithm>
 #include <map>
 #include <tuple>
-#include <type_traits>
 
 #include "batch_kernels.hpp"
 #include "diff_kernels.hpp"
@@ -55,52 +54,25 @@ static const c2<T>* twiddles(int n, int sign) {
 }
 
 
-template <typename T, int LOGN>
-static size_t fft_smem(bool row_flags) {
-  constexpr int N = 1 << LOGN;
-  constexpr int NL = FFT_THREADS * FftEpt<T>::v / N;
-  // Lines, twiddles, then (strided passes) one byte per row of pruning flags.
-  return size_t(NL * (N + 1) + N) * sizeof(c2<T>) + (row_flags ? N : 0);
-}
-
-// The register-resident z pass for FP32 meshes of 256 and 512 with loaders
-// that only read (the masked rows of shell transforms, plain transforms):
-// measured faster there.  FP64 passes and loaders with per-cell arithmetic
-// keep the LDS-staged pass, whose lower register use keeps more waves
-// resident.
-template <class Loader> struct ZRegLoader : std::false_type {};
-template <> struct ZRegLoader<LoadMaskedZBatch<float>> : std::true_type {};
-template <> struct ZRegLoader<LoadSame<float>> : std::true_type {};
-template <> struct ZRegLoader<LoadSameBatch<float>> : std::true_type {};
-
-template <typename T, int LOGN, class Loader>
-constexpr bool use_zreg() {
-  return ZRegShape<LOGN>::ok && sizeof(T) == 4 && ZRegLoader<Loader>::value;
+// Dynamic LDS above the default 64 KiB needs the kernel's attribute raised.
+template <class K>
+static void raise_lds(K kernel, size_t bytes) {
+  if (bytes > 64 * 1024)
+    TRVG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
 }
 
 template <typename T, int LOGN, class Loader>
 static void launch_z(Context& ctx, c2<T>* data, const Loader& load, int sign,
                      double read_bytes, double write_bytes, const Prune& pr) {
-  constexpr int EPT = FftEpt<T>::v;
   constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const long long nblocks = ctx.g.nmesh / E;
-  const size_t smem = fft_smem<T, LOGN>(false);
+  const long long nlines = ctx.g.nmesh / N;
   const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, read_bytes + write_bytes);
-  if constexpr (use_zreg<T, LOGN, Loader>()) {
-    static_assert(E == zreg_block<T>(), "z pass block size");
-    hipLaunchKernelGGL((fft_pass_z_reg<T, LOGN, Loader>), dim3(unsigned(nblocks)),
-                       dim3(zreg_threads<T, LOGN>()), (zreg_smem<T, LOGN>()), ctx.stream, data,
-                       load, tw, ctx.g.n[1], sign, pr);
-  } else if (ctx.g.n[1] % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_z<T, LOGN, EPT, true, Loader>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, load, tw,
-                       ctx.g.n[1], sign, pr);
-  else
-    hipLaunchKernelGGL((fft_pass_z<T, LOGN, EPT, false, Loader>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, load, tw,
-                       ctx.g.n[1], sign, pr);
+  hipLaunchKernelGGL((fft_pass_z<T, LOGN, Loader>),
+                     dim3(unsigned((nlines + z_lines(N) - 1) / z_lines(N))), dim3(FFT_THREADS),
+                     (z_smem<T, LOGN>()), ctx.stream, data, load, tw, ctx.g.n[1], nlines, sign,
+                     pr);
   TRVG_LAUNCH_CHECK();
 }
 
@@ -108,21 +80,15 @@ template <typename T, int LOGN>
 static void launch_strided(Context& ctx, c2<T>* data, long long S,
                            long long outer_stride, long long inner, int sign,
                            const Prune& pr, int prune_mode, double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const long long nblocks = ctx.g.nmesh / E;
-  const size_t smem = fft_smem<T, LOGN>(true);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
+  constexpr int NL = strided_lines<T, LOGN>();
+  const long long nlines = ctx.g.nmesh >> LOGN;
+  const c2<T>* tw = ctx_twiddles<T>(ctx, 1 << LOGN, sign);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (inner % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_strided<T, LOGN, EPT, true>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, tw, S, outer_stride,
-                       inner, sign, pr, prune_mode);
-  else
-    hipLaunchKernelGGL((fft_pass_strided<T, LOGN, EPT, false>), dim3(unsigned(nblocks)),
-                       dim3(FFT_THREADS), smem, ctx.stream, data, tw, S, outer_stride,
-                       inner, sign, pr, prune_mode);
+  auto kern = fft_pass_strided<T, LOGN>;
+  raise_lds(kern, strided_smem<T, LOGN>());
+  hipLaunchKernelGGL(kern, dim3(unsigned((nlines + NL - 1) / NL)),
+                     dim3(strided_threads<T, LOGN>()), (strided_smem<T, LOGN>()), ctx.stream,
+                     data, tw, S, outer_stride, inner, nlines, sign, pr, prune_mode);
   TRVG_LAUNCH_CHECK();
 }
 
@@ -146,23 +112,18 @@ static int ilog2(int n) {
   }
 
 // Axes of power-of-two length up to 1024 take the compile-time passes of
-// fft.hpp; other (even) lengths the mixed-radix passes of fft_gen.hpp.  Both
-// give a workgroup lines_per_block(n) lines (2048 / n for the former).
-static bool pow2_axis(int n) { return n >= 8 && n <= 1024 && (n & (n - 1)) == 0; }
-// The compile-time passes take whole blocks of 2048 elements: a power-of-two
-// axis of a mesh whose cell count is not a multiple of 2048 (other axes not
-// powers of two) goes through the mixed-radix passes too.
-static bool fast_axis(const Geom& g, int n) { return pow2_axis(n) && g.nmesh % 2048 == 0; }
-static int lines_per_block(int n) { return gen_lines_per_block(n); }
-static long long blocks_of(long long nlines, int nl) { return (nlines + nl - 1) / nl; }
-
-// Dynamic LDS above the default 64 KiB needs the kernel's attribute raised.
-template <class K>
-static void gen_lds(K kernel, size_t bytes) {
-  if (bytes > 64 * 1024)
-    TRVG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+// fft.hpp; other (even) lengths the mixed-radix passes of fft_gen.hpp.
+static bool fast_axis(int n) { return n >= 8 && n <= 1024 && (n & (n - 1)) == 0; }
+// Lines per workgroup of the z pass and of the strided passes (work lists).
+static int lines_z(int n) { return fast_axis(n) ? z_lines(n) : gen_lines_per_block(n); }
+template <typename T>
+static int lines_strided(int n) {
+  if (fast_axis(n)) {
+    TRVG_LOGN_SWITCH(ilog2(n), return (strided_lines<T, LG>()));
+  }
+  return gen_lines_per_block(n);
 }
+static long long blocks_of(long long nlines, int nl) { return (nlines + nl - 1) / nl; }
 
 template <typename T, class Loader>
 static void launch_z_gen(Context& ctx, c2<T>* data, const Loader& load, int sign,
@@ -172,7 +133,7 @@ static void launch_z_gen(Context& ctx, c2<T>* data, const Loader& load, int sign
   const long long nlines = (long long)ctx.g.n[0] * ctx.g.n[1];
   const size_t smem = gen_smem<T>(N, false);
   auto kern = fft_pass_z_gen<T, Loader>;
-  gen_lds(kern, smem);
+  raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(blocks_of(nlines, P.nl))), dim3(FFT_THREADS), smem,
                      ctx.stream, data, load, ctx_twiddles<T>(ctx, N, sign), ctx.g.n[1],
@@ -188,7 +149,7 @@ static void launch_strided_gen(Context& ctx, c2<T>* data, int N, long long S,
   const long long nlines = ctx.g.nmesh / N;
   const size_t smem = gen_smem<T>(N, true);
   auto kern = fft_pass_strided_gen<T>;
-  gen_lds(kern, smem);
+  raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(blocks_of(nlines, P.nl))), dim3(FFT_THREADS), smem,
                      ctx.stream, data, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
@@ -205,7 +166,7 @@ static void launch_z_batch_gen(Context& ctx, c2<T>* base, const BatchLoader& loa
   const long long nlines = (long long)ctx.g.n[0] * ctx.g.n[1];
   const size_t smem = gen_smem<T>(N, false);
   auto kern = fft_pass_z_batch_gen<T, BatchLoader>;
-  gen_lds(kern, smem);
+  raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
                      ctx.g.nmesh, load, ctx_twiddles<T>(ctx, N, sign), ctx.g.n[1], nlines,
@@ -222,7 +183,7 @@ static void launch_strided_batch_gen(Context& ctx, c2<T>* base, int N, long long
   const long long nlines = ctx.g.nmesh / N;
   const size_t smem = gen_smem<T>(N, true);
   auto kern = fft_pass_strided_batch_gen<T>;
-  gen_lds(kern, smem);
+  raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
                      ctx.g.nmesh, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
@@ -286,32 +247,12 @@ template <typename T, int LOGN, class BatchLoader>
 static void launch_z_batch(Context& ctx, c2<T>* base, const BatchLoader& load,
                            int sign, const Prune& pr, const double* kcut2,
                            const int2* work, int nwork, double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
   constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const size_t smem = fft_smem<T, LOGN>(false);
   const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
-  bool reg = false;
-  if constexpr (use_zreg<T, LOGN, BatchLoader>()) {
-    static_assert(E == zreg_block<T>(), "z pass block size");
-    reg = !pr.on;   // the register pass takes every listed block
-    if (reg)
-      hipLaunchKernelGGL((fft_pass_z_batch_reg<T, LOGN, BatchLoader>),
-                         dim3(unsigned((nwork + 1) / 2)), dim3(zreg_threads<T, LOGN>()),
-                         (zreg_smem<T, LOGN>()), ctx.stream, base, ctx.g.nmesh, load, tw,
-                         ctx.g.n[1], sign, work, nwork);
-  }
-  if (!reg) {
-    if (ctx.g.n[1] % (E / N) == 0)
-      hipLaunchKernelGGL((fft_pass_z_batch<T, LOGN, EPT, true, BatchLoader>),
-                         dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream,
-                         base, ctx.g.nmesh, load, tw, ctx.g.n[1], sign, pr, kcut2, work);
-    else
-      hipLaunchKernelGGL((fft_pass_z_batch<T, LOGN, EPT, false, BatchLoader>),
-                         dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream,
-                         base, ctx.g.nmesh, load, tw, ctx.g.n[1], sign, pr, kcut2, work);
-  }
+  hipLaunchKernelGGL((fft_pass_z_batch<T, LOGN, BatchLoader>), dim3(unsigned(nwork)),
+                     dim3(FFT_THREADS), (z_smem<T, LOGN>()), ctx.stream, base, ctx.g.nmesh,
+                     load, tw, ctx.g.n[1], ctx.g.nmesh / N, sign, pr, kcut2, work);
   TRVG_LAUNCH_CHECK();
 }
 
@@ -321,20 +262,14 @@ static void launch_strided_batch(Context& ctx, c2<T>* base, long long S,
                                  int sign, const Prune& pr, const double* kcut2,
                                  const int2* work, int nwork, int prune_mode,
                                  double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const size_t smem = fft_smem<T, LOGN>(true);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, sign);
+  const c2<T>* tw = ctx_twiddles<T>(ctx, 1 << LOGN, sign);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (inner % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_strided_batch<T, LOGN, EPT, true>), dim3(unsigned(nwork)),
-                       dim3(FFT_THREADS), smem, ctx.stream, base, ctx.g.nmesh, tw, S,
-                       outer_stride, inner, sign, pr, kcut2, work, prune_mode);
-  else
-    hipLaunchKernelGGL((fft_pass_strided_batch<T, LOGN, EPT, false>), dim3(unsigned(nwork)),
-                       dim3(FFT_THREADS), smem, ctx.stream, base, ctx.g.nmesh, tw, S,
-                       outer_stride, inner, sign, pr, kcut2, work, prune_mode);
+  auto kern = fft_pass_strided_batch<T, LOGN>;
+  raise_lds(kern, strided_smem<T, LOGN>());
+  hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(strided_threads<T, LOGN>()),
+                     (strided_smem<T, LOGN>()), ctx.stream, base, ctx.g.nmesh, tw, S,
+                     outer_stride, inner, ctx.g.nmesh >> LOGN, sign, pr, kcut2, work,
+                     prune_mode);
   TRVG_LAUNCH_CHECK();
 }
 
@@ -353,36 +288,55 @@ void fft3d_batch(Context& ctx, c2<T>* base, const BatchLoader& load, int sign,
   pr.dk1 = g.dk[1];
   pr.n0 = g.n[0];
   pr.n1 = g.n[1];
-  const double blk = double(FFT_THREADS * FftEpt<T>::v) * sizeof(c2<T>);
+  // Bytes of a listed block of an axis of n points with nl lines each.
+  auto blk = [](int n, int nl) { return double(nl) * n * sizeof(c2<T>); };
+  const double bz = 2. * nz * blk(g.n[2], lines_z(g.n[2]));
+  const double by = 2. * ny * blk(g.n[1], lines_strided<T>(g.n[1]));
+  const double bx = 2. * nx * blk(g.n[0], lines_strided<T>(g.n[0]));
   if (nz > 0) {
-    if (fast_axis(g, g.n[2])) {
+    if (fast_axis(g.n[2])) {
       TRVG_LOGN_SWITCH(ilog2(g.n[2]), (launch_z_batch<T, LG>(
-          ctx, base, load, sign, pr, kcut2, wz, nz, 2. * blk * nz)));
+          ctx, base, load, sign, pr, kcut2, wz, nz, bz)));
     } else {
-      launch_z_batch_gen<T>(ctx, base, load, sign, pr, kcut2, wz, nz, 2. * blk * nz);
+      launch_z_batch_gen<T>(ctx, base, load, sign, pr, kcut2, wz, nz, bz);
     }
   }
   if (ny > 0) {
-    if (fast_axis(g, g.n[1])) {
+    if (fast_axis(g.n[1])) {
       TRVG_LOGN_SWITCH(ilog2(g.n[1]), (launch_strided_batch<T, LG>(
           ctx, base, g.n[2], (long long)g.n[1] * g.n[2], g.n[2], sign, pr, kcut2, wy,
-          ny, 1, 2. * blk * ny)));
+          ny, 1, by)));
     } else {
       launch_strided_batch_gen<T>(ctx, base, g.n[1], g.n[2], (long long)g.n[1] * g.n[2],
-                                  g.n[2], sign, pr, kcut2, wy, ny, 1, 2. * blk * ny);
+                                  g.n[2], sign, pr, kcut2, wy, ny, 1, by);
     }
   }
   if (nx > 0) {
-    if (fast_axis(g, g.n[0])) {
+    if (fast_axis(g.n[0])) {
       TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_strided_batch<T, LG>(
           ctx, base, (long long)g.n[1] * g.n[2], 0, (long long)g.n[1] * g.n[2], sign,
-          pr, kcut2, wx, nx, 2, 2. * blk * nx)));
+          pr, kcut2, wx, nx, 2, bx)));
     } else {
       launch_strided_batch_gen<T>(ctx, base, g.n[0], (long long)g.n[1] * g.n[2], 0,
                                   (long long)g.n[1] * g.n[2], sign, pr, kcut2, wx, nx, 2,
-                                  2. * blk * nx);
+                                  bx);
     }
   }
+}
+
+// Every block of nf meshes, per pass.
+template <typename T>
+void full_work(const Geom& g, int nf, std::vector<int2>& wz, std::vector<int2>& wy,
+               std::vector<int2>& wx) {
+  auto fill = [&](int axis, int nl, std::vector<int2>& w) {
+    w.clear();
+    const long long nb = blocks_of(g.nmesh / g.n[axis], nl);
+    for (int f = 0; f < nf; f++)
+      for (long long b = 0; b < nb; b++) w.push_back(make_int2(f, int(b)));
+  };
+  fill(2, lines_z(g.n[2]), wz);
+  fill(1, lines_strided<T>(g.n[1]), wy);
+  fill(0, lines_strided<T>(g.n[0]), wx);
 }
 
 // Work lists of a shell slab transform over `ngroups` groups of all
@@ -396,8 +350,8 @@ void shell_slab_work(const Geom& g, const trvg_binning& kb, int nbins,
                      int ngroups, bool packed, std::vector<ShellBand>& bands,
                      std::vector<double>& kcut2, std::vector<int2>& wz,
                      std::vector<int2>& wy, std::vector<int2>& wx) {
-  const int nl_z = lines_per_block(g.n[2]), nl_y = lines_per_block(g.n[1]);
-  const long long nblk = blocks_of((long long)g.n[1] * g.n[2], lines_per_block(g.n[0]));
+  const int nl_z = lines_z(g.n[2]), nl_y = lines_strided<T>(g.n[1]);
+  const long long nblk = blocks_of((long long)g.n[1] * g.n[2], lines_strided<T>(g.n[0]));
   const int per = packed ? 2 : 1;
   const int nt = (nbins + per - 1) / per;
   bands.assign((size_t)nt * per, ShellBand{HUGE_VAL, HUGE_VAL});
@@ -488,20 +442,13 @@ template <typename T, int LOGN, class BatchLoader>
 static void launch_x_load_batch(Context& ctx, c2<T>* base, const BatchLoader& load,
                                 const Prune& pr, const double* kcut2, const int2* work,
                                 int nwork, double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  const size_t smem = fft_smem<T, LOGN>(false);
-  const c2<T>* tw = ctx_twiddles<T>(ctx, N, +1);
+  const c2<T>* tw = ctx_twiddles<T>(ctx, 1 << LOGN, +1);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (ctx.g.n[2] % (E / N) == 0)
-    hipLaunchKernelGGL((fft_pass_x_load_batch<T, LOGN, EPT, true, BatchLoader>),
-                       dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                       ctx.g.nmesh, load, tw, ctx.g.n[1], ctx.g.n[2], +1, pr, kcut2, work);
-  else
-    hipLaunchKernelGGL((fft_pass_x_load_batch<T, LOGN, EPT, false, BatchLoader>),
-                       dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                       ctx.g.nmesh, load, tw, ctx.g.n[1], ctx.g.n[2], +1, pr, kcut2, work);
+  auto kern = fft_pass_x_load_batch<T, LOGN, BatchLoader>;
+  raise_lds(kern, strided_smem<T, LOGN>());
+  hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(strided_threads<T, LOGN>()),
+                     (strided_smem<T, LOGN>()), ctx.stream, base, ctx.g.nmesh, load, tw,
+                     ctx.g.n[1], ctx.g.n[2], +1, pr, kcut2, work);
   TRVG_LAUNCH_CHECK();
 }
 
@@ -513,7 +460,7 @@ static void launch_x_load_batch_gen(Context& ctx, c2<T>* base, const BatchLoader
   const GenPlan P = make_gen_plan(N);
   const size_t smem = gen_smem<T>(N, false);
   auto kern = fft_pass_x_load_batch_gen<T, BatchLoader>;
-  gen_lds(kern, smem);
+  raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
                      ctx.g.nmesh, load, ctx_twiddles<T>(ctx, N, +1), ctx.g.n[1], ctx.g.n[2],
@@ -534,7 +481,7 @@ static void xfirst_passes(Context& ctx, c2<T>* base, const BatchLoader& load,
                           int ny, const int2* wz, int nz, double bx, double by, double bz) {
   const Geom& g = ctx.g;
   if (nx > 0) {
-    if (fast_axis(g, g.n[0])) {
+    if (fast_axis(g.n[0])) {
       TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_x_load_batch<T, LG>(
           ctx, base, load, prune_zy(g), kcut2, wx, nx, bx)));
     } else {
@@ -551,7 +498,7 @@ static void xfirst_yz(Context& ctx, c2<T>* base, const double* kcut2, const int2
   const Geom& g = ctx.g;
   const Prune pr = prune_zy(g);
   if (ny > 0) {
-    if (fast_axis(g, g.n[1])) {
+    if (fast_axis(g.n[1])) {
       TRVG_LOGN_SWITCH(ilog2(g.n[1]), (launch_strided_batch<T, LG>(
           ctx, base, g.n[2], (long long)g.n[1] * g.n[2], g.n[2], +1, pr, kcut2, wy, ny, 3,
           by)));
@@ -565,7 +512,7 @@ static void xfirst_yz(Context& ctx, c2<T>* base, const double* kcut2, const int2
   off.on = 0;
   LoadMaskedZBatch<T> lz{base, g.nmesh, kcut2, g.dk[2], g.n[2]};
   if (nz > 0) {
-    if (fast_axis(g, g.n[2])) {
+    if (fast_axis(g.n[2])) {
       TRVG_LOGN_SWITCH(ilog2(g.n[2]), (launch_z_batch<T, LG>(
           ctx, base, lz, +1, off, kcut2, wz, nz, bz)));
     } else {
@@ -613,12 +560,12 @@ static std::shared_ptr<const ShellPlan> shell_plan(Context& ctx, const trvg_binn
   }
   const int nt = packed ? (nf + 1) / 2 : nf;
   const int per = packed ? 2 : 1;
-  const int nl_x = lines_per_block(g.n[0]), nl_y = lines_per_block(g.n[1]);
+  const int nl_x = lines_strided<T>(g.n[0]), nl_y = lines_strided<T>(g.n[1]);
   const ShellBand none{HUGE_VAL, HUGE_VAL};
   std::vector<ShellBand> bands((size_t)nt * per, none);
   std::vector<double> kc(nt, 0.);
   // z blocks: every (i, j) line of the last pass.
-  const long long nblk = blocks_of((long long)g.n[0] * g.n[1], lines_per_block(g.n[2]));
+  const long long nblk = blocks_of((long long)g.n[0] * g.n[1], lines_z(g.n[2]));
   std::vector<int2> wx, wy, wz;
   const double cb = sizeof(c2<T>);
   auto pl = std::make_shared<ShellPlan>();
@@ -700,15 +647,14 @@ void slab_fft(Context& ctx, c2<T>* base, int nf) {
     if (it != cache.end()) plan = it->second;
   }
   if (!plan) {
-    std::vector<int2> w;
+    std::vector<int2> w, wy, wz;
+    full_work<T>(g, nf, wz, wy, w);
     plan = std::make_shared<ShellPlan>();
-    int* count[3] = {&plan->nx, &plan->ny, &plan->nz};
-    for (int a = 0; a < 3; a++) {
-      const long long nb = blocks_of(g.nmesh / g.n[a], lines_per_block(g.n[a]));
-      for (int f = 0; f < nf; f++)
-        for (long long b = 0; b < nb; b++) w.push_back(make_int2(f, int(b)));
-      *count[a] = int(nb) * nf;
-    }
+    plan->nx = int(w.size());
+    plan->ny = int(wy.size());
+    plan->nz = int(wz.size());
+    w.insert(w.end(), wy.begin(), wy.end());
+    w.insert(w.end(), wz.begin(), wz.end());
     const std::vector<double> kc(nf, HUGE_VAL);
     plan->kc.reset(nf);
     plan->w.reset(w.size());
@@ -732,22 +678,19 @@ void slab_fft(Context& ctx, c2<T>* base, int nf) {
 template <typename T, int LOGN>
 static void launch_x_sjl(Context& ctx, c2<T>* base, int nt, const double2* src,
                          const Spline& sp, const double* r, int ell, int m, bool packed,
-                         double bytes) {
-  constexpr int EPT = FftEpt<T>::v;
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
+                         bool far, double bytes) {
   const Geom& g = ctx.g;
-  const size_t smem = fft_smem<T, LOGN>(false);
-  const unsigned grid = unsigned((long long)g.n[1] * g.n[2] / (E / N));
+  const unsigned grid =
+      unsigned(blocks_of((long long)g.n[1] * g.n[2], strided_lines<T, LOGN>()));
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
-  if (packed)
-    hipLaunchKernelGGL((fft_x_sjl_multi<T, LOGN, EPT, true>), dim3(grid), dim3(FFT_THREADS),
-                       smem, ctx.stream, base, g.nmesh, nt, src, ctx.tab, g, sp.dev(), r, ell,
-                       m, ctx_twiddles<T>(ctx, N, +1));
-  else
-    hipLaunchKernelGGL((fft_x_sjl_multi<T, LOGN, EPT, false>), dim3(grid), dim3(FFT_THREADS),
-                       smem, ctx.stream, base, g.nmesh, nt, src, ctx.tab, g, sp.dev(), r, ell,
-                       m, ctx_twiddles<T>(ctx, N, +1));
+  auto kern = packed ? (far ? fft_x_sjl_multi<T, LOGN, true, true>
+                            : fft_x_sjl_multi<T, LOGN, true, false>)
+                     : (far ? fft_x_sjl_multi<T, LOGN, false, true>
+                            : fft_x_sjl_multi<T, LOGN, false, false>);
+  raise_lds(kern, strided_smem<T, LOGN>());
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(strided_threads<T, LOGN>()),
+                     (strided_smem<T, LOGN>()), ctx.stream, base, g.nmesh, nt, src, ctx.tab, g,
+                     sp.dev(), r, ell, m, ctx_twiddles<T>(ctx, 1 << LOGN, +1));
   TRVG_LAUNCH_CHECK();
 }
 
@@ -763,13 +706,13 @@ static void launch_x_sjl_gen(Context& ctx, c2<T>* base, int nt, const double2* s
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   if (packed) {
     auto kern = fft_x_sjl_multi_gen<T, true>;
-    gen_lds(kern, smem);
+    raise_lds(kern, smem);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(FFT_THREADS), smem, ctx.stream, base, g.nmesh,
                        nt, src, ctx.tab, g, sp.dev(), r, ell, m,
                        ctx_twiddles<T>(ctx, N, +1), P);
   } else {
     auto kern = fft_x_sjl_multi_gen<T, false>;
-    gen_lds(kern, smem);
+    raise_lds(kern, smem);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(FFT_THREADS), smem, ctx.stream, base, g.nmesh,
                        nt, src, ctx.tab, g, sp.dev(), r, ell, m,
                        ctx_twiddles<T>(ctx, N, +1), P);
@@ -808,9 +751,9 @@ void sjl_slab_ifft(Context& ctx, c2<T>* base, const double2* src, const Spline& 
     if (it != cache.end()) plan = it->second;
   }
   if (!plan) {
-    const PruneListsXF& pl = prune_lists_xfirst(g, HUGE_VAL, lines_per_block(g.n[0]),
-                                                lines_per_block(g.n[1]));
-    const long long nblk = blocks_of((long long)g.n[0] * g.n[1], lines_per_block(g.n[2]));
+    const PruneListsXF& pl = prune_lists_xfirst(g, HUGE_VAL, lines_strided<T>(g.n[0]),
+                                                lines_strided<T>(g.n[1]));
+    const long long nblk = blocks_of((long long)g.n[0] * g.n[1], lines_z(g.n[2]));
     std::vector<double> kc(nt, HUGE_VAL);
     std::vector<int2> w;   // y blocks, then z blocks
     for (int f = 0; f < nt; f++)
@@ -839,9 +782,14 @@ void sjl_slab_ifft(Context& ctx, c2<T>* base, const double2* src, const Spline& 
   // later ones read) every field.
   const double fb = double(g.nmesh) * sizeof(c2<T>) * nt;
   const double bx = double(g.nmesh) * sizeof(double2) + fb, by = 2. * fb, bz = 2. * fb;
-  if (fast_axis(g, g.n[0])) {
+  // Whether some argument |k| r leaves the spline's range.
+  double k2 = 0., rmax = 0.;
+  for (int a = 0; a < 3; a++) k2 += std::pow(g.n[a] / 2 * g.dk[a], 2);
+  for (double v : rr) rmax = std::max(rmax, v);
+  const bool far = !(std::sqrt(k2) * rmax * (1. + 1.e-9) < sp.split);
+  if (fast_axis(g.n[0])) {
     TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_x_sjl<T, LG>(ctx, base, nt, src, sp, dr.get(),
-                                                          ell, m, packed, bx)));
+                                                          ell, m, packed, far, bx)));
   } else {
     launch_x_sjl_gen<T>(ctx, base, nt, src, sp, dr.get(), ell, m, packed, bx);
   }
@@ -877,13 +825,13 @@ void fft3d(Context& ctx, c2<T>* data, const Loader& load, int sign,
   if (read_bytes < 0.) read_bytes = double(g.nmesh) * cb;
   const double zw = d_lines * g.n[2] * cb;
   const double slab_vals = slabs * g.n[1] * g.n[2];
-  if (fast_axis(g, g.n[2])) {
+  if (fast_axis(g.n[2])) {
     TRVG_LOGN_SWITCH(ilog2(g.n[2]), (launch_z<T, LG, Loader>(
         ctx, data, load, sign, read_bytes, zw, pr)));
   } else {
     launch_z_gen<T>(ctx, data, load, sign, read_bytes + zw, pr);
   }
-  if (fast_axis(g, g.n[1])) {
+  if (fast_axis(g.n[1])) {
     TRVG_LOGN_SWITCH(ilog2(g.n[1]), (launch_strided<T, LG>(
         ctx, data, g.n[2], (long long)g.n[1] * g.n[2], g.n[2], sign, pr, 1,
         zw + slab_vals * cb)));
@@ -891,7 +839,7 @@ void fft3d(Context& ctx, c2<T>* data, const Loader& load, int sign,
     launch_strided_gen<T>(ctx, data, g.n[1], g.n[2], (long long)g.n[1] * g.n[2], g.n[2],
                           sign, pr, 1, zw + slab_vals * cb);
   }
-  if (fast_axis(g, g.n[0])) {
+  if (fast_axis(g.n[0])) {
     TRVG_LOGN_SWITCH(ilog2(g.n[0]), (launch_strided<T, LG>(
         ctx, data, (long long)g.n[1] * g.n[2], 0, (long long)g.n[1] * g.n[2], sign,
         pr, 2, slab_vals * cb + double(g.nmesh) * cb)));

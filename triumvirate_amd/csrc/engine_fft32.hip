@@ -26,6 +26,8 @@ template void shell_slab_ifft<float, float>(Context&, float2*, const float2*,
                                             const trvg_binning&, const std::vector<int>&,
                                             const std::vector<int>&, int, int, bool);
 template void slab_fft<float>(Context&, c2<float>*, int);
+template void full_work<float>(const Geom&, int, std::vector<int2>&, std::vector<int2>&,
+                             std::vector<int2>&);
 template void sjl_slab_ifft<float>(Context&, c2<float>*, const double2*, const Spline&,
                                  const std::vector<double>&, const std::vector<int>&, int, int,
                                  bool);

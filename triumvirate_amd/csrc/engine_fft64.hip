@@ -10,6 +10,7 @@ TRVG_FFT3D_INST(LoadSame<double>)
 TRVG_FFT3D_INST(LoadScaleShift<double>)
 TRVG_FFT3D_INST(LoadLinear2<double>)
 TRVG_FFT3D_INST(LoadTwopt<double TRVG_COMMA double>)
+TRVG_FFT3D_INST(LoadTwopt<double TRVG_COMMA double TRVG_COMMA true>)
 TRVG_FFT3D_INST(LoadDeconv<double TRVG_COMMA double>)
 // Loaders of the differentiable path (engine_diff.hip).
 TRVG_FFT3D_INST(LoadReal<double>)
@@ -24,6 +25,8 @@ template void shell_slab_ifft<double, double>(Context&, c2<double>*, const doubl
                                            const trvg_binning&, const std::vector<int>&,
                                            const std::vector<int>&, int, int, bool);
 template void slab_fft<double>(Context&, c2<double>*, int);
+template void full_work<double>(const Geom&, int, std::vector<int2>&, std::vector<int2>&,
+                             std::vector<int2>&);
 template void sjl_slab_ifft<double>(Context&, c2<double>*, const double2*, const Spline&,
                                  const std::vector<double>&, const std::vector<int>&, int, int,
                                  bool);

@@ -198,9 +198,12 @@ BinnedStat stats_fourier(Context& ctx, const double2* fa, const double2* fb, cpl
 BinnedStat stats_config(Context& ctx, double2* t, const double2* fa, const double2* fb,
                         cplx sbar, int ell, int m, const trvg_binning& b) {
   const int nb = b.num_bins;
-  LoadTwopt<double, double> lt{fa, fb, ctx.tab, dmk(sbar.real(), sbar.imag()),
-                               1. / ctx.g.vol};
-  fft3d<double>(ctx, t, lt, +1, 2. * double(ctx.g.nmesh) * 16.);
+  const double2 sb = dmk(sbar.real(), sbar.imag());
+  const double rb = 2. * double(ctx.g.nmesh) * 16., iv = 1. / ctx.g.vol;
+  if (ctx.tab.interlace)
+    fft3d<double>(ctx, t, LoadTwopt<double, double, true>{fa, fb, ctx.tab, sb, iv}, +1, rb);
+  else
+    fft3d<double>(ctx, t, LoadTwopt<double, double>{fa, fb, ctx.tab, sb, iv}, +1, rb);
   DevArray<double> edges(nb + 1);
   ctx.upload(edges.get(), b.bin_edges, nb + 1);
   const unsigned grid = grid_for(ctx, ctx.g.nmesh, 4);

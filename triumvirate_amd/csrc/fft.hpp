@@ -1,18 +1,19 @@
 // fft.hpp -- 3-D complex FFT for gfx950: three batched 1-D passes, each a
-// radix-4/radix-2 Stockham autosort transform held in LDS (the
-// formulation of Govindaraju et al., "High performance discrete Fourier
-// transforms on graphics processors", SC 2008).
+// radix-4 Stockham autosort transform (the formulation of Govindaraju et
+// al., "High performance discrete Fourier transforms on graphics
+// processors", SC 2008) held in registers, eight elements of a line per
+// thread, with one exchange through LDS between its stages.
 //
 // Sizes: powers of two from 8 to 1024 per axis.  Sign convention as FFTW
 // (forward e^{-ikx}, backward e^{+ikx}), unnormalised.
 //
-// Each pass is in place: a workgroup loads E = 256*EPT complex elements
-// (L = E/n lines of one axis), transforms them in LDS and writes them back
-// to the same addresses, so no second buffer is needed.  The first pass
-// (along z, contiguous lines) takes a "loader" functor that produces each
-// input element from one or more source fields; shell filters, window
-// deconvolution, scalings and two-point products are fused there instead
-// of costing a separate read+write sweep of the mesh.
+// Each pass is in place: a workgroup takes whole lines of one axis, every
+// thread loads its eight elements, transforms them and writes them back to
+// the same addresses, so no second buffer is needed.  The first pass takes a
+// "loader" functor that produces each input element from one or more source
+// fields; shell filters, window deconvolution, scalings and two-point
+// products are fused there instead of costing a separate read+write sweep of
+// the mesh.
 #pragma once
 
 #include "common.hpp"
@@ -20,6 +21,7 @@
 namespace trvg {
 
 constexpr int FFT_THREADS = 256;
+
 
 // Global stores and loads of the passes' mesh data (one place for their
 // cache policy; plain accesses measured best: streaming hints gained on
@@ -29,11 +31,6 @@ __device__ __forceinline__ void st_mesh(c2<T>* p, c2<T> v) { *p = v; }
 
 template <typename T>
 __device__ __forceinline__ c2<T> ld_mesh(const c2<T>* p) { return *p; }
-
-// Elements per thread of a pass (a workgroup holds 256 * EPT elements).
-// Eight for both precisions: the FP32 passes are latency-bound, and the
-// smaller LDS footprint admits twice the workgroups per CU.
-template <typename T> struct FftEpt { static constexpr int v = 8; };
 
 // Workgroups are dispatched to the 8 XCDs round-robin by index; mapping
 // index b to logical block (b % 8) * (n / 8) + b / 8 gives each XCD (and
@@ -61,6 +58,25 @@ struct Prune {
     double kx = __dmul_rn(double(shifted(i, n0)), dk0);
     return __dmul_rn(kx, kx) < kcut2;
   }
+  // Largest |m| of a row index m with P1(i, m) (reach_j; -1: none), or with
+  // P2(m) (reach_i): the predicates fall with |m|, so rows compare as integers.
+  // Estimated in FP32 and settled by the predicate itself.
+  __device__ __forceinline__ int reach_j(int i) const {
+    const double kx = __dmul_rn(double(shifted(i, n0)), dk0);
+    return reach(__dmul_rn(kx, kx), dk1, n1 / 2);
+  }
+  __device__ __forceinline__ int reach_i() const { return reach(0., dk0, n0 / 2); }
+  __device__ __forceinline__ int reach(double k2, double dk, int top) const {
+    auto in = [&](int m) {
+      const double k = __dmul_rn(double(m), dk);
+      return __dadd_rn(k2, __dmul_rn(k, k)) < kcut2;
+    };
+    const float f = sqrtf(fmaxf(float(kcut2 - k2), 0.f)) / float(dk);
+    int m = f < float(top) ? int(f) : top;
+    while (m < top && in(m + 1)) m++;
+    while (m >= 0 && !in(m)) m--;
+    return m;
+  }
   __device__ __forceinline__ bool p1(int i, int j) const {
     double kx = __dmul_rn(double(shifted(i, n0)), dk0);
     double ky = __dmul_rn(double(shifted(j, n1)), dk1);
@@ -68,106 +84,8 @@ struct Prune {
   }
 };
 
-// In-LDS Stockham transform of L lines of length N (N = 2^LOGN) stored as
-// buf[line * (N + 1) + n] (one pad element per line against bank
-// conflicts).  W[m] = e^{sign 2 pi i m / N} (m < N) in LDS.
-template <typename T, int LOGN, int EPT>
-__device__ __forceinline__ void lds_fft_lines(c2<T>* buf, const c2<T>* W,
-                                              int sign) {
-  constexpr int N = 1 << LOGN;
-  constexpr int LS = N + 1;  // padded LDS line stride
-  constexpr int E = FFT_THREADS * EPT;
-  constexpr int NLINES = E / N;
-  const int t = threadIdx.x;
-  int Ns = 1;
-  int rem = LOGN;
-#pragma unroll
-  for (int stage = 0; stage < (LOGN + 1) / 2; stage++) {
-    if (rem >= 2) {
-      // radix-4
-      constexpr int NB = E / 4;               // butterflies per workgroup
-      constexpr int PER = NB / FFT_THREADS;   // = EPT / 4
-      c2<T> v[PER > 0 ? PER : 1][4];
-      int jj[PER > 0 ? PER : 1], ll[PER > 0 ? PER : 1];
-#pragma unroll
-      for (int u = 0; u < PER; u++) {
-        int b = t + u * FFT_THREADS;
-        int line = b / (N / 4);
-        int j = b % (N / 4);
-        jj[u] = j;
-        ll[u] = line;
-        int k = j & (Ns - 1);
-        const c2<T>* src = buf + line * LS;
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[u][q] = src[j + q * (N / 4)];
-        int tstep = k * (N / (Ns * 4));
-        v[u][1] = cmul<T>(v[u][1], W[tstep]);
-        v[u][2] = cmul<T>(v[u][2], W[2 * tstep]);
-        v[u][3] = cmul<T>(v[u][3], W[3 * tstep]);
-        c2<T> t0 = cadd<T>(v[u][0], v[u][2]);
-        c2<T> t1 = csub<T>(v[u][0], v[u][2]);
-        c2<T> t2 = cadd<T>(v[u][1], v[u][3]);
-        c2<T> d = csub<T>(v[u][1], v[u][3]);
-        // t3 = sign * i * d
-        c2<T> t3 = (sign < 0) ? mk<T>(d.y, -d.x) : mk<T>(-d.y, d.x);
-        v[u][0] = cadd<T>(t0, t2);
-        v[u][2] = csub<T>(t0, t2);
-        v[u][1] = cadd<T>(t1, t3);
-        v[u][3] = csub<T>(t1, t3);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < PER; u++) {
-        int j = jj[u];
-        int k = j & (Ns - 1);
-        int idxD = (j / Ns) * Ns * 4 + k;
-        c2<T>* dst = buf + ll[u] * LS;
-#pragma unroll
-        for (int q = 0; q < 4; q++) dst[idxD + q * Ns] = v[u][q];
-      }
-      __syncthreads();
-      Ns *= 4;
-      rem -= 2;
-    } else if (rem == 1) {
-      constexpr int NB = E / 2;
-      constexpr int PER = NB / FFT_THREADS;   // = EPT / 2
-      c2<T> v[PER][2];
-      int jj[PER], ll[PER];
-#pragma unroll
-      for (int u = 0; u < PER; u++) {
-        int b = t + u * FFT_THREADS;
-        int line = b / (N / 2);
-        int j = b % (N / 2);
-        jj[u] = j;
-        ll[u] = line;
-        int k = j & (Ns - 1);
-        const c2<T>* src = buf + line * LS;
-        v[u][0] = src[j];
-        v[u][1] = cmul<T>(src[j + N / 2], W[k * (N / (Ns * 2))]);
-        c2<T> a = v[u][0], bb = v[u][1];
-        v[u][0] = cadd<T>(a, bb);
-        v[u][1] = csub<T>(a, bb);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < PER; u++) {
-        int j = jj[u];
-        int k = j & (Ns - 1);
-        int idxD = (j / Ns) * Ns * 2 + k;
-        c2<T>* dst = buf + ll[u] * LS;
-        dst[idxD] = v[u][0];
-        dst[idxD + Ns] = v[u][1];
-      }
-      __syncthreads();
-      Ns *= 2;
-      rem -= 1;
-    }
-  }
-  (void)NLINES;
-}
-
 // ---------------------------------------------------------------------------
-// Register-resident DFTs for the z pass.
+// Register-resident DFTs.
 // ---------------------------------------------------------------------------
 
 // cos(pi k / 16) for k in [0, 16] (k > 8 by symmetry).
@@ -236,244 +154,205 @@ __device__ __forceinline__ void dft_reg(c2<T>* v, T sgn) {
   for (int k = 0; k < R; k++) v[k] = o[k];
 }
 
-// Shape of the register z pass for N = 2^LOGN = A * B: A threads per line,
-// B elements per thread (B a multiple of A); a workgroup takes the block of
-// every pass, FFT_THREADS * FftEpt<T> elements.
-template <int LOGN> struct ZRegShape { static constexpr bool ok = false; };
-template <> struct ZRegShape<8> {
-  static constexpr bool ok = true;
-  static constexpr int A = 16, B = 16;
-};
-template <> struct ZRegShape<9> {
-  static constexpr bool ok = true;
-  static constexpr int A = 16, B = 32;
-};
+// ---------------------------------------------------------------------------
+// Line transforms: N = 2^LOGN points as stages of radix 2^LR, the last one of
+// what is left.  Thread j < N / 8 of a line holds its elements j + e N / 8,
+// e < 8, before and after (so global accesses of neighbouring threads are
+// adjacent at both ends); between two stages the line goes through LDS once.
+//
+// Bound by HBM (80-90 % of the copy rate) where the mesh exceeds the caches.
+// Against radix-4 stages with the line in LDS throughout, a transform
+// crosses LDS 6 times instead of 10 (N = 256), starts from the loads
+// themselves and ends in the stores, and masked rows are loaded together
+// instead of one after the other.  Radix 4 (47 registers in FP32, 72 in
+// FP64 for N = 256: eight and seven waves per SIMD) beats radix 8 (90 and
+// 126), whose fewer exchanges do not make up for the waves.  Measured,
+// before and after, in us: strided pass of 256^3 FP32 63 -> 48, FP64 103 ->
+// 86, of 512^3 FP32 698 -> 455; y pass of 30 FP32 fields of 512^3 17.0 ->
+// 12.3 ms; masked z pass of the same 17.6 -> 11.6 ms (there against a
+// register transform of 16 x 32 points), of 12.5 FP64 fields of 256^3 849 ->
+// 574 us.
+// ---------------------------------------------------------------------------
+
+// Log2 of the radix of the stages.
+constexpr int FFT_LR = 2;
+
+// LDS position of element n: one element of padding per eight, which spreads
+// the writes of the first stage (stride 8) over all banks.
+__host__ __device__ __forceinline__ constexpr int fft_pad(int n) { return n + n / 8; }
+
+// LDS elements between the lines of a workgroup: nl lanes in a row belong to
+// different lines (1: to the same), and are kept on different banks.
 template <typename T>
-constexpr int zreg_block() { return FFT_THREADS * FftEpt<T>::v; }
+constexpr int fft_line_stride(int n, int nl) {
+  const int banks = 128 / int(sizeof(c2<T>));   // elements across the banks
+  const int base = fft_pad(n);
+  if (nl == 1) return base;
+  const int want = nl >= banks ? 1 : banks / nl;
+  return base + ((want - base) % banks + banks) % banks;
+}
+
+// Twiddles in LDS, per stage (span Ns, radix R) the (R - 1) Ns factors
+// w^{q k N / (Ns R)}, k fastest: N - 8 of them at most.  tw: e^{sign 2 pi i m / N}.
+template <typename T, int LOGN, int LR = FFT_LR, int LD = LR>
+__device__ __forceinline__ void fft_fill_twiddles(c2<T>* W, const c2<T>* __restrict__ tw,
+                                                  int t, int nt) {
+  if constexpr (LD < LOGN) {
+    constexpr int N = 1 << LOGN, Ns = 1 << LD;
+    constexpr int R = 1 << (LOGN - LD >= LR ? LR : LOGN - LD);
+    for (int i = t; i < (R - 1) * Ns; i += nt) {
+      const int q = i / Ns + 1, k = i % Ns;
+      W[i] = tw[q * k * (N / (Ns * R))];
+    }
+    fft_fill_twiddles<T, LOGN, LR, LD + LR>(W + (R - 1) * Ns, tw, t, nt);
+  }
+}
+
+// Stages from span 2^LD on.  `lb`: this line in LDS.  WAVE: the line's
+// threads are one wave's, which needs no barrier.  AGAIN: LDS may still be
+// read by an earlier transform of the workgroup.
+template <typename T, int LOGN, int LR, bool WAVE, bool AGAIN, int LD = 0>
+__device__ __forceinline__ void fft_stages(c2<T> (&v)[8], c2<T>* lb, const c2<T>* W, int j,
+                                           T sgn) {
+  constexpr int N = 1 << LOGN, M = N / 8, Ns = 1 << LD;
+  constexpr int R = 1 << (LOGN - LD >= LR ? LR : LOGN - LD);
+  constexpr int NB = 8 / R;                 // butterflies per thread
+  constexpr bool LAST = LD + LR >= LOGN;
+  auto sync = [] {
+    if (WAVE) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+      __syncthreads();
+    }
+  };
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const int jb = j + b * M, k = jb & (Ns - 1);
+    c2<T> x[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      x[q] = v[b + q * NB];
+      if (LD > 0 && q > 0) x[q] = cmul<T>(x[q], W[(q - 1) * Ns + k]);
+    }
+    dft_reg<T, R>(x, sgn);
+#pragma unroll
+    for (int r = 0; r < R; r++) v[b + r * NB] = x[r];
+  }
+  if constexpr (!LAST) {
+    if (LD > 0 || AGAIN) sync();
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      const int jb = j + b * M, k = jb & (Ns - 1);
+      const int d = (jb / Ns) * (Ns * R) + k;
+#pragma unroll
+      for (int r = 0; r < R; r++) lb[fft_pad(d + r * Ns)] = v[b + r * NB];
+    }
+    sync();
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = lb[fft_pad(j + e * M)];
+    fft_stages<T, LOGN, LR, WAVE, AGAIN, LD + LR>(v, lb, LD > 0 ? W + (R - 1) * Ns : W, j, sgn);
+  }
+}
+
+// Threads of a workgroup of the strided passes: rows of `bytes` contiguous
+// bytes (several lines of neighbouring columns), within 256..1024 threads.
+// From 512 points on 256 threads would hold rows of 32 bytes, half a sector
+// of HBM; up to 256 points rows of 64 bytes measured no slower than 128, and
+// the smaller blocks prune better.
 template <typename T, int LOGN>
-constexpr int zreg_threads() { return zreg_block<T>() / ZRegShape<LOGN>::B; }
+constexpr int strided_threads() {
+  const int bytes = LOGN >= 9 ? 128 : 64;
+  const int nt = bytes / int(sizeof(c2<T>)) * ((1 << LOGN) / 8);
+  return nt < 256 ? 256 : (nt > 1024 ? 1024 : nt);
+}
 template <typename T, int LOGN>
-constexpr size_t zreg_smem() {
-  return size_t((zreg_block<T>() >> LOGN) * ZRegShape<LOGN>::B *
-                    (ZRegShape<LOGN>::A + 1) +
+constexpr int strided_lines() { return strided_threads<T, LOGN>() * 8 >> LOGN; }
+template <typename T, int LOGN>
+constexpr size_t strided_smem() {
+  return size_t(strided_lines<T, LOGN>() *
+                    fft_line_stride<T>(1 << LOGN, strided_lines<T, LOGN>()) +
                 (1 << LOGN)) * sizeof(c2<T>);
 }
-
-// z pass of block `blk` (L = zreg_block / N whole lines) as
-// N = A * B: with n = n1 + A n2 and k = k2 + B k1,
-//   X[k2 + B k1] = sum_n1 w_A^{n1 k1} w_N^{n1 k2} sum_n2 x[n1 + A n2] w_B^{n2 k2}.
-// Thread (line, n1) loads its B elements (lanes of a line read A adjacent
-// elements per load), takes the inner DFT in registers, applies w_N^{n1 k2}
-// and writes to LDS; after one exchange each thread takes B / A outer DFTs
-// of length A in registers and stores A adjacent outputs per lane group.
-// One LDS round trip per element instead of one per radix-4 stage.
-// Loads of block `blk`: thread (l, q) takes elements k = q + A n2 of line
-// l of the block (lanes of a line read A adjacent elements per load).
-template <typename T, int LOGN, class Loader>
-__device__ __forceinline__ void zreg_load(c2<T>* v, const Loader& load, int n1,
-                                          long long blk) {
-  constexpr int N = 1 << LOGN;
-  constexpr int A = ZRegShape<LOGN>::A, B = ZRegShape<LOGN>::B;
-  constexpr int L = zreg_block<T>() / N;
-  const int l = threadIdx.x / A, q = threadIdx.x % A;
-  const long long line = blk * L + l;
-  const int i = int(line / n1), j = int(line % n1);
-  const long long g0 = line * N;
-#pragma unroll
-  for (int n2 = 0; n2 < B; n2++) {
-    const int k = q + A * n2;
-    v[n2] = load(g0 + k, i, j, k);
-  }
-}
-
-// Transform of the loaded block and its store: the inner DFT in registers,
-// w_N^{n1 k2} and one LDS exchange, the outer DFTs in registers, A adjacent
-// outputs per lane group.  W (the N twiddles) is in LDS; the LDS line
-// buffer may be reused by the next block of the workgroup.
+// Lines of a workgroup of the z pass (256 threads).
+constexpr int z_lines(int n) { return FFT_THREADS * 8 / n; }
 template <typename T, int LOGN>
-__device__ __forceinline__ void zreg_transform_store(c2<T>* v, c2<T>* __restrict__ data,
-                                                     const c2<T>* W, c2<T>* buf,
-                                                     int sign, long long blk) {
-  constexpr int N = 1 << LOGN;
-  constexpr int A = ZRegShape<LOGN>::A, B = ZRegShape<LOGN>::B;
-  constexpr int L = zreg_block<T>() / N;
-  constexpr int AP = A + 1;        // padded stride between k2 rows in LDS
-  constexpr int LSTR = B * AP;     // LDS elements per line
-  const int l = threadIdx.x / A, q = threadIdx.x % A;
-  const T sgn = T(sign);
-  dft_reg<T, B>(v, sgn);
-  __syncthreads();
-  c2<T>* lb = buf + l * LSTR;
-  lb[q] = v[0];
-#pragma unroll
-  for (int k2 = 1; k2 < B; k2++) lb[k2 * AP + q] = cmul<T>(v[k2], W[q * k2]);
-  __syncthreads();
-  c2<T>* out = data + (blk * L + l) * N;
-#pragma unroll
-  for (int r = 0; r < B / A; r++) {
-    const int k2 = q + A * r;
-    c2<T> u[A];
-#pragma unroll
-    for (int m = 0; m < A; m++) u[m] = lb[k2 * AP + m];
-    dft_reg<T, A>(u, sgn);
-#pragma unroll
-    for (int k1 = 0; k1 < A; k1++) st_mesh<T>(out + k2 + B * k1, u[k1]);
-  }
+constexpr size_t z_smem() {
+  return size_t(z_lines(1 << LOGN) * fft_line_stride<T>(1 << LOGN, 1) + (1 << LOGN)) *
+         sizeof(c2<T>);
 }
 
-// z pass of block `blk` (L = zreg_block / N whole lines) as
-// N = A * B: with n = n1 + A n2 and k = k2 + B k1,
-//   X[k2 + B k1] = sum_n1 w_A^{n1 k1} w_N^{n1 k2} sum_n2 x[n1 + A n2] w_B^{n2 k2}.
-// One LDS round trip per element instead of one per radix-4 stage.
-template <typename T, int LOGN, class Loader>
-__device__ __forceinline__ void fft_z_block_reg(c2<T>* __restrict__ data,
-                                                const Loader& load,
-                                                const c2<T>* __restrict__ tw, int n1,
-                                                int sign, const Prune& pr, long long blk) {
-  constexpr int N = 1 << LOGN;
-  constexpr int A = ZRegShape<LOGN>::A, B = ZRegShape<LOGN>::B;
-  constexpr int L = zreg_block<T>() / N;
-  constexpr int NT = L * A;
-  extern __shared__ char smem_raw[];
-  c2<T>* buf = reinterpret_cast<c2<T>*>(smem_raw);
-  c2<T>* W = buf + L * B * (A + 1);
-  const int t = threadIdx.x;
-  if (pr.on) {
-    // Skip the workgroup if none of its lines is needed (uniform exit).
-    bool any = false;
-    for (int ll = 0; ll < L && !any; ll++) {
-      const long long ln = blk * L + ll;
-      any = pr.p1(int(ln / n1), int(ln % n1));
-    }
-    if (!any) return;
-  }
-  for (int m = t; m < N; m += NT) W[m] = tw[m];
-  c2<T> v[B];
-  zreg_load<T, LOGN>(v, load, n1, blk);
-  zreg_transform_store<T, LOGN>(v, data, W, buf, sign, blk);
-}
-
-template <typename T, int LOGN, class Loader>
-__global__ void __launch_bounds__((zreg_threads<T, LOGN>()))
-fft_pass_z_reg(c2<T>* __restrict__ data, Loader load, const c2<T>* __restrict__ tw,
-               int n1, int sign, Prune pr) {
-  fft_z_block_reg<T, LOGN>(data, load, tw, n1, sign, pr, xcd_block(blockIdx.x, gridDim.x));
-}
-
-// Batched unpruned register z pass, two work items (field, block) per
-// workgroup: the loads of the second are issued before the first is
-// transformed, so each wave keeps twice the bytes in flight.
-template <typename T, int LOGN, class BatchLoader>
-__global__ void __launch_bounds__((zreg_threads<T, LOGN>()))
-fft_pass_z_batch_reg(c2<T>* __restrict__ base, long long fstride, BatchLoader load,
-                     const c2<T>* __restrict__ tw, int n1, int sign,
-                     const int2* __restrict__ work, int nwork) {
-  constexpr int N = 1 << LOGN;
-  constexpr int A = ZRegShape<LOGN>::A, B = ZRegShape<LOGN>::B;
-  constexpr int L = zreg_block<T>() / N;
-  constexpr int NT = L * A;
-  extern __shared__ char smem_raw[];
-  c2<T>* buf = reinterpret_cast<c2<T>*>(smem_raw);
-  c2<T>* W = buf + L * B * (A + 1);
-  for (int m = threadIdx.x; m < N; m += NT) W[m] = tw[m];
-  const long long b0 = 2LL * xcd_block(blockIdx.x, gridDim.x);
-  const bool two = b0 + 1 < nwork;   // uniform over the workgroup
-  const int2 w0 = work[b0];
-  c2<T> v[B], vn[B];
-  zreg_load<T, LOGN>(v, load.field(w0.x), n1, w0.y);
-  int2 w1 = w0;
-  if (two) {
-    w1 = work[b0 + 1];
-    zreg_load<T, LOGN>(vn, load.field(w1.x), n1, w1.y);
-  }
-  zreg_transform_store<T, LOGN>(v, base + w0.x * fstride, W, buf, sign, w0.y);
-  if (two) zreg_transform_store<T, LOGN>(vn, base + w1.x * fstride, W, buf, sign, w1.y);
-}
+// Loaders that read several fields or evaluate harmonics per cell.
+template <class Loader> struct HeavyLoader { static constexpr bool value = false; };
 
 // First pass along z (contiguous lines), with a fused loader, for block
-// `blk` of the mesh at `data`.
+// `blk` of the mesh at `data` (z_lines(N) lines; the last block of a mesh may
+// hold fewer of its nlines).
 // Loader: c2<T> operator()(long long g, int i, int j, int k) const.
-// FAST (n1 a multiple of the lines per block, as for every mesh whose z
-// size fits NLINES lines per row): the block's lines share i, so indices
-// need no division.
-template <typename T, int LOGN, int EPT, bool FAST, class Loader>
-__device__ __forceinline__ void fft_z_block(c2<T>* __restrict__ data,
-                                            const Loader& load,
-                                            const c2<T>* __restrict__ tw,
-                                            int n1, int sign, const Prune& pr,
+template <typename T, int LOGN, class Loader>
+__device__ __forceinline__ void fft_z_block(c2<T>* __restrict__ data, const Loader& load,
+                                            const c2<T>* __restrict__ tw, int n1,
+                                            long long nlines, int sign, const Prune& pr,
                                             long long blk) {
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  constexpr int NLINES = E / N;
-  extern __shared__ char smem_raw[];
-  constexpr int LS = N + 1;
+  constexpr int N = 1 << LOGN, M = N / 8;
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  constexpr int LS = fft_line_stride<T>(N, 1);
   c2<T>* buf = reinterpret_cast<c2<T>*>(smem_raw);
-  c2<T>* W = buf + NLINES * LS;
-  const int t = threadIdx.x;
-  const long long line0 = blk * NLINES;
-  const long long base = line0 * N;
-  const int i0 = int(line0 / n1), j0 = int(line0 % n1);
+  c2<T>* W = buf + z_lines(N) * LS;
+  const int t = threadIdx.x, l = t / M, j = t % M;
+  // Threads past the last line repeat it and do not write (loads without a
+  // branch stay in flight together).
+  const bool valid = blk * z_lines(N) + l < nlines;
+  const long long line = valid ? blk * z_lines(N) + l : nlines - 1;
+  const int i1 = int(unsigned(line) / unsigned(n1)), j1 = int(unsigned(line) % unsigned(n1));
   if (pr.on) {
     // Skip the workgroup if none of its lines is needed (uniform exit).
     bool any = false;
-    for (int l = 0; l < NLINES && !any; l++) {
-      if (FAST) {
-        any = pr.p1(i0, j0 + l);
-      } else {
-        const long long line = line0 + l;
-        any = pr.p1(int(line / n1), int(line % n1));
-      }
+    for (int q = 0; q < z_lines(N) && !any; q++) {
+      const long long ln = blk * z_lines(N) + q;
+      any = ln < nlines && pr.p1(int(ln / n1), int(ln % n1));
     }
     if (!any) return;
   }
-  for (int m = t; m < N; m += FFT_THREADS) W[m] = tw[m];
+  fft_fill_twiddles<T, LOGN>(W, tw, t, FFT_THREADS);
+  c2<T> v[8];
 #pragma unroll
-  for (int e = 0; e < EPT; e++) {
-    const int idx = t + e * FFT_THREADS;
-    const int k = idx % N;
-    int i, j;
-    if (FAST) {
-      i = i0;
-      j = j0 + idx / N;
-    } else {
-      const long long line = line0 + idx / N;
-      i = int(line / n1);
-      j = int(line % n1);
-    }
-    buf[(idx / N) * LS + k] = load(base + idx, i, j, k);
+  for (int e = 0; e < 8; e++) {
+    const int k = j + e * M;
+    v[e] = load(line * N + k, i1, j1, k);
+    // Loaders with per-cell arithmetic: four cells at a time, which keeps the
+    // registers (and with them the waves) of the pass within bounds.
+    if (HeavyLoader<Loader>::value && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   }
-  __syncthreads();
-  lds_fft_lines<T, LOGN, EPT>(buf, W, sign);
-  c2<T>* out = data + base;
+  if (M <= 64) __syncthreads();   // the twiddles; the stages stay within a wave
+  fft_stages<T, LOGN, FFT_LR, (M <= 64), false>(v, buf + l * LS, W, j, T(sign));
+  if (!valid) return;
+  c2<T>* out = data + line * N + j;
 #pragma unroll
-  for (int e = 0; e < EPT; e++) {
-    const int idx = t + e * FFT_THREADS;
-    st_mesh<T>(out + idx, buf[(idx / N) * LS + idx % N]);
-  }
+  for (int e = 0; e < 8; e++) st_mesh<T>(out + e * M, v[e]);
 }
 
-template <typename T, int LOGN, int EPT, bool FAST, class Loader>
+template <typename T, int LOGN, class Loader>
 __global__ void __launch_bounds__(FFT_THREADS)
 fft_pass_z(c2<T>* __restrict__ data, Loader load, const c2<T>* __restrict__ tw,
-           int n1, int sign, Prune pr) {
-  fft_z_block<T, LOGN, EPT, FAST>(data, load, tw, n1, sign, pr,
-                                  xcd_block(blockIdx.x, gridDim.x));
+           int n1, long long nlines, int sign, Prune pr) {
+  fft_z_block<T, LOGN>(data, load, tw, n1, nlines, sign, pr, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Batched first pass over several fields (a slab of meshes `fstride` apart):
 // work[b] = (field, block) lists only the blocks with needed lines, so
 // blocks outside every band cost nothing.  BatchLoader::field(q) returns
 // the loader of field q; kcut2[q] is that field's pruning radius.
-template <typename T, int LOGN, int EPT, bool FAST, class BatchLoader>
+template <typename T, int LOGN, class BatchLoader>
 __global__ void __launch_bounds__(FFT_THREADS)
 fft_pass_z_batch(c2<T>* __restrict__ base, long long fstride, BatchLoader load,
-                 const c2<T>* __restrict__ tw, int n1, int sign, Prune pr,
+                 const c2<T>* __restrict__ tw, int n1, long long nlines, int sign, Prune pr,
                  const double* __restrict__ kcut2, const int2* __restrict__ work) {
   const int2 wk = work[xcd_block(blockIdx.x, gridDim.x)];
   Prune p = pr;
   p.kcut2 = kcut2[wk.x];
-  fft_z_block<T, LOGN, EPT, FAST>(base + wk.x * fstride, load.field(wk.x), tw,
-                                  n1, sign, p, wk.y);
+  fft_z_block<T, LOGN>(base + wk.x * fstride, load.field(wk.x), tw, n1, nlines, sign, p, wk.y);
 }
 
 // Strided pass: lines of length N with element stride S.  Line `id` starts
@@ -481,225 +360,140 @@ fft_pass_z_batch(c2<T>* __restrict__ base, long long fstride, BatchLoader load,
 // adjacent in memory within a slice:
 //   y pass: S = n2, inner = n2, outer_stride = n1*n2;
 //   x pass: S = n1*n2, inner = n1*n2, outer_stride = 0.
-// Each workgroup takes L = E/N consecutive lines.
+// Each workgroup takes strided_lines consecutive lines (the last fewer).
 //
 // prune_mode (with pr.on): 1 = y pass (slab i = id / inner must satisfy P2,
 // row j read only where P1(i, j)); 2 = x pass (row i read only where P2(i));
 // 3 = y pass of the x-first order (Prune over the (z, y) axes: line k =
 // id % inner written only where P2(k), row j read only where P1(k, j)).
-//
-// FAST (inner a multiple of L): the block's lines lie in one slice, so the
-// slice's pruning flags go to LDS once per block and each thread steps a
-// pointer by a constant per element (thread t always owns line t % L).
-template <typename T, int LOGN, int EPT, bool FAST>
+template <typename T, int LOGN>
 __device__ __forceinline__ void fft_strided_block(
     c2<T>* __restrict__ data, const c2<T>* __restrict__ tw, long long S,
-    long long outer_stride, long long inner, int sign, const Prune& pr,
+    long long outer_stride, long long inner, long long nlines, int sign, const Prune& pr,
     int prune_mode, long long blk) {
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  constexpr int NLINES = E / N;
-  constexpr int NSTEP = FFT_THREADS / NLINES;   // rows advanced per element
-  extern __shared__ char smem_raw[];
-  constexpr int LS = N + 1;
+  constexpr int N = 1 << LOGN, M = N / 8;
+  constexpr int NL = strided_lines<T, LOGN>();
+  constexpr int LS = fft_line_stride<T>(N, NL);
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   c2<T>* buf = reinterpret_cast<c2<T>*>(smem_raw);
-  c2<T>* W = buf + NLINES * LS;
-  unsigned char* row_in = reinterpret_cast<unsigned char*>(W + N);   // [N]
-  const int t = threadIdx.x;
-  const long long id0 = blk * NLINES;
-  if (FAST) {
-    const long long slice0 = id0 / inner;
-    const bool m3 = pr.on && prune_mode == 3;
-    if (pr.on && prune_mode == 1 && !pr.p2(int(slice0))) return;
-    if (m3) {
-      bool any = false;
-      for (int l = 0; l < NLINES && !any; l++) any = pr.p2(int(id0 % inner) + l);
-      if (!any) return;
+  c2<T>* W = buf + NL * LS;
+  const int t = threadIdx.x, l = t % NL, j = t / NL;
+  const bool valid = blk * NL + l < nlines;
+  const long long id = valid ? blk * NL + l : nlines - 1;
+  // Line counts fit 32 bits (axes up to 2048).
+  const unsigned in = unsigned(inner), slice = unsigned(id) / in, col = unsigned(id) % in;
+  bool line_in = valid;
+  if (pr.on && prune_mode != 2) {
+    bool any = false;   // uniform exit when no line is needed
+    for (int q = 0; q < NL && !any; q++) {
+      const unsigned ln = unsigned(blk * NL + q);
+      any = ln < nlines && pr.p2(int(prune_mode == 1 ? ln / in : ln % in));
     }
-    for (int m = t; m < N; m += FFT_THREADS) {
-      W[m] = tw[m];
-      bool need = true;
-      if (pr.on) {
-        if (prune_mode == 1) need = pr.p1(int(slice0), m);
-        else if (prune_mode == 2) need = pr.p2(m);
-      }
-      row_in[m] = need;
-    }
-    __syncthreads();
-    const int l = t % NLINES, n0 = t / NLINES;
-    const int kl = int(id0 % inner) + l;   // this thread's line (prune mode 3)
-    c2<T>* line = data + (slice0 * outer_stride + id0 % inner + l);
-    const long long step = (long long)NSTEP * S;
-    c2<T>* p = line + (long long)n0 * S;
-#pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      const int n = n0 + e * NSTEP;
-      const bool need = m3 ? pr.p1(kl, n) : bool(row_in[n]);
-      buf[l * LS + n] = need ? ld_mesh<T>(p) : mk<T>(T(0), T(0));
-      p += step;
-    }
-    __syncthreads();
-    lds_fft_lines<T, LOGN, EPT>(buf, W, sign);
-    if (m3 && !pr.p2(kl)) return;
-    p = line + (long long)n0 * S;
-#pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      st_mesh<T>(p, buf[l * LS + n0 + e * NSTEP]);
-      p += step;
-    }
-    return;
-  }
-  if (pr.on && prune_mode == 1) {
-    bool any = false;
-    for (int l = 0; l < NLINES && !any; l++) any = pr.p2(int((id0 + l) / inner));
     if (!any) return;
+    line_in = valid && pr.p2(int(prune_mode == 1 ? slice : col));
   }
-  if (pr.on && prune_mode == 3) {
-    bool any = false;
-    for (int l = 0; l < NLINES && !any; l++) any = pr.p2(int((id0 + l) % inner));
-    if (!any) return;
-  }
-  for (int m = t; m < N; m += FFT_THREADS) W[m] = tw[m];
-  // Global element (n, l): line id0 + l, position n; LDS line-major [l][n].
+  fft_fill_twiddles<T, LOGN>(W, tw, t, strided_threads<T, LOGN>());
+  c2<T>* p = data + (long long)slice * outer_stride + col + (long long)j * S;
+  const long long step = (long long)M * S;
+  c2<T> v[8];
+  if (pr.on) {
+    const int reach =
+        !line_in ? -1 : (prune_mode == 2 ? pr.reach_i() : pr.reach_j(int(prune_mode == 1 ? slice : col)));
 #pragma unroll
-  for (int e = 0; e < EPT; e++) {
-    const int idx = t + e * FFT_THREADS;
-    const int n = idx / NLINES, l = idx % NLINES;
-    const long long id = id0 + l;
-    const long long base = (id / inner) * outer_stride + id % inner;
-    bool need = true;
-    if (pr.on) {
-      if (prune_mode == 1) {
-        const int i = int(id / inner);
-        need = pr.p2(i) && pr.p1(i, n);
-      } else if (prune_mode == 2) {
-        need = pr.p2(n);
-      } else if (prune_mode == 3) {
-        need = pr.p1(int(id % inner), n);
-      }
+    for (int e = 0; e < 8; e++) {
+      const int m = shifted(j + e * M, N);
+      v[e] = (m < 0 ? -m : m) <= reach ? ld_mesh<T>(p + e * step) : mk<T>(T(0), T(0));
     }
-    buf[l * LS + n] = need ? ld_mesh<T>(data + base + (long long)n * S) : mk<T>(T(0), T(0));
-  }
-  __syncthreads();
-  lds_fft_lines<T, LOGN, EPT>(buf, W, sign);
+  } else {
 #pragma unroll
-  for (int e = 0; e < EPT; e++) {
-    const int idx = t + e * FFT_THREADS;
-    const int n = idx / NLINES, l = idx % NLINES;
-    const long long id = id0 + l;
-    const long long base = (id / inner) * outer_stride + id % inner;
-    if (pr.on && prune_mode == 1 && !pr.p2(int(id / inner))) continue;
-    if (pr.on && prune_mode == 3 && !pr.p2(int(id % inner))) continue;
-    st_mesh<T>(data + base + (long long)n * S, buf[l * LS + n]);
+    for (int e = 0; e < 8; e++) v[e] = ld_mesh<T>(p + e * step);
   }
+  fft_stages<T, LOGN, FFT_LR, false, false>(v, buf + l * LS, W, j, T(sign));
+  if (!line_in) return;
+#pragma unroll
+  for (int e = 0; e < 8; e++) st_mesh<T>(p + e * step, v[e]);
 }
 
-template <typename T, int LOGN, int EPT, bool FAST>
-__global__ void __launch_bounds__(FFT_THREADS)
+template <typename T, int LOGN>
+__global__ void __launch_bounds__((strided_threads<T, LOGN>()))
 fft_pass_strided(c2<T>* __restrict__ data, const c2<T>* __restrict__ tw,
-                 long long S, long long outer_stride, long long inner,
+                 long long S, long long outer_stride, long long inner, long long nlines,
                  int sign, Prune pr, int prune_mode) {
-  fft_strided_block<T, LOGN, EPT, FAST>(data, tw, S, outer_stride, inner, sign, pr,
-                                        prune_mode, xcd_block(blockIdx.x, gridDim.x));
+  fft_strided_block<T, LOGN>(data, tw, S, outer_stride, inner, nlines, sign, pr, prune_mode,
+                             xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Batched strided pass over a slab of fields, work[b] = (field, block).
-template <typename T, int LOGN, int EPT, bool FAST>
-__global__ void __launch_bounds__(FFT_THREADS)
+template <typename T, int LOGN>
+__global__ void __launch_bounds__((strided_threads<T, LOGN>()))
 fft_pass_strided_batch(c2<T>* __restrict__ base, long long fstride,
                        const c2<T>* __restrict__ tw, long long S,
-                       long long outer_stride, long long inner, int sign,
+                       long long outer_stride, long long inner, long long nlines, int sign,
                        Prune pr, const double* __restrict__ kcut2,
                        const int2* __restrict__ work, int prune_mode) {
   const int2 wk = work[xcd_block(blockIdx.x, gridDim.x)];
   Prune p = pr;
   p.kcut2 = kcut2[wk.x];
-  fft_strided_block<T, LOGN, EPT, FAST>(base + wk.x * fstride, tw, S, outer_stride,
-                                        inner, sign, p, prune_mode, wk.y);
+  fft_strided_block<T, LOGN>(base + wk.x * fstride, tw, S, outer_stride, inner, nlines, sign,
+                             p, prune_mode, wk.y);
 }
 
 // First pass of the x-first order: lines along x (length N = n0, element
 // stride S = n1 n2), line id = j n2 + k, with a fused loader
 // load(g, i, j, k).  Prune over the (z, y) axes: a block runs only if one of
-// its lines has P1(k, j); it writes all its lines (lines outside the band
-// load as zeros).  FAST (n2 a multiple of the lines per block): the block's
-// lines share j.
-template <typename T, int LOGN, int EPT, bool FAST, class Loader>
+// its lines has P1(k, j), and only those lines are written (the y pass
+// reads no other).
+template <typename T, int LOGN, class Loader>
 __device__ __forceinline__ void fft_x_load_block(c2<T>* __restrict__ data,
                                                  const Loader& load,
                                                  const c2<T>* __restrict__ tw,
                                                  int n1, int n2, int sign,
                                                  const Prune& pr, long long blk) {
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  constexpr int NLINES = E / N;
-  constexpr int NSTEP = FFT_THREADS / NLINES;
-  extern __shared__ char smem_raw[];
-  constexpr int LS = N + 1;
+  constexpr int N = 1 << LOGN, M = N / 8;
+  constexpr int NL = strided_lines<T, LOGN>();
+  constexpr int LS = fft_line_stride<T>(N, NL);
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   c2<T>* buf = reinterpret_cast<c2<T>*>(smem_raw);
-  c2<T>* W = buf + NLINES * LS;
-  const int t = threadIdx.x;
+  c2<T>* W = buf + NL * LS;
+  const int t = threadIdx.x, l = t % NL, r0 = t / NL;
   const long long S = (long long)n1 * n2;
-  const long long id0 = blk * NLINES;
+  const long long id = blk * NL + l;
+  const int j = int(unsigned(id) / unsigned(n2)), k = int(unsigned(id) % unsigned(n2));
+  bool line_in = id < S;
   if (pr.on) {
-    bool any = false;
-    for (int l = 0; l < NLINES && !any; l++) {
-      const long long id = id0 + l;
-      any = pr.p1(int(id % n2), int(id / n2));
+    bool any = false;   // uniform exit when no line is needed
+    for (int q = 0; q < NL && !any; q++) {
+      const unsigned ln = unsigned(blk * NL + q);
+      any = ln < S && pr.p1(int(ln % unsigned(n2)), int(ln / unsigned(n2)));
     }
     if (!any) return;
+    line_in = line_in && pr.p1(k, j);
   }
-  for (int m = t; m < N; m += FFT_THREADS) W[m] = tw[m];
-  if (FAST) {
-    const int l = t % NLINES, r0 = t / NLINES;
-    const int j = int(id0 / n2), k = int(id0 % n2) + l;
-    const long long g0 = id0 + l;
+  fft_fill_twiddles<T, LOGN>(W, tw, t, strided_threads<T, LOGN>());
+  c2<T> v[8];
 #pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      const int n = r0 + e * NSTEP;
-      buf[l * LS + n] = load(g0 + (long long)n * S, n, j, k);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      const int idx = t + e * FFT_THREADS;
-      const int n = idx / NLINES, l = idx % NLINES;
-      const long long id = id0 + l;
-      buf[l * LS + n] = load(id + (long long)n * S, n, int(id / n2), int(id % n2));
-    }
+  for (int e = 0; e < 8; e++) {
+    const int n = r0 + e * M;
+    v[e] = line_in ? load(id + (long long)n * S, n, j, k) : mk<T>(T(0), T(0));
+    if (HeavyLoader<Loader>::value && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   }
-  __syncthreads();
-  lds_fft_lines<T, LOGN, EPT>(buf, W, sign);
-  if (FAST) {
-    const int l = t % NLINES, r0 = t / NLINES;
-    c2<T>* p = data + id0 + l + (long long)r0 * S;
-    const long long step = (long long)NSTEP * S;
+  fft_stages<T, LOGN, FFT_LR, false, false>(v, buf + l * LS, W, r0, T(sign));
+  if (!line_in) return;
 #pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      st_mesh<T>(p, buf[l * LS + r0 + e * NSTEP]);
-      p += step;
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      const int idx = t + e * FFT_THREADS;
-      const int n = idx / NLINES, l = idx % NLINES;
-      st_mesh<T>(data + id0 + l + (long long)n * S, buf[l * LS + n]);
-    }
-  }
+  for (int e = 0; e < 8; e++) st_mesh<T>(data + id + (long long)(r0 + e * M) * S, v[e]);
 }
 
 // Batched x-first loader pass, work[b] = (field, block).
-template <typename T, int LOGN, int EPT, bool FAST, class BatchLoader>
-__global__ void __launch_bounds__(FFT_THREADS)
+template <typename T, int LOGN, class BatchLoader>
+__global__ void __launch_bounds__((strided_threads<T, LOGN>()))
 fft_pass_x_load_batch(c2<T>* __restrict__ base, long long fstride, BatchLoader load,
                       const c2<T>* __restrict__ tw, int n1, int n2, int sign, Prune pr,
                       const double* __restrict__ kcut2, const int2* __restrict__ work) {
   const int2 wk = work[xcd_block(blockIdx.x, gridDim.x)];
   Prune p = pr;
   p.kcut2 = kcut2[wk.x];
-  fft_x_load_block<T, LOGN, EPT, FAST>(base + wk.x * fstride, load.field(wk.x), tw, n1,
-                                       n2, sign, p, wk.y);
+  fft_x_load_block<T, LOGN>(base + wk.x * fstride, load.field(wk.x), tw, n1, n2, sign, p,
+                            wk.y);
 }
 
 // Identity loader (plain in-place transform).

@@ -260,11 +260,10 @@ struct LoadShellPairBatch {
 template <typename T>
 struct LoadMaskedZ {
   const c2<T>* src;
-  double kcut2, dkz;
-  int nz;
+  int reach, nz;   // rows |k| <= reach were written
   __device__ c2<T> operator()(long long g, int, int, int k) const {
-    const double kz = __dmul_rn(double(shifted(k, nz)), dkz);
-    return __dmul_rn(kz, kz) < kcut2 ? ld_mesh<T>(src + g) : mk<T>(T(0), T(0));
+    const int m = shifted(k, nz);
+    return (m < 0 ? -m : m) <= reach ? ld_mesh<T>(src + g) : mk<T>(T(0), T(0));
   }
 };
 
@@ -276,7 +275,11 @@ struct LoadMaskedZBatch {
   double dkz;
   int nz;
   __device__ LoadMaskedZ<T> field(int f) const {
-    return LoadMaskedZ<T>{base + (long long)f * fstride, kcut2[f], dkz, nz};
+    Prune p{};
+    p.kcut2 = kcut2[f];
+    p.dk0 = dkz;
+    p.n0 = nz;
+    return LoadMaskedZ<T>{base + (long long)f * fstride, p.reach_i(), nz};
   }
 };
 
@@ -310,35 +313,43 @@ struct LoadShellBatch {
 // of its elements once, then for each transform fills LDS with
 // j_l(|k| r_f) times that factor (PACKED: two radii in the real and
 // imaginary parts, r < 0 absent), transforms and writes field f.
-template <typename T, int LOGN, int EPT, bool PACKED>
-__global__ void __launch_bounds__(FFT_THREADS)
+// Radix-8 stages: the factors and |k| of its elements leave few waves to
+// hide barriers behind, so fewer stages win (512^3 FP32, 30 fields: 14.7 ms
+// against 19.4 with radix 4).
+constexpr int SJL_LR = 3;
+
+// FAR: some |k| r reaches the end of the spline, past which j_l is evaluated
+// directly; without it the kernel does not carry that code's registers.
+template <typename T, int LOGN, bool PACKED, bool FAR>
+__global__ void __launch_bounds__((strided_threads<T, LOGN>()))
 fft_x_sjl_multi(c2<T>* __restrict__ base, long long fstride, int nt,
                 const double2* __restrict__ src, AxisTables tab, Geom geo, SplineDev sj,
                 const double* __restrict__ r, int ell, int m,
                 const c2<T>* __restrict__ tw) {
-  constexpr int N = 1 << LOGN;
-  constexpr int E = FFT_THREADS * EPT;
-  constexpr int NLINES = E / N;
-  constexpr int LS = N + 1;
-  extern __shared__ char smem_raw[];
+  constexpr int N = 1 << LOGN, M = N / 8;
+  constexpr int NL = strided_lines<T, LOGN>();
+  constexpr int LS = fft_line_stride<T>(N, NL);
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   c2<T>* buf = reinterpret_cast<c2<T>*>(smem_raw);
-  c2<T>* W = buf + NLINES * LS;
-  const int t = threadIdx.x;
+  c2<T>* W = buf + NL * LS;
+  const int t = threadIdx.x, l = t % NL, r0 = t / NL;
   const int n1 = geo.n[1], n2 = geo.n[2];
   const long long S = (long long)n1 * n2;
-  const long long id0 = xcd_block(blockIdx.x, gridDim.x) * NLINES;
-  for (int q = t; q < N; q += FFT_THREADS) W[q] = tw[q];
+  const long long id = xcd_block(blockIdx.x, gridDim.x) * NL + l;
+  const bool valid = id < S;
+  fft_fill_twiddles<T, LOGN, SJL_LR>(W, tw, t, strided_threads<T, LOGN>());
   // Per element: y_lm src / W / V in the working precision (FP32 fields
   // take j_l and the product in FP32) and |k|.
-  c2<T> fac[EPT];
-  double km[EPT];
+  c2<T> fac[8];
+  double km[8];
   const double inv_vol = 1. / geo.vol;
+  const int j = int(unsigned(id) / unsigned(n2)), k = int(unsigned(id) % unsigned(n2));
 #pragma unroll
-  for (int e = 0; e < EPT; e++) {
-    const int idx = t + e * FFT_THREADS;
-    const int n = idx / NLINES, l = idx % NLINES;
-    const long long id = id0 + l;
-    const int j = int(id / n2), k = int(id % n2);
+  for (int e = 0; e < 8; e++) {
+    const int n = r0 + e * M;
+    fac[e] = mk<T>(T(0), T(0));
+    km[e] = 0.;
+    if (!valid) continue;
     const double kx = grid_coord(n, geo.n[0], geo.dk[0]);
     const double ky = grid_coord(j, n1, geo.dk[1]);
     const double kz = grid_coord(k, n2, geo.dk[2]);
@@ -349,37 +360,27 @@ fft_x_sjl_multi(c2<T>* __restrict__ base, long long fstride, int nt,
     fac[e] = mk<T>(T(fe.x), T(fe.y));
   }
   for (int f = 0; f < nt; f++) {
-    const double r0 = PACKED ? r[2 * f] : r[f];
-    const double r1 = PACKED ? r[2 * f + 1] : -1.;
+    const double ra = PACKED ? r[2 * f] : r[f];
+    const double rb = PACKED ? r[2 * f + 1] : -1.;
+    c2<T> v[8];
 #pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      const int idx = t + e * FFT_THREADS;
+    for (int e = 0; e < 8; e++) {
       T j0, j1 = T(0);
       if (sizeof(T) == 4) {
-        j0 = T(sj.eval32(km[e] * r0));
-        if (PACKED && r1 >= 0.) j1 = T(sj.eval32(km[e] * r1));
+        j0 = T(sj.eval32<FAR>(km[e] * ra));
+        if (PACKED && rb >= 0.) j1 = T(sj.eval32<FAR>(km[e] * rb));
       } else {
-        j0 = T(sj.eval(km[e] * r0));
-        if (PACKED && r1 >= 0.) j1 = T(sj.eval(km[e] * r1));
+        j0 = T(sj.eval<FAR>(km[e] * ra));
+        if (PACKED && rb >= 0.) j1 = T(sj.eval<FAR>(km[e] * rb));
       }
-      c2<T> val;
-      if (PACKED) {
-        val = mk<T>(j0 * fac[e].x - j1 * fac[e].y, j0 * fac[e].y + j1 * fac[e].x);
-      } else {
-        val = mk<T>(j0 * fac[e].x, j0 * fac[e].y);
-      }
-      buf[(idx % NLINES) * LS + idx / NLINES] = val;
+      v[e] = PACKED ? mk<T>(j0 * fac[e].x - j1 * fac[e].y, j0 * fac[e].y + j1 * fac[e].x)
+                    : mk<T>(j0 * fac[e].x, j0 * fac[e].y);
     }
-    __syncthreads();
-    lds_fft_lines<T, LOGN, EPT>(buf, W, +1);
-    c2<T>* out = base + (long long)f * fstride;
+    fft_stages<T, LOGN, SJL_LR, false, true>(v, buf + l * LS, W, r0, T(1));
+    if (!valid) continue;
+    c2<T>* out = base + (long long)f * fstride + id;
 #pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      const int idx = t + e * FFT_THREADS;
-      const int n = idx / NLINES, l = idx % NLINES;
-      out[id0 + l + (long long)n * S] = buf[l * LS + n];
-    }
-    __syncthreads();
+    for (int e = 0; e < 8; e++) st_mesh<T>(out + (long long)(r0 + e * M) * S, v[e]);
   }
 }
 
@@ -454,7 +455,9 @@ fft_x_sjl_multi_gen(c2<T>* __restrict__ base, long long fstride, int nt,
 }
 
 // (f_a f_b^* / C1 - S C1 / C1) / V  (field.cpp:3007-3025, 3271-3289).
-template <typename T, typename S = T>
+// ILV: interlaced meshes; a template parameter so that the plain loader does
+// not carry the registers of the isotropic C1 (sines and cosines per cell).
+template <typename T, typename S = T, bool ILV = false>
 struct LoadTwopt {
   const c2<S>* fa;
   const c2<S>* fb;
@@ -467,14 +470,28 @@ struct LoadTwopt {
     c2<S> a = fa[g], b = fb[g];
     if (g == 0) b.x += S(fb_dc);
     double2 pk = dmul(dmk(a.x, a.y), dmk(b.x, -double(b.y)));
-    double c1 = alias_at(tab, i, j, k);
-    double w = tab.interlace ? window_at(tab, i, j, k) * window_at(tab, i, j, k)
-                             : c1;
-    double2 sn = dmk(sbar.x * c1 / w, sbar.y * c1 / w);
-    pk = dmk(pk.x / w - sn.x, pk.y / w - sn.y);
-    return mk<T>(T(pk.x * inv_vol), T(pk.y * inv_vol));
+    double iw, cw;   // 1 / W and C1 / W; W = C1 for plain meshes
+    if (ILV) {
+      const double w = window_at(tab, i, j, k);
+      iw = 1. / (w * w);
+      cw = alias_at(tab, i, j, k) * iw;
+    } else {
+      iw = 1. / (c1_axis(tab.sin2[0][i], tab.order) * c1_axis(tab.sin2[1][j], tab.order) *
+                 c1_axis(tab.sin2[2][k], tab.order));
+      cw = 1.;
+    }
+    return mk<T>(T((pk.x * iw - sbar.x * cw) * inv_vol), T((pk.y * iw - sbar.y * cw) * inv_vol));
   }
 };
+
+template <typename T, typename S, bool ILV>
+struct HeavyLoader<LoadTwopt<T, S, ILV>> { static constexpr bool value = true; };
+template <typename T, typename S>
+struct HeavyLoader<LoadDeconv<T, S>> { static constexpr bool value = true; };
+template <typename T, typename S>
+struct HeavyLoader<LoadShell<T, S>> { static constexpr bool value = true; };
+template <typename T, typename S>
+struct HeavyLoader<LoadShellPair<T, S>> { static constexpr bool value = true; };
 
 // ---------------------------------------------------------------------------
 // Bin location
