@@ -131,7 +131,7 @@ static void launch_z_gen(Context& ctx, c2<T>* data, const Loader& load, int sign
   const int N = ctx.g.n[2];
   const GenPlan P = make_gen_plan(N);
   const long long nlines = (long long)ctx.g.n[0] * ctx.g.n[1];
-  const size_t smem = gen_smem<T>(N, false);
+  const size_t smem = gen_smem<T>(N);
   auto kern = fft_pass_z_gen<T, Loader>;
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
@@ -147,13 +147,13 @@ static void launch_strided_gen(Context& ctx, c2<T>* data, int N, long long S,
                                const Prune& pr, int prune_mode, double bytes) {
   const GenPlan P = make_gen_plan(N);
   const long long nlines = ctx.g.nmesh / N;
-  const size_t smem = gen_smem<T>(N, true);
+  const size_t smem = gen_smem<T>(N);
   auto kern = fft_pass_strided_gen<T>;
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(blocks_of(nlines, P.nl))), dim3(FFT_THREADS), smem,
                      ctx.stream, data, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
-                     nlines, pr, prune_mode, P);
+                     nlines, sign, pr, prune_mode, P);
   TRVG_LAUNCH_CHECK();
 }
 
@@ -164,7 +164,7 @@ static void launch_z_batch_gen(Context& ctx, c2<T>* base, const BatchLoader& loa
   const int N = ctx.g.n[2];
   const GenPlan P = make_gen_plan(N);
   const long long nlines = (long long)ctx.g.n[0] * ctx.g.n[1];
-  const size_t smem = gen_smem<T>(N, false);
+  const size_t smem = gen_smem<T>(N);
   auto kern = fft_pass_z_batch_gen<T, BatchLoader>;
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
@@ -181,13 +181,13 @@ static void launch_strided_batch_gen(Context& ctx, c2<T>* base, int N, long long
                                      int nwork, int prune_mode, double bytes) {
   const GenPlan P = make_gen_plan(N);
   const long long nlines = ctx.g.nmesh / N;
-  const size_t smem = gen_smem<T>(N, true);
+  const size_t smem = gen_smem<T>(N);
   auto kern = fft_pass_strided_batch_gen<T>;
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
                      ctx.g.nmesh, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
-                     nlines, pr, kcut2, work, prune_mode, P);
+                     nlines, sign, pr, kcut2, work, prune_mode, P);
   TRVG_LAUNCH_CHECK();
 }
 
@@ -458,7 +458,7 @@ static void launch_x_load_batch_gen(Context& ctx, c2<T>* base, const BatchLoader
                                     int nwork, double bytes) {
   const int N = ctx.g.n[0];
   const GenPlan P = make_gen_plan(N);
-  const size_t smem = gen_smem<T>(N, false);
+  const size_t smem = gen_smem<T>(N);
   auto kern = fft_pass_x_load_batch_gen<T, BatchLoader>;
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
@@ -701,7 +701,7 @@ static void launch_x_sjl_gen(Context& ctx, c2<T>* base, int nt, const double2* s
   const Geom& g = ctx.g;
   const int N = g.n[0];
   const GenPlan P = make_gen_plan(N);
-  const size_t smem = gen_smem<T>(N, false);
+  const size_t smem = gen_smem<T>(N);
   const unsigned grid = unsigned(blocks_of((long long)g.n[1] * g.n[2], P.nl));
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   if (packed) {

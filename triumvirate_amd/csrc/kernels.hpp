@@ -393,7 +393,7 @@ fft_x_sjl_multi_gen(c2<T>* __restrict__ base, long long fstride, int nt,
                     const double2* __restrict__ src, AxisTables tab, Geom geo,
                     SplineDev sj, const double* __restrict__ r, int ell, int m,
                     const c2<T>* __restrict__ tw, GenPlan P) {
-  constexpr int MAXE = GEN_ELEMS / FFT_THREADS;
+  constexpr int MAXE = GEN_MAXE;
   const int N = P.n, LS = N + 1;
   GenSmem<T> sm(P);
   const int n1 = geo.n[1], n2 = geo.n[2];
@@ -403,6 +403,9 @@ fft_x_sjl_multi_gen(c2<T>* __restrict__ base, long long fstride, int nt,
   const int nl = int(min((long long)P.nl, S - id0));
   const int total = nl * N;
   for (int q = threadIdx.x; q < N; q += FFT_THREADS) sm.W[q] = tw[q];
+  const GenSplit jk(id0, n2);
+  const bool whole = nl == P.nl;
+  auto split = [&](int idx) { return whole ? P.by_nl.div(idx) : idx / nl; };
   c2<T> fac[MAXE];
   double km[MAXE];
   const double inv_vol = 1. / geo.vol;
@@ -412,9 +415,10 @@ fft_x_sjl_multi_gen(c2<T>* __restrict__ base, long long fstride, int nt,
     fac[e] = mk<T>(T(0), T(0));
     km[e] = 0.;
     if (idx >= total) continue;
-    const int n = idx / nl, l = idx % nl;
+    const int n = split(idx), l = idx - n * nl;
     const long long id = id0 + l;
-    const int j = int(id / n2), k = int(id % n2);
+    int j, k;
+    jk.at(l, j, k);
     const double kx = grid_coord(n, geo.n[0], geo.dk[0]);
     const double ky = grid_coord(j, n1, geo.dk[1]);
     const double kz = grid_coord(k, n2, geo.dk[2]);
@@ -441,13 +445,14 @@ fft_x_sjl_multi_gen(c2<T>* __restrict__ base, long long fstride, int nt,
       }
       const c2<T> val = PACKED ? mk<T>(j0 * fac[e].x - j1 * fac[e].y, j0 * fac[e].y + j1 * fac[e].x)
                                : mk<T>(j0 * fac[e].x, j0 * fac[e].y);
-      sm.a[(idx % nl) * LS + idx / nl] = val;
+      const int n = split(idx);
+      sm.a[(idx - n * nl) * LS + n] = val;
     }
     __syncthreads();
-    const c2<T>* R = lds_fft_gen<T>(sm.a, sm.b, sm.W, P, nl);
+    const c2<T>* R = lds_fft_gen<T>(sm.a, sm.b, sm.W, P, nl, +1);
     c2<T>* out = base + (long long)f * fstride;
     for (int idx = threadIdx.x; idx < total; idx += FFT_THREADS) {
-      const int n = idx / nl, l = idx % nl;
+      const int n = split(idx), l = idx - n * nl;
       st_mesh<T>(out + id0 + l + (long long)n * S, R[l * LS + n]);
     }
     __syncthreads();
