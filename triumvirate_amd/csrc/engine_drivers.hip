@@ -694,10 +694,11 @@ struct TwoPt {
   std::vector<cplx> pk, sn;
 };
 
-// FieldStats::compute_ylm_wgtd_2pt_stats_in_fourier (field.cpp:2511-2703).
+// FieldStats::compute_ylm_wgtd_2pt_stats_in_fourier (field.cpp:2511-2703);
+// fb_dc is added to fb at k = 0.
 template <typename T>
-static void twopt_fourier(Context& ctx, const c2<T>* fa, const c2<T>* fb, cplx sbar,
-                          int ell, int m, const trvg_binning& kb, double modes_in_range,
+static void twopt_fourier(Context& ctx, const c2<T>* fa, const c2<T>* fb, double fb_dc,
+                          cplx sbar, int ell, int m, const trvg_binning& kb, double modes_in_range,
                           std::function<void(TwoPt&&)> sink) {
   const int nb = kb.num_bins;
   std::shared_ptr<const TwoptMapData> map = twopt_map(ctx, kb.bin_edges, nb);
@@ -712,7 +713,7 @@ static void twopt_fourier(Context& ctx, const c2<T>* fa, const c2<T>* fb, cplx s
   hipLaunchKernelGGL(kern, dim3(grid), dim3(RED_THREADS),
                      twopt_smem(nb, 4, ctx.g), ctx.stream, fa, fb, ctx.g, ctx.tab,
                      dmk(sbar.real(), sbar.imag()), ell, m, map->view(), nb,
-                     cnt.get(), part.get());
+                     cnt.get(), part.get(), fb_dc);
   TRVG_LAUNCH_CHECK();
   reduce_cols(ctx, part.get(), int(grid), nb * 4, sum.get());
   const unsigned long long* hc = ctx.download(cnt.get(), nb);
@@ -1199,15 +1200,19 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
 
   // Common fields in FP64 whatever the shell precision T: the shot-noise
   // path (two-point statistics, S_ij_k) subtracts nearly equal quantities.
-  DevArray<double2> dn00 = take_prefill(0, 0), N00(nm);
+  DevArray<double2> dn00 = take_prefill(0, 0), N00(survey ? nm : 0);
   const bool dn00_pre = dn00.get() != nullptr;
   if (!dn00_pre) dn00.reset(nm);
   if (survey) {
     build_survey_pair_k(ctx, dn00.get(), N00.get(), d, *r, alpha, 0, 0, dn00_pre);
   } else {
     build_field_k<double>(ctx, dn00.get(), d, r, false, alpha, 0, 0, false, true);
-    build_field_k<double>(ctx, N00.get(), d, r, false, alpha, 0, 0, true, false);
   }
+  // A box has unit weights: N_00 is the density itself, dn_00 with the mean
+  // (the particle count) back at k = 0, so it is neither assigned nor
+  // transformed.
+  const double2* N00p = survey ? N00.get() : dn00.get();
+  const double N_dc = survey ? 0. : double(d.n);
   ShellStats ss = shell_stats(ctx, kb);
   double modes_in_range = 0.;
   for (int n : ss.nmodes) modes_in_range += n;
@@ -1290,7 +1295,7 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
     for (const Term& tm : enumerate_terms(p, survey)) {
       const bool lm_zero = !survey || (p.ELL == 0 && tm.M == 0);
       const double2* dnLMp = dn00.get();
-      const double2* NLMp = N00.get();
+      const double2* NLMp = N00p;
       if (!lm_zero) {
         if (!NLM.get()) NLM.reset(nm);
         DevArray<double2> own = take_prefill(p.ELL, tm.M);
@@ -1384,15 +1389,15 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
       };
       const bool shared = p.ell1 == 0 && p.ell2 == 0 && tm.m1 == tm.m2;
       if (p.ell2 == 0)
-        twopt_fourier<double>(ctx, dn00.get(), NLMp, Sbar, p.ell1, tm.m1, kb,
+        twopt_fourier<double>(ctx, dn00.get(), NLMp, N_dc, Sbar, p.ell1, tm.m1, kb,
                               modes_in_range, twopt_sink(true, shared));
       if (p.ell1 == 0 && !shared)
-        twopt_fourier<double>(ctx, dn00.get(), NLMp, Sbar, p.ell2, tm.m2, kb,
+        twopt_fourier<double>(ctx, dn00.get(), NLMp, N_dc, Sbar, p.ell2, tm.m2, kb,
                               modes_in_range, twopt_sink(false, true));
       const int key_ell = lm_zero ? -1 : p.ELL, key_m = lm_zero ? 0 : tm.M;
       if (key_ell != t_ell || key_m != t_m || Sbar != t_sbar) {
-        LoadTwopt<T, double> lt{dnLMp, N00.get(), ctx.tab,
-                             dmk(Sbar.real(), Sbar.imag()), 1. / g.vol};
+        LoadTwopt<T, double> lt{dnLMp, N00p, ctx.tab, dmk(Sbar.real(), Sbar.imag()),
+                                1. / g.vol, N_dc};
         fft3d<T>(ctx, tfield.get(), lt, +1, 2. * double(nm) * sizeof(double2));
         t_ell = key_ell;
         t_m = key_m;
@@ -1452,7 +1457,7 @@ Result run_3pcf(Context& ctx, const DeviceCatalogue& d,
   out.n1.resize(dim); out.n2.resize(dim);
   out.raw.assign(dim, 0.); out.shot.assign(dim, 0.);
 
-  DevArray<double2> dn00(nm), N00(nm);
+  DevArray<double2> dn00(nm), N00(survey ? nm : 0);
   if (win) {
     build_single_field_k(ctx, dn00.get(), d, alpha, 0, 0, false);
     build_single_field_k(ctx, N00.get(), d, alpha, 0, 0, true);
@@ -1460,8 +1465,10 @@ Result run_3pcf(Context& ctx, const DeviceCatalogue& d,
     build_survey_pair_k(ctx, dn00.get(), N00.get(), d, *r, alpha, 0, 0);
   } else {
     build_field_k<double>(ctx, dn00.get(), d, r, false, alpha, 0, 0, false, true);
-    build_field_k<double>(ctx, N00.get(), d, r, false, alpha, 0, 0, true, false);
   }
+  // N_00 of a box from dn_00, as in run_bispec_multi.
+  const double2* N00p = survey ? N00.get() : dn00.get();
+  const double N_dc = survey ? 0. : double(d.n);
 
   const Spline& sja = cached_spline(ctx.dev, p.ell1, ctx.stream);
   const Spline& sjb = cached_spline(ctx.dev, p.ell2, ctx.stream);
@@ -1495,8 +1502,8 @@ Result run_3pcf(Context& ctx, const DeviceCatalogue& d,
     const cplx Sbar = survey ? sbar.at({p.ELL, tm.M}) : cplx(double(d.n), 0.);
 
     // Shot noise first: defines r_eff and n_pairs (threept.cpp:1223-1367).
-    LoadTwopt<T, double> lt{dnLMp, N00.get(), ctx.tab, dmk(Sbar.real(), Sbar.imag()),
-                         1. / g.vol};
+    LoadTwopt<T, double> lt{dnLMp, N00p, ctx.tab, dmk(Sbar.real(), Sbar.imag()),
+                            1. / g.vol, N_dc};
     fft3d<T>(ctx, tfield.get(), lt, +1, 2. * double(nm) * sizeof(double2));
     ShotBins3pcf sb = shot_bins_3pcf<T>(ctx, tfield.get(), p.ell1, tm.m1, p.ell2,
                                         tm.m2, rb);

@@ -161,7 +161,7 @@ BinnedStat stats_fourier(Context& ctx, const double2* fa, const double2* fb, cpl
     hipLaunchKernelGGL(kern, dim3(grid), dim3(RED_THREADS),
                        twopt_smem(nb, 5, ctx.g), ctx.stream, fa, fb, ctx.g, ctx.tab,
                        dmk(sbar.real(), sbar.imag()), ell, m, map->view(), nb, cnt.get(),
-                       part.get());
+                       part.get(), 0.);
     TRVG_LAUNCH_CHECK();
   }
   reduce_cols(ctx, part.get(), int(grid), nb * 5, sum.get());

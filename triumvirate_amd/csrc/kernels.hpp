@@ -804,8 +804,8 @@ static __global__ void __launch_bounds__(RED_THREADS)
 k_twopt_fourier(const c2<T>* __restrict__ fa, const c2<T>* __restrict__ fb,
                 Geom g, AxisTables tab, double2 sbar, int ell, int m, TwoptMap map,
                 int nb, unsigned long long* __restrict__ counts,
-                double* __restrict__ part) {
-  k_twopt_fourier_body<T, NV, ILV>(fa, fb, g, tab, sbar, ell, m, map, nb, counts, part);
+                double* __restrict__ part, double fb_dc) {
+  k_twopt_fourier_body<T, NV, ILV>(fa, fb, g, tab, sbar, ell, m, map, nb, counts, part, fb_dc);
 }
 
 // ---------------------------------------------------------------------------
