@@ -52,3 +52,38 @@ def test_fp32_pair_sums_match_fp64(degrees, nb, ng):
     err = np.max(np.abs(out[0]['zeta_raw'] - out[1]['zeta_raw'])) / scale
     print(f"  {err:.2e}", flush=True)
     assert err < 4e-7 * ng ** 1.5
+
+
+@pytest.mark.parametrize('precision,eps', [('fp64', 4e-15), ('fp32', 4e-7)])
+@pytest.mark.parametrize('degrees', DEGREES, ids=lambda d: ''.join(map(str, d)))
+@pytest.mark.parametrize('form,idx', [('diag', 0), ('off-diag', 1), ('row', 2)])
+@pytest.mark.parametrize('nb,ng', [(4, 14), (9, 16), (17, 18)])
+def test_pair_lists_match_full_tables(degrees, precision, eps, form, idx, nb, ng):
+    """Lists of about one pair per field are streamed; the same pairs of the
+    full table come from the tiled kernels.  Batches of eight pairs: lists of
+    3 to 17, meshes with a remainder.  The fields are the same, the sums cancel
+    as above: eps sqrt(cells) of max |zeta| (eps ten roundings in FP64)."""
+    from triumvirate_amd import _lib
+    from triumvirate_amd import threept as T
+    from triumvirate_amd.dataobjs import Binning
+    print(f"pair lists {degrees} {precision} {form} bins {nb} mesh {ng}", flush=True)
+    be = T.CLibBackend(_lib.load())
+    ps = cf.make_test_paramset(assignment='cic', ngrid=dict.fromkeys('xyz', ng),
+                               boxsize=dict.fromkeys('xyz', 400.))
+    b = Binning('config', 'lin', bin_min=30., bin_max=180., num_bins=nb)
+    out = []
+    for f in (form, 'full'):
+        d, r = P.survey_pair(1500, 4000, 360., seed=9, weights=True)
+        out.append(T._compute_3pt_stats_survey_like(
+            be, '3pcf', d, r, paramset=ps, degrees=degrees, binning=b, form=f,
+            idx_bin=idx, precision=precision)['zeta_raw'])
+    if out[1].size == nb * nb:
+        full = out[1].reshape(nb, nb)
+    else:                      # equal degrees: only the upper triangle
+        full = np.full((nb, nb), np.nan, out[1].dtype)
+        full[np.triu_indices(nb)] = out[1]
+    want = {'diag': np.diag(full), 'off-diag': np.diag(full, idx), 'row': full[idx]}[form]
+    assert out[0].shape == want.shape
+    err = np.nanmax(np.abs(out[0] - want)) / np.nanmax(np.abs(full))
+    print(f"  {err:.2e}", flush=True)
+    assert err < eps * ng ** 1.5

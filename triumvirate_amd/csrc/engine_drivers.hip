@@ -571,8 +571,8 @@ static void pair_reduce_mfma(Context& ctx, const float2* FA, int na, const float
   });
 }
 
-// pair_reduce on the vector units (k_pair_lds): FP64 fields and two real
-// sides.
+// pair_reduce of a table on the vector units (k_pair_lds): FP64 fields and two
+// real sides.
 template <typename T>
 static void pair_reduce_lds(Context& ctx, const c2<T>* FA, int na, bool a_packed,
                             const c2<T>* FB, int nbf, bool b_packed, const c2<T>* G,
@@ -661,6 +661,63 @@ static void pair_reduce_lds(Context& ctx, const c2<T>* FA, int na, bool a_packed
   });
 }
 
+template <typename T, int MODE>
+static auto pair_list_kernel(int np) {
+  switch (np) {
+    case 2: return k_pair_list<T, MODE, 2>;
+    case 4: return k_pair_list<T, MODE, 4>;
+    case 6: return k_pair_list<T, MODE, 6>;
+    default: return k_pair_list<T, MODE, 8>;
+  }
+}
+
+// pair_reduce of a short list (k_pair_list; FP32 only with two real sides), in
+// equal batches of at most
+// eight pairs.
+template <typename T>
+static void pair_reduce_list(Context& ctx, const c2<T>* FA, bool a_packed, const c2<T>* FB,
+                             bool b_packed, const c2<T>* G, const std::vector<int2>& pairs,
+                             std::function<void(std::vector<cplx>&&)> sink) {
+  const long long nm = ctx.g.nmesh;
+  const int np = int(pairs.size());
+  const int batches = (np + 7) / 8;
+  // Even, so that the two fields of a packed mesh fall into one batch.
+  const int per = ((np + batches - 1) / batches + 1) / 2 * 2;
+  const int width = batches * per;
+  // Four blocks per CU in all: at eight the streams of a large mesh take 5 to
+  // 10 % longer.
+  const unsigned grid = unsigned(std::min<long long>(
+      (nm + 255) / 256, std::max(1, ctx.sm_count * 4 / batches)));
+  DevArray<int2> dl(np);
+  ctx.upload(dl.get(), pairs.data(), np);
+  DevArray<double2> part((size_t)grid * width), sum(width);
+  {
+    std::set<int> ma, mb;
+    for (const int2& q : pairs) {
+      ma.insert(a_packed ? q.x / 2 : q.x);
+      mb.insert(b_packed ? q.y / 2 : q.y);
+    }
+    ProfScope ps(ctx, KC_PAIR_REDUCE,
+                 double(ma.size() + mb.size() + batches) * double(nm) * sizeof(c2<T>));
+    auto kern = pair_list_kernel<T, 2>(per);
+    if constexpr (sizeof(T) == 8)
+      if (!a_packed) kern = b_packed ? pair_list_kernel<T, 1>(per) : pair_list_kernel<T, 0>(per);
+    hipLaunchKernelGGL(kern, dim3(batches, grid), dim3(256), 0, ctx.stream, FA, FB, G, nm,
+                       dl.get(), np, part.get());
+    TRVG_LAUNCH_CHECK();
+  }
+  reduce_cols(ctx, part.get(), int(grid), width, sum.get());
+  const double2* h = ctx.download(sum.get(), width);
+  ctx.keep_until_flush(std::move(dl));
+  ctx.keep_until_flush(std::move(part));
+  ctx.keep_until_flush(std::move(sum));
+  ctx.defer([h, np, sink = std::move(sink)]() {
+    std::vector<cplx> out(np);
+    for (int d = 0; d < np; d++) out[d] = cplx(h[d].x, h[d].y);
+    sink(std::move(out));
+  });
+}
+
 // S_p = sum_x F_a(x) F_b(x) G(x) for pairs p = (a, b) of logical fields,
 // handed to `sink` at the next ctx.flush() (the launches are only queued).
 // A side / B side packed: real fields stored two per complex mesh (logical
@@ -686,7 +743,14 @@ static void pair_reduce(Context& ctx, const c2<T>* FA, int na, bool a_packed,
       return;
     }
   }
-  pair_reduce_lds<T>(ctx, FA, na, a_packed, FB, nbf, b_packed, G, pairs, std::move(sink));
+  // Lists with about one pair per field (diagonal, off-diagonal, row) are
+  // streamed: they read no mesh twice.  Fuller tables reuse staged rows (the
+  // 16 x 16 tables of FP32 complex sides above are at the memory rate for
+  // lists too: 20 diagonal pairs at 256^3 307 us there, 347 us streamed).
+  if (!pairs.empty() && int(pairs.size()) <= na + nbf)
+    pair_reduce_list<T>(ctx, FA, a_packed, FB, b_packed, G, pairs, std::move(sink));
+  else
+    pair_reduce_lds<T>(ctx, FA, na, a_packed, FB, nbf, b_packed, G, pairs, std::move(sink));
 }
 
 struct TwoPt {
