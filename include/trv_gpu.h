@@ -384,6 +384,14 @@ int trvg_compute_bispec_multi_observer(const trvg_catalogue* data,
                                        const double* norm_factors,
                                        trvg_bispec_result* outs);
 
+/* out[i] = (in[i] + add) - sub for i < n (n >= 1), then modulo `period` (the
+ * result in [0, period)) when period > 0 and some value is outside, on the
+ * host worker threads: the coordinate shifts of the box drivers.
+ * extremes[2] receives the least and the greatest result (NaN if there is
+ * one).  Needs no device. */
+int trvg_host_shift(const double* in, double* out, long long n, double add,
+                    double sub, double period, double* extremes);
+
 /* Frees the cached device work buffers (they are otherwise kept for reuse
  * by later calls). */
 int trvg_release_workspace(void);

@@ -216,3 +216,82 @@ def test_unit_weight_columns_are_not_passed_to_the_engine():
     assert c.engine_columns()[4] is None
     d = ParticleCatalogue(x, x, x, nz=1., wc=np.ones(8))
     assert d.engine_columns()[5] is not None   # arrays are passed as given
+
+
+@pytest.mark.parametrize('n', [1, 65535, 65536, 70001])
+def test_catalogue_shifts_match_numpy(n):
+    """Coordinate shifts on the engine's host threads (from 65536 particles)
+    are the numpy expressions bit by bit: values inside and outside the box,
+    at its edges, a NaN, and columns changed in place since construction."""
+    from triumvirate_amd import _lib
+    from triumvirate_amd.catalogue import ParticleCatalogue
+    _lib.load()
+    rng = np.random.default_rng(n)
+    L = [700., 1000., 1300.]
+    for spread, nan in ((1., False), (2.5, False), (1., True)):
+        pos = [rng.uniform(-0.5, 0.5, n) * spread * b + 37. for b in L]
+        pos[0][-1] = pos[0][0]
+        cat = ParticleCatalogue(*pos, nz=1.)
+        if nan:
+            cat['y'][n // 2] = np.nan         # in place: bounds stay as they were
+            pos[1][n // 2] = np.nan
+        want = {}
+        for ax, p, b in zip('xyz', pos, L):
+            lo, hi = cat.bounds[ax]
+            want[ax] = (p + b / 2. - (hi + lo) / 2.) % b
+        other = cat.shallow_copy()
+        cat.periodise(L)
+        for ax, p in zip('xyz', pos):
+            assert np.array_equal(cat[ax], want[ax], equal_nan=True)
+            assert np.array_equal(cat.bounds[ax], (want[ax].min(), want[ax].max()),
+                                  equal_nan=True)
+            assert np.array_equal(other[ax], p, equal_nan=True)
+        cat.offset_coords([1.5, -2., 0.])
+        for ax, o in zip('xyz', (1.5, -2., 0.)):
+            assert np.array_equal(cat[ax], want[ax] - o, equal_nan=True)
+
+
+@pytest.mark.parametrize('term', [1., 3., 0.1, 1. / 3., 1. + 2. ** -52, 1.5 - 2. ** -52,
+                                  2. ** 40 + 1., 6.02e-4 ** 2])
+@pytest.mark.parametrize('n', [1, 2, 70000, 1000003])
+def test_equal_terms_sum_in_catalogue_order(n, term):
+    """Sums of equal terms bit by bit as the additions in catalogue order
+    (terms with few and many bits, ties between two roundings)."""
+    from triumvirate_amd import _lib
+    from triumvirate_amd import threept as T
+    from triumvirate_amd.catalogue import ParticleCatalogue
+    from triumvirate_amd._abi import CatalogueView
+    be = T.CLibBackend(_lib.load())
+    x = np.linspace(0., 1., n)
+    cat = ParticleCatalogue(x, x, x, nz=1., ws=term)
+    want = np.add.accumulate(np.full(n, term))[-1]
+    assert be.norm_particles(CatalogueView(*cat.columns()), 1.) == 1. / want
+
+
+def test_host_sums_and_forked_process():
+    """Normalisation sums over worker threads against numpy (rounding of 7e4
+    terms: 1e-12), and the same sums in a forked process, which has no
+    worker threads."""
+    import multiprocessing as mp
+    from triumvirate_amd import _lib
+    from triumvirate_amd import threept as T
+    from triumvirate_amd.catalogue import ParticleCatalogue
+    from triumvirate_amd._abi import CatalogueView
+    be = T.CLibBackend(_lib.load())
+    rng = np.random.default_rng(5)
+    n = 70001
+    nz, ws, wc = rng.uniform(0.5, 1.5, (3, n))
+    cat = ParticleCatalogue(*rng.uniform(0., 100., (3, n)), nz=nz, ws=ws, wc=wc)
+
+    def norm():
+        return be.norm_particles(CatalogueView(*cat.columns()), 0.5)
+
+    want = 1. / (0.5 * np.sum(ws * nz ** 2 * wc ** 3))
+    assert abs(norm() / want - 1.) < 1e-12
+    ctx = mp.get_context('fork')
+    q = ctx.SimpleQueue()
+    p = ctx.Process(target=lambda: q.put(norm()))
+    p.start()
+    p.join(60)
+    assert p.exitcode == 0
+    assert abs(q.get() / want - 1.) < 1e-12

@@ -290,6 +290,9 @@ def declare_extensions(lib):
     lib.trvg_compute_3pcf_dev.argtypes = [vp, vp, P(Params), P(Binning),
                                           C.c_double, P(ThreePCFResult)]
     lib.trvg_compute_3pcf_dev.restype = C.c_int
+    lib.trvg_host_shift.argtypes = [_dp, _dp, C.c_longlong, C.c_double,
+                                    C.c_double, C.c_double, _dp]
+    lib.trvg_host_shift.restype = C.c_int
     lib.trvg_release_workspace.argtypes = []
     lib.trvg_release_workspace.restype = C.c_int
     lib.trvg_mesh_assign.argtypes = [P(Catalogue), _dp, P(Params), C.c_int,

@@ -42,3 +42,8 @@ def load():
             raise ImportError("libtrvgpu.so ABI version mismatch.")
         _lib = lib
         return lib
+
+
+def loaded():
+    """The handle if :func:`load` has succeeded, else None."""
+    return _lib

@@ -2,6 +2,7 @@
 //
 // Every entry point converts C++ exceptions into a status code plus a
 // thread-local message (trvg_last_error); HIP failures are never ignored.
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -189,19 +190,60 @@ void write_2pcf(const TwoPtResult& r, trvg_2pcf_result* out) {
   out->dim = nb;
 }
 
-// sum_p f(ws_p, wc_p, nz_p) over a host catalogue.
+// 0 + t + t + ... (n times, t > 0), every addition rounded.  Within a binade of
+// s each addition adds the same multiple of its ulp, except where t lies half
+// way between two multiples (then step by step).
+double repeated_sum(double t, long long n) {
+  double s = 0.;
+  while (n > 0) {
+    const double s1 = s + t, d = s1 - s;
+    const double top = std::ldexp(1., std::ilogb(s1) + 1);
+    const double ulp = top * 0x1p-53;
+    long long k = 1;
+    if (s >= t && s >= 0.5 * top && 2. * std::fabs(t - d) != ulp) {
+      if (d == 0.) return s;
+      const double room = std::floor((top - s) / d) - 1.;
+      k = room >= 1. ? std::min(n, (long long)(std::min(room, 0x1p53))) : 1;
+    }
+    s = k == 1 ? s1 : s + double(k) * d;
+    n -= k;
+  }
+  return s;
+}
+
+// sum_p f(ws_p, wc_p, nz_p) over a host catalogue: one partial sum per
+// worker thread, added in their order.  Equal terms (uniform density, unit
+// weights), whose rounding errors add up instead of cancelling, give the sum
+// in catalogue order.
 template <class F>
 double particle_sum(const trvg_catalogue* c, F f) {
   if (c == nullptr || c->x == nullptr)
     throw Error(TRVG_ERR_DATA, "Particle data are uninitialised.");
   const long long st = c->stride > 0 ? c->stride : 1;
+  auto term = [&](long long i) {
+    return f(c->ws ? c->ws[i * st] : 1., c->wc ? c->wc[i * st] : 1.,
+             c->nz ? c->nz[i * st] : 0.);
+  };
+  if (c->ntotal < 1) return 0.;
+  const double t0 = term(0);
+  std::vector<double> part(host_threads(), 0.);
+  std::vector<char> equal(host_threads(), 1);
+  host_ranges(c->ntotal, [&](long long b, long long e, int t) {
+    double s = 0.;
+    bool eq = true;
+    for (long long i = b; i < e; i++) {
+      const double v = term(i);
+      s += v;
+      eq &= v == t0;
+    }
+    part[t] = s;
+    equal[t] = eq;
+  });
+  if (std::count(equal.begin(), equal.end(), 0) == 0 && t0 > 0. && std::isnormal(t0) &&
+      t0 < 1e300)
+    return repeated_sum(t0, c->ntotal);
   double s = 0.;
-  for (long long i = 0; i < c->ntotal; i++) {
-    const double ws = c->ws ? c->ws[i * st] : 1.;
-    const double wc = c->wc ? c->wc[i * st] : 1.;
-    const double nz = c->nz ? c->nz[i * st] : 0.;
-    s += f(ws, wc, nz);
-  }
+  for (double v : part) s += v;
   return s;
 }
 
@@ -254,19 +296,54 @@ int trvg_result_dim(int shape, int num_bins, int idx_bin, int* dim) {
   return guarded([&] { *dim = result_dim(shape, num_bins, idx_bin); });
 }
 
+int trvg_host_shift(const double* in, double* out, long long n, double add, double sub,
+                    double period, double* extremes) {
+  return guarded([&] {
+    if (n < 1 || in == nullptr || out == nullptr || extremes == nullptr)
+      throw Error(TRVG_ERR_PARAM, "Column to shift is missing.");
+    std::vector<double> lo(host_threads(), HUGE_VAL), hi(host_threads(), -HUGE_VAL);
+    // f of every value, and the extremes of the results (NaN if one is).
+    auto pass = [&](auto f) {
+      host_ranges(n, [&](long long b, long long e, int t) {
+        double l = HUGE_VAL, h = -HUGE_VAL;
+        bool nan = false;
+        for (long long i = b; i < e; i++) {
+          const double v = f(i);
+          out[i] = v;
+          l = v < l ? v : l;
+          h = v > h ? v : h;
+          nan |= v != v;
+        }
+        lo[t] = nan ? NAN : l;
+        hi[t] = nan ? NAN : h;
+      });
+      double l = HUGE_VAL, h = -HUGE_VAL;
+      bool nan = false;
+      for (size_t t = 0; t < lo.size(); t++) {
+        nan |= lo[t] != lo[t];
+        l = std::min(l, lo[t]);
+        h = std::max(h, hi[t]);
+      }
+      extremes[0] = nan ? NAN : l;
+      extremes[1] = nan ? NAN : h;
+    };
+    pass([=](long long i) { return (in[i] + add) - sub; });
+    if (period > 0. && !(extremes[0] >= 0. && extremes[1] < period))
+      pass([=](long long i) {
+        // As Python's % on floats: the result takes the period's sign.
+        double r = std::fmod(out[i], period);
+        if (r < 0.) r += period;
+        return r == 0. ? 0. : r;
+      });
+  });
+}
+
 int trvg_calc_bispec_normalisation_from_particles(
     const trvg_catalogue* c, double alpha, double* norm_factor) {
   return guarded([&] {
-    if (c == nullptr || c->x == nullptr)
-      throw Error(TRVG_ERR_DATA, "Particle data are uninitialised.");
-    const long long st = c->stride > 0 ? c->stride : 1;
-    double s = 0.;
-    for (long long i = 0; i < c->ntotal; i++) {
-      double ws = c->ws ? c->ws[i * st] : 1.;
-      double wc = c->wc ? c->wc[i * st] : 1.;
-      double nz = c->nz ? c->nz[i * st] : 0.;
-      s += ws * std::pow(nz, 2) * std::pow(wc, 3);
-    }
+    const double s = particle_sum(c, [](double ws, double wc, double nz) {
+      return ws * std::pow(nz, 2) * std::pow(wc, 3);
+    });
     if (s == 0.)
       throw Error(TRVG_ERR_DATA,
                   "Particle 'nz' values appear to be all zeros. "

@@ -162,6 +162,11 @@ void upload_catalogue(const trvg_catalogue* c, const double* los,
                       Context* sort_for = nullptr, bool los32 = false,
                       const double* observer = nullptr, bool fixed_pos = false);
 
+// Host worker threads (upload.hip): fn(begin, end, part) over [0, n) in
+// contiguous parts, one per thread; returns the number of parts.
+int host_threads();
+int host_ranges(long long n, const std::function<void(long long, long long, int)>& fn);
+
 // ---------------------------------------------------------------------------
 // Spherical Bessel spline (host build, device tables).
 // ---------------------------------------------------------------------------

@@ -12,6 +12,8 @@
 // ws * wc is not transferred: the device fills it.  The host returns once
 // every chunk is gathered; the copies complete in stream order before the
 // kernels that read them.
+#include <unistd.h>
+
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
@@ -48,6 +50,8 @@ class HostWorkers {
     return *w;
   }
   int size() const { return nthreads_; }
+  // False in a process forked since: the threads stayed with the parent.
+  bool alive() const { return getpid() == pid_; }
 
   void run(const std::function<void(int)>& fn) {
     std::lock_guard<std::mutex> serial(run_mu_);
@@ -69,7 +73,7 @@ class HostWorkers {
   }
 
  private:
-  explicit HostWorkers(int n) : nthreads_(n) {
+  explicit HostWorkers(int n) : nthreads_(n), pid_(getpid()) {
     for (int t = 1; t < n; t++) {
       std::thread th([this, t] { loop(t); });
       th.detach();   // lives for the process
@@ -94,12 +98,36 @@ class HostWorkers {
   }
 
   int nthreads_;
+  pid_t pid_;
   std::mutex run_mu_, mu_;
   std::condition_variable cv_, done_cv_;
   const std::function<void(int)>* job_ = nullptr;
   long gen_ = 0;
   int pending_ = 0;
 };
+
+}  // namespace
+
+int host_threads() { return HostWorkers::get().size(); }
+
+// fn(begin, end, part) over [0, n) in host_threads() contiguous parts on the
+// worker threads; in one part for short ranges (below 65536 items a serial
+// loop takes less than waking the threads) and in a forked process.
+int host_ranges(long long n, const std::function<void(long long, long long, int)>& fn) {
+  HostWorkers& w = HostWorkers::get();
+  const int parts = n < (1 << 16) || !w.alive() ? 1 : w.size();
+  if (parts == 1) {
+    fn(0, n, 0);
+    return 1;
+  }
+  w.run([&](int t) {
+    const long long b = n * t / parts, e = n * (t + 1) / parts;
+    if (e > b) fn(b, e, t);
+  });
+  return parts;
+}
+
+namespace {
 
 // ---------------------------------------------------------------------------
 // Page-locked staging ring (one per stream: a stream serves one call at a

@@ -421,7 +421,8 @@ def _compute_3pt_stats_sim_like(backend, kind, catalogue_data, paramset=None,
 
     boxsize = [paramset['boxsize'][a] for a in 'xyz']
     catalogue_data.periodise(boxsize)
-    if not catalogue_data['nz'].any():
+    nz = catalogue_data['nz']
+    if not (nz[:1].any() or nz.any()):
         catalogue_data.compute_mean_density(boxsize=boxsize)
 
     data_v = _view(catalogue_data)

@@ -166,12 +166,7 @@ def _mesh_mixed_norm(backend, catalogue_data, catalogue_rand, paramset, alpha):
     n = int(math.ceil(L / CELLSIZE))
     n += n % 2
     L = n * CELLSIZE
-    d = ParticleCatalogue(*catalogue_data.columns()[:3],
-                          nz=catalogue_data['nz'], ws=catalogue_data['ws'],
-                          wc=catalogue_data['wc'])
-    r = ParticleCatalogue(*catalogue_rand.columns()[:3],
-                          nz=catalogue_rand['nz'], ws=catalogue_rand['ws'],
-                          wc=catalogue_rand['wc'])
+    d, r = catalogue_data.shallow_copy(), catalogue_rand.shallow_copy()
     if paramset['alignment'] == 'pad':
         if paramset['padscale'] == 'grid':
             d.pad([L] * 3, ngrid=[n] * 3, ngrid_pad=paramset['padfactor'],
@@ -268,7 +263,8 @@ def _compute_2pt_stats_sim_like(backend, kind, catalogue_data, paramset=None,
     _prepare_box(paramset, catalogue_data)
     boxsize = [paramset['boxsize'][a] for a in 'xyz']
     catalogue_data.periodise(boxsize)
-    if not catalogue_data['nz'].any():
+    nz = catalogue_data['nz']
+    if not (nz[:1].any() or nz.any()):
         catalogue_data.compute_mean_density(boxsize=boxsize)
     data_v = _view(catalogue_data)
     params = _params_struct(paramset)
