@@ -67,6 +67,39 @@ def test_fft3d_general_sizes(eng, shape, prec):
         assert err < tol, (sign, err)
 
 
+@pytest.mark.parametrize('shape', [(14, 42, 70), (126, 14, 22), (50, 98, 34),
+                                   (250, 10, 14), (18, 162, 28), (14, 10, 686)])
+@pytest.mark.parametrize('prec,bound', [(64, 16.5 * 2. ** -53), (32, 8. * 2. ** -24)])
+def test_fft3d_mixed_radices(eng, shape, prec, bound):
+    """Register butterflies of radix 2 to 7 in every order, powers of odd
+    radices, the direct form (11, 17), last blocks of fewer lines.  Error in
+    the rms, over at most 16 stages of the three axes.  FP32: one to two
+    roundings a stage, 2 sqrt(16) = 8 eps.  FP64: also the twiddles, cosines of
+    angles 2 pi k / n that are themselves rounded (2 pi eps at most, 2 pi /
+    sqrt(3) = 3.6 eps rms): sqrt(16 (3.6^2 + 2^2)) = 16.5 eps."""
+    from triumvirate_amd import _abi
+    print(f"fft3d mixed shape={shape} prec={prec}", flush=True)
+    g = np.random.default_rng(12)
+    a = g.normal(size=shape) + 1j * g.normal(size=shape)
+    if prec == 32:
+        a = a.astype(np.complex64).astype(complex)
+    p = _abi.Params()
+    for i in range(3):
+        p.boxsize[i] = 1.
+        p.ngrid[i] = shape[i]
+    p.assignment_order = 3
+    p.precision = prec
+    p.device = -1
+    for sign, ref in ((-1, np.fft.fftn(a)), (+1, np.fft.ifftn(a) * a.size)):
+        buf = np.ascontiguousarray(a).view(np.float64).copy()
+        assert eng.trvg_fft3d(C.byref(p), _abi.dptr(buf), sign) == 0, \
+            eng.trvg_last_error()
+        out = buf.view(np.complex128).reshape(shape)
+        err = np.sqrt(np.mean(np.abs(out - ref) ** 2) / np.mean(np.abs(ref) ** 2))
+        print(f"  {sign:+d} {err:.2e}", flush=True)
+        assert err < bound, (sign, err)
+
+
 CASES = [
     # (kind, degrees, form, geometry, scheme, ngrid)
     ('bispec', (0, 0, 0), 'full', 'gpp', 'tsc', (24, 24, 24)),
