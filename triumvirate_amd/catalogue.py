@@ -23,8 +23,9 @@ from . import _abi, _lib
 def _shifted(a, add, sub, period=0.):
     """``(a + add) - sub``, modulo `period` if positive, as a new array, and
     its extremes.  Long columns go through the engine's host threads once
-    the engine is loaded (8e6 particles, three axes: 90 ms in numpy, most
-    of it the modulo, 8 ms there; a shorter column costs more to hand over).
+    the engine is loaded (1e6 values with modulo, eight threads: 14.5 ms in
+    numpy, 0.47 ms there; at 65536 threads and a serial loop take the same
+    0.15 ms).
     The modulo is left out where it changes nothing (every value already in
     [0, period))."""
     lib = _lib.loaded()
