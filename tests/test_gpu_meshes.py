@@ -3,8 +3,9 @@ reference plans FFTW for any size (field.cpp:246-339) and its drivers derive
 even meshes from the Nyquist cutoff (parameters.cpp:1434-1463).
 
 * 3-D transforms against numpy.fft (FFTW convention): 1e-12 (FP64),
-  2e-6 (FP32) of max |X|, for radices 2, 3, 5, 13, 53 and a 2048-point
-  axis (one line per workgroup).
+  2e-6 (FP32) of max |X|, for radices 2, 3, 5, 13, 53, a 2048-point
+  axis (one line per workgroup) and the longest power-of-two passes (512,
+  1024: the most LDS a workgroup takes).
 * Estimators against the oracle (whose transform takes a direct DFT for
   such sizes) at 1e-10: box and survey bispectra, 3PCFs, power spectrum
   with interlacing, correlation function and window; FP32 within 1e-5 of
@@ -43,7 +44,9 @@ def oracle_backend():
 
 
 @pytest.mark.parametrize('shape', [(12, 18, 30), (96, 8, 10), (8, 106, 8),
-                                   (24, 40, 26), (10, 8, 2048), (2048, 8, 10)])
+                                   (24, 40, 26), (10, 8, 2048), (2048, 8, 10),
+                                   (1024, 8, 8), (8, 1024, 8), (8, 8, 1024),
+                                   (512, 8, 8), (8, 512, 8)])
 @pytest.mark.parametrize('prec', [64, 32])
 def test_fft3d_general_sizes(eng, shape, prec):
     from triumvirate_amd import _abi
@@ -106,6 +109,8 @@ CASES = [
     ('bispec', (2, 0, 2), 'diag', 'lpp', 'pcs', (30, 40, 48)),
     ('3pcf', (1, 1, 0), 'full', 'lpp', 'cic', (30, 30, 30)),
     ('3pcf', (0, 0, 0), 'diag', 'gpp', 'tsc', (26, 26, 26)),
+    ('3pcf', (1, 1, 0), 'diag', 'lpp', 'cic', (1024, 8, 8)),   # j_l x pass
+    ('bispec', (0, 0, 0), 'diag', 'gpp', 'tsc', (8, 1024, 8)),
 ]
 
 

@@ -193,7 +193,8 @@ constexpr int fft_line_stride(int n, int nl) {
 }
 
 // Twiddles in LDS, per stage (span Ns, radix R) the (R - 1) Ns factors
-// w^{q k N / (Ns R)}, k fastest: N - 8 of them at most.  tw: e^{sign 2 pi i m / N}.
+// w^{q k N / (Ns R)}, k fastest: N - 2^LR of them (the spans add up so).  tw:
+// e^{sign 2 pi i m / N}.
 template <typename T, int LOGN, int LR = FFT_LR, int LD = LR>
 __device__ __forceinline__ void fft_fill_twiddles(c2<T>* W, const c2<T>* __restrict__ tw,
                                                   int t, int nt) {
@@ -256,31 +257,50 @@ __device__ __forceinline__ void fft_stages(c2<T> (&v)[8], c2<T>* lb, const c2<T>
   }
 }
 
+// LDS of a workgroup: nl lines (stride `ls`) and the twiddles of its stages,
+// n minus the first radix of them at most.
+constexpr size_t FFT_LDS = 160 * 1024;
+template <typename T>
+constexpr size_t fft_lds(int n, int nl, int ls) {
+  return size_t(nl * ls + n - (1 << FFT_LR)) * sizeof(c2<T>);
+}
+template <typename T>
+constexpr size_t strided_lds(int logn, int nt) {
+  const int nl = nt * 8 >> logn;
+  return fft_lds<T>(1 << logn, nl, fft_line_stride<T>(1 << logn, nl));
+}
+
 // Threads of a workgroup of the strided passes: rows of `bytes` contiguous
 // bytes (several lines of neighbouring columns), within 256..1024 threads.
 // From 512 points on 256 threads would hold rows of 32 bytes, half a sector
 // of HBM; up to 256 points rows of 64 bytes measured no slower than 128, and
-// the smaller blocks prune better.
+// the smaller blocks prune better.  Eight FP64 lines of 1024 points do not
+// fit LDS: rows of 64 bytes there (x pass of 1024 x 512 x 256: 2.06 ms; rows
+// of 32 bytes 2.20).
 template <typename T, int LOGN>
 constexpr int strided_threads() {
   const int bytes = LOGN >= 9 ? 128 : 64;
-  const int nt = bytes / int(sizeof(c2<T>)) * ((1 << LOGN) / 8);
-  return nt < 256 ? 256 : (nt > 1024 ? 1024 : nt);
+  int nt = bytes / int(sizeof(c2<T>)) * ((1 << LOGN) / 8);
+  nt = nt < 256 ? 256 : (nt > 1024 ? 1024 : nt);
+  while (strided_lds<T>(LOGN, nt) > FFT_LDS) nt /= 2;
+  return nt;
 }
 template <typename T, int LOGN>
 constexpr int strided_lines() { return strided_threads<T, LOGN>() * 8 >> LOGN; }
 template <typename T, int LOGN>
 constexpr size_t strided_smem() {
-  return size_t(strided_lines<T, LOGN>() *
-                    fft_line_stride<T>(1 << LOGN, strided_lines<T, LOGN>()) +
-                (1 << LOGN)) * sizeof(c2<T>);
+  constexpr size_t bytes = strided_lds<T>(LOGN, strided_threads<T, LOGN>());
+  static_assert(bytes <= FFT_LDS, "lines of a strided workgroup exceed LDS");
+  return bytes;
 }
 // Lines of a workgroup of the z pass (256 threads).
 constexpr int z_lines(int n) { return FFT_THREADS * 8 / n; }
 template <typename T, int LOGN>
 constexpr size_t z_smem() {
-  return size_t(z_lines(1 << LOGN) * fft_line_stride<T>(1 << LOGN, 1) + (1 << LOGN)) *
-         sizeof(c2<T>);
+  constexpr int N = 1 << LOGN;
+  constexpr size_t bytes = fft_lds<T>(N, z_lines(N), fft_line_stride<T>(N, 1));
+  static_assert(bytes <= FFT_LDS, "lines of a z workgroup exceed LDS");
+  return bytes;
 }
 
 // Loaders that read several fields or evaluate harmonics per cell.
