@@ -11,6 +11,7 @@
 #include "batch_kernels.hpp"
 #include "diff_kernels.hpp"
 #include "engine.hpp"
+#include "prune_lists.hpp"
 
 namespace trvg {
 
@@ -196,16 +197,8 @@ static void launch_strided_batch_gen(Context& ctx, c2<T>* base, int N, long long
 // over only the blocks whose lines lie in each bin's band.
 // ---------------------------------------------------------------------------
 
-// Blocks of the z and y passes holding a line inside a pruning radius, for
-// one geometry (computed once per radius).  The host predicate carries a
-// relative margin over the kernels' exactly rounded one, so every block the
-// kernels would use is listed (a listed block with no needed line only
-// writes zeros that no later pass reads).
-struct PruneLists {
-  std::vector<int> zblocks, yblocks;
-  double d_lines = 0., slabs = 0.;   // needed z lines and y slabs
-};
-
+// Work lists of one geometry, pass shape and radius (prune_lists.hpp), built
+// once.
 static const PruneLists& prune_lists(const Geom& g, double kcut2, int nl_z,
                                      int nl_y) {
   static std::mutex mu;
@@ -215,31 +208,7 @@ static const PruneLists& prune_lists(const Geom& g, double kcut2, int nl_z,
   std::lock_guard<std::mutex> lk(mu);
   auto it = cache.find(key);
   if (it != cache.end()) return *it->second;
-  auto pl = std::make_unique<PruneLists>();
-  const double kc = kcut2 * (1. + 1.e-12);
-  std::vector<char> slab_in(g.n[0]), line_in((size_t)g.n[0] * g.n[1]);
-  for (int i = 0; i < g.n[0]; i++) {
-    const double kx = shifted(i, g.n[0]) * g.dk[0];
-    slab_in[i] = kx * kx < kc;
-    pl->slabs += (kx * kx < kcut2);
-    for (int j = 0; j < g.n[1]; j++) {
-      const double ky = shifted(j, g.n[1]) * g.dk[1];
-      line_in[(size_t)i * g.n[1] + j] = kx * kx + ky * ky < kc;
-      pl->d_lines += (kx * kx + ky * ky < kcut2);
-    }
-  }
-  const long long nlines = (long long)g.n[0] * g.n[1];
-  for (long long b = 0; b * nl_z < nlines; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_z && !any; l++) any = line_in[b * nl_z + l];
-    if (any) pl->zblocks.push_back(int(b));
-  }
-  const long long ylines = (long long)g.n[0] * g.n[2];   // (i, k) lines
-  for (long long b = 0; b * nl_y < ylines; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_y && !any; l++) any = slab_in[(b * nl_y + l) / g.n[2]];
-    if (any) pl->yblocks.push_back(int(b));
-  }
+  auto pl = std::make_unique<PruneLists>(make_prune_lists(g.n, g.dk, kcut2, nl_z, nl_y));
   return *(cache[key] = std::move(pl));
 }
 
@@ -393,11 +362,6 @@ static Prune prune_zy(const Geom& g) {
   return pr;
 }
 
-struct PruneListsXF {
-  std::vector<int> xblocks, yblocks;
-  double x_lines = 0., y_lines = 0.;   // needed x lines, written y lines
-};
-
 static const PruneListsXF& prune_lists_xfirst(const Geom& g, double kcut2, int nl_x,
                                               int nl_y) {
   static std::mutex mu;
@@ -407,34 +371,8 @@ static const PruneListsXF& prune_lists_xfirst(const Geom& g, double kcut2, int n
   std::lock_guard<std::mutex> lk(mu);
   auto it = cache.find(key);
   if (it != cache.end()) return *it->second;
-  auto pl = std::make_unique<PruneListsXF>();
-  const double kc = kcut2 * (1. + 1.e-12);
-  const int n1 = g.n[1], n2 = g.n[2];
-  std::vector<char> kz_in(n2), line_in((size_t)n1 * n2);
-  double nkz = 0.;
-  for (int k = 0; k < n2; k++) {
-    const double kz = shifted(k, n2) * g.dk[2];
-    kz_in[k] = kz * kz < kc;
-    nkz += (kz * kz < kcut2);
-    for (int j = 0; j < n1; j++) {
-      const double ky = shifted(j, n1) * g.dk[1];
-      line_in[(size_t)j * n2 + k] = kz * kz + ky * ky < kc;
-      pl->x_lines += (kz * kz + ky * ky < kcut2);
-    }
-  }
-  pl->y_lines = nkz * g.n[0];
-  const long long xl = (long long)n1 * n2;
-  for (long long b = 0; b * nl_x < xl; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_x && !any; l++) any = line_in[b * nl_x + l];
-    if (any) pl->xblocks.push_back(int(b));
-  }
-  const long long yl = (long long)g.n[0] * n2;
-  for (long long b = 0; b * nl_y < yl; b++) {
-    bool any = false;
-    for (int l = 0; l < nl_y && !any; l++) any = kz_in[(b * nl_y + l) % n2];
-    if (any) pl->yblocks.push_back(int(b));
-  }
+  auto pl =
+      std::make_unique<PruneListsXF>(make_prune_lists_xfirst(g.n, g.dk, kcut2, nl_x, nl_y));
   return *(cache[key] = std::move(pl));
 }
 
