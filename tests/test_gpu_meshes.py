@@ -103,6 +103,34 @@ def test_fft3d_mixed_radices(eng, shape, prec, bound):
         assert err < bound, (sign, err)
 
 
+@pytest.mark.parametrize('shape', [(96, 96, 96), (90, 126, 70), (200, 48, 50),
+                                   (98, 54, 250)])
+def test_fft3d_fp32_scale(eng, shape):
+    """FP32 lines of mixed length carry no rounded constants: the factor
+    between the transform and numpy's is 1 to a tenth of eps = 2^-24 (rounding
+    of 1.2e5 cells and more averages to 0.01 eps; a constant rounded to FP32 is
+    off by up to eps / 2 and scales every mode)."""
+    from triumvirate_amd import _abi
+    print(f"fft3d scale shape={shape}", flush=True)
+    g = np.random.default_rng(3)
+    a = (g.normal(size=shape) + 1j * g.normal(size=shape)).astype(np.complex64)
+    a = a.astype(complex)
+    p = _abi.Params()
+    for i in range(3):
+        p.boxsize[i] = 1.
+        p.ngrid[i] = shape[i]
+    p.assignment_order = 3
+    p.precision = 32
+    p.device = -1
+    buf = a.view(np.float64).copy()
+    assert eng.trvg_fft3d(C.byref(p), _abi.dptr(buf), -1) == 0, \
+        eng.trvg_last_error()
+    out, ref = buf.view(np.complex128).reshape(shape), np.fft.fftn(a)
+    scale = np.vdot(ref, out).real / np.vdot(ref, ref).real - 1.
+    print(f"  {scale:.2e}", flush=True)
+    assert abs(scale) < 0.1 * 2. ** -24
+
+
 CASES = [
     # (kind, degrees, form, geometry, scheme, ngrid)
     ('bispec', (0, 0, 0), 'full', 'gpp', 'tsc', (24, 24, 24)),

@@ -126,6 +126,13 @@ static int lines_strided(int n) {
 }
 static long long blocks_of(long long nlines, int nl) { return (nlines + nl - 1) / nl; }
 
+// Twiddles of a mixed-radix pass: FP64 but where outputs are formed directly.
+template <typename T>
+static const void* gen_twiddles(const Context& ctx, const GenPlan& P, int sign) {
+  if (P.direct) return ctx_twiddles<T>(ctx, P.n, sign);
+  return ctx_twiddles<double>(ctx, P.n, sign);
+}
+
 template <typename T, class Loader>
 static void launch_z_gen(Context& ctx, c2<T>* data, const Loader& load, int sign,
                          double bytes, const Prune& pr) {
@@ -137,7 +144,7 @@ static void launch_z_gen(Context& ctx, c2<T>* data, const Loader& load, int sign
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(blocks_of(nlines, P.nl))), dim3(FFT_THREADS), smem,
-                     ctx.stream, data, load, ctx_twiddles<T>(ctx, N, sign), ctx.g.n[1],
+                     ctx.stream, data, load, gen_twiddles<T>(ctx, P, sign), ctx.g.n[1],
                      nlines, sign, pr, P);
   TRVG_LAUNCH_CHECK();
 }
@@ -153,7 +160,7 @@ static void launch_strided_gen(Context& ctx, c2<T>* data, int N, long long S,
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(blocks_of(nlines, P.nl))), dim3(FFT_THREADS), smem,
-                     ctx.stream, data, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
+                     ctx.stream, data, gen_twiddles<T>(ctx, P, sign), S, outer_stride, inner,
                      nlines, sign, pr, prune_mode, P);
   TRVG_LAUNCH_CHECK();
 }
@@ -170,7 +177,7 @@ static void launch_z_batch_gen(Context& ctx, c2<T>* base, const BatchLoader& loa
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_Z64 : KC_FFT_Z, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                     ctx.g.nmesh, load, ctx_twiddles<T>(ctx, N, sign), ctx.g.n[1], nlines,
+                     ctx.g.nmesh, load, gen_twiddles<T>(ctx, P, sign), ctx.g.n[1], nlines,
                      sign, pr, kcut2, work, P);
   TRVG_LAUNCH_CHECK();
 }
@@ -187,7 +194,7 @@ static void launch_strided_batch_gen(Context& ctx, c2<T>* base, int N, long long
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                     ctx.g.nmesh, ctx_twiddles<T>(ctx, N, sign), S, outer_stride, inner,
+                     ctx.g.nmesh, gen_twiddles<T>(ctx, P, sign), S, outer_stride, inner,
                      nlines, sign, pr, kcut2, work, prune_mode, P);
   TRVG_LAUNCH_CHECK();
 }
@@ -401,7 +408,7 @@ static void launch_x_load_batch_gen(Context& ctx, c2<T>* base, const BatchLoader
   raise_lds(kern, smem);
   ProfScope ps(ctx, sizeof(T) == 8 ? KC_FFT_STRIDED64 : KC_FFT_STRIDED, bytes);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwork)), dim3(FFT_THREADS), smem, ctx.stream, base,
-                     ctx.g.nmesh, load, ctx_twiddles<T>(ctx, N, +1), ctx.g.n[1], ctx.g.n[2],
+                     ctx.g.nmesh, load, gen_twiddles<T>(ctx, P, +1), ctx.g.n[1], ctx.g.n[2],
                      pr, kcut2, work, P);
   TRVG_LAUNCH_CHECK();
 }
@@ -647,13 +654,13 @@ static void launch_x_sjl_gen(Context& ctx, c2<T>* base, int nt, const double2* s
     raise_lds(kern, smem);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(FFT_THREADS), smem, ctx.stream, base, g.nmesh,
                        nt, src, ctx.tab, g, sp.dev(), r, ell, m,
-                       ctx_twiddles<T>(ctx, N, +1), P);
+                       gen_twiddles<T>(ctx, P, +1), P);
   } else {
     auto kern = fft_x_sjl_multi_gen<T, false>;
     raise_lds(kern, smem);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(FFT_THREADS), smem, ctx.stream, base, g.nmesh,
                        nt, src, ctx.tab, g, sp.dev(), r, ell, m,
-                       ctx_twiddles<T>(ctx, N, +1), P);
+                       gen_twiddles<T>(ctx, P, +1), P);
   }
   TRVG_LAUNCH_CHECK();
 }

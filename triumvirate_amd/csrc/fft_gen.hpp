@@ -18,6 +18,15 @@
 // loader pass and the j_l multi-field x pass, each also over (field, block)
 // work lists.
 //
+// FP32 lines are FP32 in memory and LDS, but their register butterflies are
+// formed in FP64, with FP64 twiddles.  A rounded constant (a twiddle, cos 2 pi
+// / 5) is the same for every line, so its error does not average out over a
+// mesh as that of rounded data does: with FP32 butterflies an FP32 window
+// function of 96^3 was off by 1.7e-7 (every output formed directly: 1.2e-7),
+// with FP64 ones by 2.2e-8.  FP64 products issue at the rate of FP32 ones; the
+// strided pass of 200^3 FP32 takes 62 us (FP32 butterflies 51, every output
+// formed directly 142).
+//
 // What bounded them: integer divisions (three or more per element, some in
 // 64 bits, and four per output of every stage) and p LDS reads per output.
 // Indexes now come from one multiplication with a reciprocal of the plan,
@@ -83,12 +92,14 @@ inline GenPlan make_gen_plan(int n) {
   return p;
 }
 
-// Dynamic LDS of a pass: the line buffer (padded stride N + 1; two of them
-// where outputs are formed directly) and the N twiddles.
+// Dynamic LDS of a pass: the N twiddles (FP64, of a length whose outputs are
+// formed directly in the lines' precision) and the line buffer (padded stride
+// N + 1; two of them for the latter).
 template <typename T>
 inline size_t gen_smem(int n) {
   const GenPlan p = make_gen_plan(n);
-  return size_t((p.direct ? 2 : 1) * p.nl * (n + 1) + n) * sizeof(c2<T>);
+  return size_t(p.direct ? 2 : 1) * p.nl * (n + 1) * sizeof(c2<T>) +
+         size_t(n) * (p.direct ? sizeof(c2<T>) : sizeof(double2));
 }
 
 // cos and sin of 2 pi k / p at compile time (Taylor series about 0 after
@@ -140,8 +151,8 @@ __device__ __forceinline__ void dft_odd(c2<T>* x, T sgn) {
 
 // Stage s of radix P over the buffer `a`, in place.
 template <typename T, int P>
-__device__ __forceinline__ void gen_stage(c2<T>* a, const c2<T>* W, const GenPlan& pl, int s,
-                                          int Ns, int nl, T sgn) {
+__device__ __forceinline__ void gen_stage(c2<T>* a, const double2* W, const GenPlan& pl, int s,
+                                          int Ns, int nl, double sgn) {
   constexpr int NB = (GEN_ELEMS / P + FFT_THREADS - 1) / FFT_THREADS;
   const int N = pl.n, LS = N + 1, Np = N / P, total = nl * Np;
   const int tstep = N / (Ns * P);
@@ -155,11 +166,17 @@ __device__ __forceinline__ void gen_stage(c2<T>* a, const c2<T>* W, const GenPla
     const int jq = pl.by_ns[s].div(j), k = j - jq * Ns;
     const c2<T>* src = a + line * LS + j;
     d[b] = line * LS + jq * Ns * P + k;
-    x[b][0] = src[0];
+    double2 y[P];
 #pragma unroll
-    for (int q = 1; q < P; q++) x[b][q] = cmul<T>(src[q * Np], W[q * k * tstep]);
-    if constexpr (P % 2 == 0) dft_reg<T, P>(x[b], sgn);
-    else dft_odd<T, P>(x[b], sgn);
+    for (int q = 0; q < P; q++) {
+      const c2<T> v = src[q * Np];
+      y[q] = dmk(v.x, v.y);
+      if (q > 0) y[q] = dmul(y[q], W[q * k * tstep]);
+    }
+    if constexpr (P % 2 == 0) dft_reg<double, P>(y, sgn);
+    else dft_odd<double, P>(y, sgn);
+#pragma unroll
+    for (int q = 0; q < P; q++) x[b][q] = mk<T>(T(y[q].x), T(y[q].y));
   }
   __syncthreads();
 #pragma unroll
@@ -174,23 +191,25 @@ __device__ __forceinline__ void gen_stage(c2<T>* a, const c2<T>* W, const GenPla
 // The nl lines of a (line stride N + 1) are transformed; returns the buffer
 // (a, or b of the direct lengths) holding the result.  Ends with a barrier.
 template <typename T>
-__device__ __forceinline__ c2<T>* lds_fft_gen(c2<T>* a, c2<T>* b, const c2<T>* W,
+__device__ __forceinline__ c2<T>* lds_fft_gen(c2<T>* a, c2<T>* b, const void* tw,
                                               const GenPlan& P, int nl, int sign) {
   const int N = P.n, LS = N + 1;
   int Ns = 1;
   if (!P.direct) {
+    const double2* W = static_cast<const double2*>(tw);
     for (int s = 0; s < P.nst; s++) {
       switch (P.radix[s]) {
-        case 2: gen_stage<T, 2>(a, W, P, s, Ns, nl, T(sign)); break;
-        case 3: gen_stage<T, 3>(a, W, P, s, Ns, nl, T(sign)); break;
-        case 4: gen_stage<T, 4>(a, W, P, s, Ns, nl, T(sign)); break;
-        case 5: gen_stage<T, 5>(a, W, P, s, Ns, nl, T(sign)); break;
-        default: gen_stage<T, 7>(a, W, P, s, Ns, nl, T(sign)); break;
+        case 2: gen_stage<T, 2>(a, W, P, s, Ns, nl, sign); break;
+        case 3: gen_stage<T, 3>(a, W, P, s, Ns, nl, sign); break;
+        case 4: gen_stage<T, 4>(a, W, P, s, Ns, nl, sign); break;
+        case 5: gen_stage<T, 5>(a, W, P, s, Ns, nl, sign); break;
+        default: gen_stage<T, 7>(a, W, P, s, Ns, nl, sign); break;
       }
       Ns *= P.radix[s];
     }
     return a;
   }
+  const c2<T>* W = static_cast<const c2<T>*>(tw);
   const int total = nl * N;
   for (int s = 0; s < P.nst; s++) {
     const int p = P.radix[s];
@@ -221,17 +240,27 @@ __device__ __forceinline__ c2<T>* lds_fft_gen(c2<T>* a, c2<T>* b, const c2<T>* W
   return a;
 }
 
+// LDS of a pass, and its twiddles copied there from the table `tw`.
 template <typename T>
 struct GenSmem {
   c2<T>* a;
   c2<T>* b;
-  c2<T>* W;
+  void* W;
   __device__ explicit GenSmem(const GenPlan& P) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    const int LS = P.n + 1;
-    a = reinterpret_cast<c2<T>*>(smem_raw);
-    b = a + P.nl * LS;
-    W = P.direct ? b + P.nl * LS : b;
+    W = smem_raw;
+    a = reinterpret_cast<c2<T>*>(smem_raw +
+                                 P.n * (P.direct ? sizeof(c2<T>) : sizeof(double2)));
+    b = a + P.nl * (P.n + 1);
+  }
+  __device__ __forceinline__ void fill(const GenPlan& P, const void* tw) const {
+    if (P.direct) {
+      for (int m = threadIdx.x; m < P.n; m += FFT_THREADS)
+        static_cast<c2<T>*>(W)[m] = static_cast<const c2<T>*>(tw)[m];
+    } else {
+      for (int m = threadIdx.x; m < P.n; m += FFT_THREADS)
+        static_cast<double2*>(W)[m] = static_cast<const double2*>(tw)[m];
+    }
   }
 };
 
@@ -251,10 +280,10 @@ struct GenSplit {
 // z pass (contiguous lines, line index = i n1 + j) with a loader.
 template <typename T, class Loader>
 __device__ __forceinline__ void fft_z_block_gen(c2<T>* __restrict__ data, const Loader& load,
-                                const c2<T>* __restrict__ tw, int n1, long long nlines,
+                                const void* __restrict__ tw, int n1, long long nlines,
                                 int sign, const Prune& pr, const GenPlan& P,
                                 long long blk) {
-  const int N = P.n, LS = N + 1;
+  const int N = P.n;
   GenSmem<T> sm(P);
   const long long line0 = blk * P.nl;
   if (line0 >= nlines) return;
@@ -269,7 +298,7 @@ __device__ __forceinline__ void fft_z_block_gen(c2<T>* __restrict__ data, const 
     }
     if (!any) return;
   }
-  for (int m = threadIdx.x; m < N; m += FFT_THREADS) sm.W[m] = tw[m];
+  sm.fill(P, tw);
   // Threads past the end repeat the last element (no branch, so the loads
   // stay in flight together).
   c2<T> v[GEN_MAXE];
@@ -298,7 +327,7 @@ __device__ __forceinline__ void fft_z_block_gen(c2<T>* __restrict__ data, const 
 
 template <typename T, class Loader>
 __global__ void __launch_bounds__(FFT_THREADS)
-fft_pass_z_gen(c2<T>* __restrict__ data, Loader load, const c2<T>* __restrict__ tw,
+fft_pass_z_gen(c2<T>* __restrict__ data, Loader load, const void* __restrict__ tw,
                int n1, long long nlines, int sign, Prune pr, GenPlan P) {
   fft_z_block_gen<T>(data, load, tw, n1, nlines, sign, pr, P, blockIdx.x);
 }
@@ -306,7 +335,7 @@ fft_pass_z_gen(c2<T>* __restrict__ data, Loader load, const c2<T>* __restrict__ 
 template <typename T, class BatchLoader>
 __global__ void __launch_bounds__(FFT_THREADS)
 fft_pass_z_batch_gen(c2<T>* __restrict__ base, long long fstride, BatchLoader load,
-                     const c2<T>* __restrict__ tw, int n1, long long nlines, int sign,
+                     const void* __restrict__ tw, int n1, long long nlines, int sign,
                      Prune pr, const double* __restrict__ kcut2,
                      const int2* __restrict__ work, GenPlan P) {
   const int2 wk = work[blockIdx.x];
@@ -320,7 +349,7 @@ fft_pass_z_batch_gen(c2<T>* __restrict__ base, long long fstride, BatchLoader lo
 // element stride S) with the pruning modes of fft_strided_block.
 template <typename T>
 __device__ __forceinline__ void fft_strided_block_gen(
-    c2<T>* __restrict__ data, const c2<T>* __restrict__ tw, long long S,
+    c2<T>* __restrict__ data, const void* __restrict__ tw, long long S,
     long long outer_stride, long long inner, long long nlines, int sign, const Prune& pr,
     int prune_mode, const GenPlan& P, long long blk) {
   const int N = P.n, LS = N + 1;
@@ -338,7 +367,7 @@ __device__ __forceinline__ void fft_strided_block_gen(
     }
     if (!any) return;
   }
-  for (int m = threadIdx.x; m < N; m += FFT_THREADS) sm.W[m] = tw[m];
+  sm.fill(P, tw);
   // Element (n, l): consecutive threads take consecutive lines (nl of them,
   // which is P.nl but in the last block).
   const bool whole = nl == P.nl;
@@ -391,7 +420,7 @@ __device__ __forceinline__ void fft_strided_block_gen(
 
 template <typename T>
 __global__ void __launch_bounds__(FFT_THREADS)
-fft_pass_strided_gen(c2<T>* __restrict__ data, const c2<T>* __restrict__ tw, long long S,
+fft_pass_strided_gen(c2<T>* __restrict__ data, const void* __restrict__ tw, long long S,
                      long long outer_stride, long long inner, long long nlines, int sign,
                      Prune pr, int prune_mode, GenPlan P) {
   fft_strided_block_gen<T>(data, tw, S, outer_stride, inner, nlines, sign, pr, prune_mode, P,
@@ -401,7 +430,7 @@ fft_pass_strided_gen(c2<T>* __restrict__ data, const c2<T>* __restrict__ tw, lon
 template <typename T>
 __global__ void __launch_bounds__(FFT_THREADS)
 fft_pass_strided_batch_gen(c2<T>* __restrict__ base, long long fstride,
-                           const c2<T>* __restrict__ tw, long long S, long long outer_stride,
+                           const void* __restrict__ tw, long long S, long long outer_stride,
                            long long inner, long long nlines, int sign, Prune pr,
                            const double* __restrict__ kcut2, const int2* __restrict__ work,
                            int prune_mode, GenPlan P) {
@@ -418,7 +447,7 @@ fft_pass_strided_batch_gen(c2<T>* __restrict__ base, long long fstride,
 template <typename T, class Loader>
 __device__ __forceinline__ void fft_x_load_block_gen(c2<T>* __restrict__ data,
                                      const Loader& load,
-                                     const c2<T>* __restrict__ tw, int n1, int n2,
+                                     const void* __restrict__ tw, int n1, int n2,
                                      const Prune& pr, const GenPlan& P, long long blk) {
   const int N = P.n, LS = N + 1;
   GenSmem<T> sm(P);
@@ -436,7 +465,7 @@ __device__ __forceinline__ void fft_x_load_block_gen(c2<T>* __restrict__ data,
     }
     if (!any) return;
   }
-  for (int m = threadIdx.x; m < N; m += FFT_THREADS) sm.W[m] = tw[m];
+  sm.fill(P, tw);
   const bool whole = nl == P.nl;
   auto split = [&](int idx, int& n, int& l) {
     n = whole ? P.by_nl.div(idx) : idx / nl;
@@ -465,7 +494,7 @@ __device__ __forceinline__ void fft_x_load_block_gen(c2<T>* __restrict__ data,
 template <typename T, class BatchLoader>
 __global__ void __launch_bounds__(FFT_THREADS)
 fft_pass_x_load_batch_gen(c2<T>* __restrict__ base, long long fstride, BatchLoader load,
-                          const c2<T>* __restrict__ tw, int n1, int n2, Prune pr,
+                          const void* __restrict__ tw, int n1, int n2, Prune pr,
                           const double* __restrict__ kcut2, const int2* __restrict__ work,
                           GenPlan P) {
   const int2 wk = work[blockIdx.x];

@@ -392,7 +392,7 @@ __global__ void __launch_bounds__(FFT_THREADS)
 fft_x_sjl_multi_gen(c2<T>* __restrict__ base, long long fstride, int nt,
                     const double2* __restrict__ src, AxisTables tab, Geom geo,
                     SplineDev sj, const double* __restrict__ r, int ell, int m,
-                    const c2<T>* __restrict__ tw, GenPlan P) {
+                    const void* __restrict__ tw, GenPlan P) {
   constexpr int MAXE = GEN_MAXE;
   const int N = P.n, LS = N + 1;
   GenSmem<T> sm(P);
@@ -402,7 +402,7 @@ fft_x_sjl_multi_gen(c2<T>* __restrict__ base, long long fstride, int nt,
   if (id0 >= S) return;
   const int nl = int(min((long long)P.nl, S - id0));
   const int total = nl * N;
-  for (int q = threadIdx.x; q < N; q += FFT_THREADS) sm.W[q] = tw[q];
+  sm.fill(P, tw);
   const GenSplit jk(id0, n2);
   const bool whole = nl == P.nl;
   auto split = [&](int idx) { return whole ? P.by_nl.div(idx) : idx / nl; };
