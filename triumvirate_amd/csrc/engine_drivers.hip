@@ -508,10 +508,11 @@ static void launch_pair_mfma(Context& ctx, unsigned grid, size_t smem, const flo
   TRVG_LAUNCH_CHECK();
 }
 
-// pair_reduce of FP32 fields with a complex A side on the matrix cores
-// (k_pair_mfma).
-static void pair_reduce_mfma(Context& ctx, const float2* FA, int na, const float2* FB, int nbf, bool b_packed, const float2* G,
-                             PairPart want, const std::vector<int2>& pairs,
+// pair_reduce of a table of FP32 fields with a complex A side on the matrix
+// cores (k_pair_mfma).
+static void pair_reduce_mfma(Context& ctx, const float2* FA, int na, const float2* FB,
+                             int nbf, bool b_packed, const float2* G, PairPart want,
+                             const std::vector<int2>& pairs,
                              std::function<void(std::vector<cplx>&&)> sink) {
   const int mode = b_packed ? 1 : 0;
   const bool full = want == PAIR_FULL;
@@ -671,9 +672,8 @@ static auto pair_list_kernel(int np) {
   }
 }
 
-// pair_reduce of a short list (k_pair_list; FP32 only with two real sides), in
-// equal batches of at most
-// eight pairs.
+// pair_reduce of a short list (k_pair_list), in equal batches of at most eight
+// pairs.
 template <typename T>
 static void pair_reduce_list(Context& ctx, const c2<T>* FA, bool a_packed, const c2<T>* FB,
                              bool b_packed, const c2<T>* G, const std::vector<int2>& pairs,
@@ -700,7 +700,6 @@ static void pair_reduce_list(Context& ctx, const c2<T>* FA, bool a_packed, const
     ProfScope ps(ctx, KC_PAIR_REDUCE,
                  double(ma.size() + mb.size() + batches) * double(nm) * sizeof(c2<T>));
     auto kern = pair_list_kernel<T, 2>(per);
-    if constexpr (sizeof(T) == 8)
       if (!a_packed) kern = b_packed ? pair_list_kernel<T, 1>(per) : pair_list_kernel<T, 0>(per);
     hipLaunchKernelGGL(kern, dim3(batches, grid), dim3(256), 0, ctx.stream, FA, FB, G, nm,
                        dl.get(), np, part.get());
@@ -737,20 +736,22 @@ static void pair_reduce(Context& ctx, const c2<T>* FA, int na, bool a_packed,
   }
   if (a_packed && !g_real)
     throw Error(TRVG_ERR_INTERNAL, "Real shell pairs need a real G field.");
+  // Lists with about one pair per field (diagonal, off-diagonal, row) are
+  // streamed: they read no mesh twice, and every product is added in FP64.
+  // Fuller tables reuse staged rows.  (FP32 lists with a complex side on the
+  // matrix cores, 20 diagonal pairs at 256^3: 541 us against 680 streamed, but
+  // with 32 cells summed in FP32 where the vector kernel, 778 us, had four.)
+  if (!pairs.empty() && int(pairs.size()) <= na + nbf) {
+    pair_reduce_list<T>(ctx, FA, a_packed, FB, b_packed, G, pairs, std::move(sink));
+    return;
+  }
   if constexpr (sizeof(T) == 4) {
     if (!a_packed) {
       pair_reduce_mfma(ctx, FA, na, FB, nbf, b_packed, G, want, pairs, std::move(sink));
       return;
     }
   }
-  // Lists with about one pair per field (diagonal, off-diagonal, row) are
-  // streamed: they read no mesh twice.  Fuller tables reuse staged rows (the
-  // 16 x 16 tables of FP32 complex sides above are at the memory rate for
-  // lists too: 20 diagonal pairs at 256^3 307 us there, 347 us streamed).
-  if (!pairs.empty() && int(pairs.size()) <= na + nbf)
-    pair_reduce_list<T>(ctx, FA, a_packed, FB, b_packed, G, pairs, std::move(sink));
-  else
-    pair_reduce_lds<T>(ctx, FA, na, a_packed, FB, nbf, b_packed, G, pairs, std::move(sink));
+  pair_reduce_lds<T>(ctx, FA, na, a_packed, FB, nbf, b_packed, G, pairs, std::move(sink));
 }
 
 struct TwoPt {

@@ -2205,8 +2205,11 @@ namespace trvg {
 // direct to LDS and double buffered.  Each of the four waves takes a quarter
 // of a chunk's cells and every tile; lane (i = lane % 16, k = lane / 16)
 // reads field i of a tile at two cells per 16-byte access, which feed two
-// matrix instructions.  Sums of one chunk (32 cells) stay in FP32 and are
-// then added in FP64.
+// matrix instructions.  FP32 sums are added in FP64 every 8 cells for tables of
+// one tile, every 32 for larger ones (the vector kernel: 2 to 8 up to 16
+// fields a side, 12 to 32 above).  Every 8 throughout costs 2 x 2 tiles a third
+// (complex with real, 256^3: 892 -> 1222 us) for an error that the fields'
+// own hides: 24 bins of a survey, 192^3, 3.0e-8 -> 2.4e-8.
 //
 // MODE 0: complex sides; 1: B side real, two per mesh.  FULL: complex sums;
 // else real parts only (of the sums, or with `rot` of -i times them), half
@@ -2242,6 +2245,7 @@ k_pair_mfma(const float2* __restrict__ FA, int na, const float2* __restrict__ FB
   using L = PairLds<float>;
   constexpr int NC = FULL ? 2 : 1;              // sums per pair
   constexpr int SUMS = NTA * NTB * PM_TILE * PM_TILE;
+  constexpr int CHAIN = NTA * NTB == 1 ? 8 : L::LDC / 4;   // cells summed in FP32
   extern __shared__ __attribute__((aligned(16))) char smp_raw[];
   const int MA = pair_rows_a(MODE, na);
   const int MB = same ? 0 : pair_rows_b(MODE, nbf);
@@ -2293,13 +2297,7 @@ k_pair_mfma(const float2* __restrict__ FA, int na, const float2* __restrict__ FB
 
   // This wave's quarter of the chunk in `buf`.
   auto reduce = [&](const char* buf) {
-    f32x4 acc[NC][NTA][NTB];
-#pragma unroll
-    for (int n = 0; n < NC; n++)
-#pragma unroll
-      for (int a = 0; a < NTA; a++)
-#pragma unroll
-        for (int b = 0; b < NTB; b++) acc[n][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[NC][NTA][NTB] = {};
     const char* gbuf = buf + (size_t)(MA + MB) * L::ROWB;
 #pragma unroll
     for (int c8 = 0; c8 < L::LDC / 4; c8 += 8) {
@@ -2365,15 +2363,18 @@ k_pair_mfma(const float2* __restrict__ FA, int na, const float2* __restrict__ FB
           }
         }
       }
+      if (c8 + 8 < CHAIN) continue;
+#pragma unroll
+      for (int n = 0; n < NC; n++)
+#pragma unroll
+        for (int a = 0; a < NTA; a++)
+#pragma unroll
+          for (int b = 0; b < NTB; b++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) sum[n][a][b][r] += double(acc[n][a][b][r]);
+            acc[n][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
     }
-#pragma unroll
-    for (int n = 0; n < NC; n++)
-#pragma unroll
-      for (int a = 0; a < NTA; a++)
-#pragma unroll
-        for (int b = 0; b < NTB; b++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) sum[n][a][b][r] += double(acc[n][a][b][r]);
   };
 
   int cur = 0;
