@@ -88,29 +88,34 @@ struct Prune {
 // Register-resident DFTs.
 // ---------------------------------------------------------------------------
 
-// cos(pi k / 16) for k in [0, 16] (k > 8 by symmetry).
-__host__ __device__ constexpr double cos_pi16(int k) {
-  return k > 8   ? -cos_pi16(16 - k)
-         : k == 0 ? 1.0
-         : k == 1 ? 0.9807852804032304
-         : k == 2 ? 0.9238795325112867
-         : k == 3 ? 0.8314696123025452
-         : k == 4 ? 0.7071067811865476
-         : k == 5 ? 0.5555702330196023
-         : k == 6 ? 0.38268343236508984
-         : k == 7 ? 0.19509032201612833
-                  : 0.0;
+// cos and sin of 2 pi k / p at compile time (Taylor series about 0 after
+// reduction to |x| <= pi).
+constexpr double cx_series(double x, bool odd) {
+  double term = odd ? x : 1., sum = term;
+  for (int i = odd ? 2 : 1; i < 60; i += 2) {
+    term *= -x * x / (double(i) * double(i + 1));
+    sum += term;
+  }
+  return sum;
+}
+constexpr double cx_turn(int k, int p) {
+  const int r = k % p;
+  return 2. * 3.14159265358979323846 * double(2 * r > p ? r - p : r) / double(p);
 }
 
-// d * e^{sgn i pi k / 16} for k in [0, 16); k is a constant after
-// unrolling, so the trivial factors (1, +-i) cost no multiplications.
+// d * e^{sgn i pi k / 4} for k in [0, 4); k is a constant after unrolling, so
+// the trivial factors (1, +-i) cost no multiplications.  FP32: cos pi / 4 in two
+// parts, as the twiddles below.
 template <typename T>
-__device__ __forceinline__ c2<T> rot_pi16(c2<T> d, int k, T sgn) {
+__device__ __forceinline__ c2<T> rot_pi4(c2<T> d, int k, T sgn) {
   if (k == 0) return d;
-  if (k == 8) return mk<T>(-sgn * d.y, sgn * d.x);
-  const T c = T(cos_pi16(k));
-  const T sn = sgn * T(cos_pi16(8 - k > 0 ? 8 - k : k - 8));
-  return mk<T>(d.x * c - d.y * sn, d.x * sn + d.y * c);
+  const c2<T> r = mk<T>(-sgn * d.y, sgn * d.x);   // d * sgn i
+  if (k == 2) return r;
+  const c2<T> s = k == 1 ? cadd<T>(d, r) : csub<T>(r, d);
+  constexpr T c = T(0.70710678118654752440);
+  constexpr T l = T(0.70710678118654752440 - double(c));
+  if (sizeof(T) == 4) return mk<T>(s.x * c + s.x * l, s.y * c + s.y * l);
+  return mk<T>(s.x * c, s.y * c);
 }
 
 // One decimation-in-frequency radix-2 stage of length LEN over v[0, R),
@@ -125,7 +130,7 @@ struct DifStages {
       for (int j = 0; j < H; j++) {
         const c2<T> a = v[s + j], b = v[s + j + H];
         v[s + j] = cadd<T>(a, b);
-        v[s + j + H] = rot_pi16<T>(csub<T>(a, b), (32 / LEN) * j, sgn);
+        v[s + j + H] = rot_pi4<T>(csub<T>(a, b), (8 / LEN) * j, sgn);
       }
     }
     DifStages<T, R, H>::run(v, sgn);
@@ -142,10 +147,10 @@ __host__ __device__ constexpr int bitrev(int k, int bits) {
 __host__ __device__ constexpr int ilog2c(int r) { return r <= 1 ? 0 : 1 + ilog2c(r / 2); }
 
 // v <- DFT_R(v): X[k] = sum_n v[n] e^{sgn 2 pi i n k / R}, natural order in
-// and out (R a power of two <= 32, held in registers).
+// and out (R a power of two <= 8, held in registers).
 template <typename T, int R>
 __device__ __forceinline__ void dft_reg(c2<T>* v, T sgn) {
-  static_assert(R >= 1 && R <= 32 && (R & (R - 1)) == 0, "register DFT size");
+  static_assert(R >= 1 && R <= 8 && (R & (R - 1)) == 0, "register DFT size");
   DifStages<T, R, R>::run(v, sgn);
   c2<T> o[R];
 #pragma unroll
@@ -192,9 +197,44 @@ constexpr int fft_line_stride(int n, int nl) {
   return base + ((want - base) % banks + banks) % banks;
 }
 
+// FP32 twiddles of the stages up to span 16 are kept in two parts: these stages
+// use a handful of angles (multiples of 2 pi / 64) over and over, so that their
+// rounding scales every mode alike (e^{i pi / 4} alone is short by 1.7e-8)
+// and does not average out over a mesh.  With single parts a transform of 64^3
+// to 256^3 comes out short by 6e-8, a bispectrum by 1.8e-7; with both parts by
+// less than 3e-9 and 2 to 4e-8.  Strided pass of 256^3 42.5 -> 43.8 us, z pass 48.8
+// -> 52.0.  Second parts of cos and sin 2 pi m / 64:
+constexpr int FFT_LO = 64;
+struct TwiddleLo {
+  float2 v[FFT_LO];
+};
+constexpr TwiddleLo make_twiddle_lo() {
+  TwiddleLo t{};
+  for (int m = 0; m < FFT_LO; m++) {
+    const double c = cx_series(cx_turn(m, FFT_LO), false), s = cx_series(cx_turn(m, FFT_LO), true);
+    t.v[m].x = float(c - double(float(c)));
+    t.v[m].y = float(s - double(float(s)));
+  }
+  return t;
+}
+static __device__ const TwiddleLo twiddle_lo = make_twiddle_lo();
+
+// x w, and for FP32 the second part l of w.
+template <typename T>
+__device__ __forceinline__ c2<T> tw_mul(c2<T> x, c2<T> w, c2<T> l) {
+  return mk<T>(fma(x.x, w.x, fma(-x.y, w.y, fma(x.x, l.x, -x.y * l.y))),
+               fma(x.x, w.y, fma(x.y, w.x, fma(x.x, l.y, x.y * l.x))));
+}
+
 // Twiddles in LDS, per stage (span Ns, radix R) the (R - 1) Ns factors
 // w^{q k N / (Ns R)}, k fastest: N - 2^LR of them (the spans add up so).  tw:
 // e^{sign 2 pi i m / N}.
+template <typename T>
+__device__ __forceinline__ void fft_fill_lo(c2<T>* lo, int t, T sgn) {
+  if constexpr (sizeof(T) == 4) {
+    if (t < FFT_LO) lo[t] = mk<T>(twiddle_lo.v[t].x, sgn * twiddle_lo.v[t].y);
+  }
+}
 template <typename T, int LOGN, int LR = FFT_LR, int LD = LR>
 __device__ __forceinline__ void fft_fill_twiddles(c2<T>* W, const c2<T>* __restrict__ tw,
                                                   int t, int nt) {
@@ -213,8 +253,8 @@ __device__ __forceinline__ void fft_fill_twiddles(c2<T>* W, const c2<T>* __restr
 // threads are one wave's, which needs no barrier.  AGAIN: LDS may still be
 // read by an earlier transform of the workgroup.
 template <typename T, int LOGN, int LR, bool WAVE, bool AGAIN, int LD = 0>
-__device__ __forceinline__ void fft_stages(c2<T> (&v)[8], c2<T>* lb, const c2<T>* W, int j,
-                                           T sgn) {
+__device__ __forceinline__ void fft_stages(c2<T> (&v)[8], c2<T>* lb, const c2<T>* W,
+                                           const c2<T>* lo, int j, T sgn) {
   constexpr int N = 1 << LOGN, M = N / 8, Ns = 1 << LD;
   constexpr int R = 1 << (LOGN - LD >= LR ? LR : LOGN - LD);
   constexpr int NB = 8 / R;                 // butterflies per thread
@@ -235,7 +275,11 @@ __device__ __forceinline__ void fft_stages(c2<T> (&v)[8], c2<T>* lb, const c2<T>
 #pragma unroll
     for (int q = 0; q < R; q++) {
       x[q] = v[b + q * NB];
-      if (LD > 0 && q > 0) x[q] = cmul<T>(x[q], W[(q - 1) * Ns + k]);
+      if (LD > 0 && q > 0) {
+        const c2<T> w = W[(q - 1) * Ns + k];
+        if constexpr (sizeof(T) == 4 && Ns <= 16) x[q] = tw_mul<T>(x[q], w, lo[q * k * (FFT_LO / (Ns * R))]);
+        else x[q] = cmul<T>(x[q], w);
+      }
     }
     dft_reg<T, R>(x, sgn);
 #pragma unroll
@@ -253,7 +297,7 @@ __device__ __forceinline__ void fft_stages(c2<T> (&v)[8], c2<T>* lb, const c2<T>
     sync();
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] = lb[fft_pad(j + e * M)];
-    fft_stages<T, LOGN, LR, WAVE, AGAIN, LD + LR>(v, lb, LD > 0 ? W + (R - 1) * Ns : W, j, sgn);
+    fft_stages<T, LOGN, LR, WAVE, AGAIN, LD + LR>(v, lb, LD > 0 ? W + (R - 1) * Ns : W, lo, j, sgn);
   }
 }
 
@@ -262,7 +306,8 @@ __device__ __forceinline__ void fft_stages(c2<T> (&v)[8], c2<T>* lb, const c2<T>
 constexpr size_t FFT_LDS = 160 * 1024;
 template <typename T>
 constexpr size_t fft_lds(int n, int nl, int ls) {
-  return size_t(nl * ls + n - (1 << FFT_LR)) * sizeof(c2<T>);
+  return size_t(nl * ls + n - (1 << FFT_LR)) * sizeof(c2<T>) +
+         (sizeof(T) == 4 ? FFT_LO * sizeof(float2) : 0);
 }
 template <typename T>
 constexpr size_t strided_lds(int logn, int nt) {
@@ -335,7 +380,9 @@ __device__ __forceinline__ void fft_z_block(c2<T>* __restrict__ data, const Load
     }
     if (!any) return;
   }
+  c2<T>* lo = W + N - (1 << FFT_LR);
   fft_fill_twiddles<T, LOGN>(W, tw, t, FFT_THREADS);
+  fft_fill_lo<T>(lo, t, T(sign));
   c2<T> v[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) {
@@ -346,7 +393,7 @@ __device__ __forceinline__ void fft_z_block(c2<T>* __restrict__ data, const Load
     if (HeavyLoader<Loader>::value && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   }
   if (M <= 64) __syncthreads();   // the twiddles; the stages stay within a wave
-  fft_stages<T, LOGN, FFT_LR, (M <= 64), false>(v, buf + l * LS, W, j, T(sign));
+  fft_stages<T, LOGN, FFT_LR, (M <= 64), false>(v, buf + l * LS, W, lo, j, T(sign));
   if (!valid) return;
   c2<T>* out = data + line * N + j;
 #pragma unroll
@@ -412,7 +459,9 @@ __device__ __forceinline__ void fft_strided_block(
     if (!any) return;
     line_in = valid && pr.p2(int(prune_mode == 1 ? slice : col));
   }
+  c2<T>* lo = W + N - (1 << FFT_LR);
   fft_fill_twiddles<T, LOGN>(W, tw, t, strided_threads<T, LOGN>());
+  fft_fill_lo<T>(lo, t, T(sign));
   c2<T>* p = data + (long long)slice * outer_stride + col + (long long)j * S;
   const long long step = (long long)M * S;
   c2<T> v[8];
@@ -428,7 +477,7 @@ __device__ __forceinline__ void fft_strided_block(
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] = ld_mesh<T>(p + e * step);
   }
-  fft_stages<T, LOGN, FFT_LR, false, false>(v, buf + l * LS, W, j, T(sign));
+  fft_stages<T, LOGN, FFT_LR, false, false>(v, buf + l * LS, W, lo, j, T(sign));
   if (!line_in) return;
 #pragma unroll
   for (int e = 0; e < 8; e++) st_mesh<T>(p + e * step, v[e]);
@@ -489,7 +538,9 @@ __device__ __forceinline__ void fft_x_load_block(c2<T>* __restrict__ data,
     if (!any) return;
     line_in = line_in && pr.p1(k, j);
   }
+  c2<T>* lo = W + N - (1 << FFT_LR);
   fft_fill_twiddles<T, LOGN>(W, tw, t, strided_threads<T, LOGN>());
+  fft_fill_lo<T>(lo, t, T(sign));
   c2<T> v[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) {
@@ -497,7 +548,7 @@ __device__ __forceinline__ void fft_x_load_block(c2<T>* __restrict__ data,
     v[e] = line_in ? load(id + (long long)n * S, n, j, k) : mk<T>(T(0), T(0));
     if (HeavyLoader<Loader>::value && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   }
-  fft_stages<T, LOGN, FFT_LR, false, false>(v, buf + l * LS, W, r0, T(sign));
+  fft_stages<T, LOGN, FFT_LR, false, false>(v, buf + l * LS, W, lo, r0, T(sign));
   if (!line_in) return;
 #pragma unroll
   for (int e = 0; e < 8; e++) st_mesh<T>(data + id + (long long)(r0 + e * M) * S, v[e]);

@@ -102,21 +102,6 @@ inline size_t gen_smem(int n) {
          size_t(n) * (p.direct ? sizeof(c2<T>) : sizeof(double2));
 }
 
-// cos and sin of 2 pi k / p at compile time (Taylor series about 0 after
-// reduction to |x| <= pi).
-constexpr double cx_series(double x, bool odd) {
-  double term = odd ? x : 1., sum = term;
-  for (int i = odd ? 2 : 1; i < 60; i += 2) {
-    term *= -x * x / (double(i) * double(i + 1));
-    sum += term;
-  }
-  return sum;
-}
-constexpr double cx_turn(int k, int p) {
-  const int r = k % p;
-  return 2. * 3.14159265358979323846 * double(2 * r > p ? r - p : r) / double(p);
-}
-
 // x <- DFT_P(x), P odd: with s_q = x_q + x_{P-q}, d_q = x_q - x_{P-q},
 // X_{r, P-r} = x_0 + sum_q cos(2 pi q r / P) s_q +- i sgn sum_q sin(..) d_q.
 template <typename T, int P>

@@ -337,7 +337,9 @@ fft_x_sjl_multi(c2<T>* __restrict__ base, long long fstride, int nt,
   const long long S = (long long)n1 * n2;
   const long long id = xcd_block(blockIdx.x, gridDim.x) * NL + l;
   const bool valid = id < S;
+  c2<T>* lo = W + N - (1 << FFT_LR);
   fft_fill_twiddles<T, LOGN, SJL_LR>(W, tw, t, strided_threads<T, LOGN>());
+  fft_fill_lo<T>(lo, t, T(1));
   // Per element: y_lm src / W / V in the working precision (FP32 fields
   // take j_l and the product in FP32) and |k|.
   c2<T> fac[8];
@@ -376,7 +378,7 @@ fft_x_sjl_multi(c2<T>* __restrict__ base, long long fstride, int nt,
       v[e] = PACKED ? mk<T>(j0 * fac[e].x - j1 * fac[e].y, j0 * fac[e].y + j1 * fac[e].x)
                     : mk<T>(j0 * fac[e].x, j0 * fac[e].y);
     }
-    fft_stages<T, LOGN, SJL_LR, false, true>(v, buf + l * LS, W, r0, T(1));
+    fft_stages<T, LOGN, SJL_LR, false, true>(v, buf + l * LS, W, lo, r0, T(1));
     if (!valid) continue;
     c2<T>* out = base + (long long)f * fstride + id;
 #pragma unroll
