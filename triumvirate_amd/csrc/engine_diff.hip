@@ -32,19 +32,18 @@ struct DiffGroup {
   DevArray<c2<T>> D, G, F;
 };
 
-// D(k) of the mesh, then per group G and the shells.
+// D(k) of the mesh, then per group of `bins` G and the shells.
 template <typename T>
 std::vector<DiffGroup<T>> diff_groups(Context& ctx, const trvg_binning& kb, const T* mesh,
-                                      const std::vector<int>& nmodes) {
+                                      const std::vector<int>& nmodes,
+                                      const std::vector<int>& bins) {
   const Geom g = ctx.g;
-  std::vector<int> all(kb.num_bins);
-  for (int b = 0; b < kb.num_bins; b++) all[b] = b;
   DevArray<c2<T>> D(g.nmesh);
   fft3d<T>(ctx, D.get(), LoadReal<T>{mesh, T(g.vol_cell)}, -1, double(g.nmesh) * sizeof(T));
   std::vector<DiffGroup<T>> out;
-  for (const MeshGroup& gr : plan_mesh_groups(g, kb, all, all, true, sizeof(c2<T>))) {
+  for (const MeshGroup& gr : plan_mesh_groups(g, kb, bins, bins, true, sizeof(c2<T>))) {
     DiffGroup<T> d;
-    d.bins = gr.pairs;   // pair b is bin b with itself
+    for (int q : gr.pairs) d.bins.push_back(bins[q]);   // a bin pairs with itself
     d.coarse = gr.coarse;
     d.g = gr.coarse ? mesh_of(g, gr.n) : g;
     d.nt = (int(d.bins.size()) + 1) / 2;
@@ -74,7 +73,9 @@ std::vector<double> diff_bispec_forward(Context& ctx, const trvg_binning& kb,
                                         std::vector<int>& nmodes) {
   ShellStats ss = shell_stats(ctx, kb);
   nmodes = ss.nmodes;
-  std::vector<DiffGroup<T>> groups = diff_groups<T>(ctx, kb, mesh, ss.nmodes);
+  std::vector<int> bins(kb.num_bins);
+  for (int b = 0; b < kb.num_bins; b++) bins[b] = b;
+  std::vector<DiffGroup<T>> groups = diff_groups<T>(ctx, kb, mesh, ss.nmodes, bins);
   std::vector<const double*> h;
   for (DiffGroup<T>& d : groups) {
     const int nv = 2 * d.nt;
@@ -107,7 +108,12 @@ void diff_bispec_backward(Context& ctx, const trvg_binning& kb, double norm,
   const long long nm = g.nmesh;
   const int nb = kb.num_bins;
   ShellStats ss = shell_stats(ctx, kb);
-  std::vector<DiffGroup<T>> groups = diff_groups<T>(ctx, kb, mesh, ss.nmodes);
+  // Bins that contribute: none costs transforms, or spreads a mesh's infinities
+  // and NaN, without a cotangent.
+  std::vector<int> bins;
+  for (int b = 0; b < nb; b++)
+    if (grad_bk[b] != 0. && ss.nmodes[b] != 0) bins.push_back(b);
+  std::vector<DiffGroup<T>> groups = diff_groups<T>(ctx, kb, mesh, ss.nmodes, bins);
   DevArray<c2<T>> acc(nm);
   const unsigned grid = grid_for(ctx, nm);
   hipLaunchKernelGGL((k_zero<T>), dim3(grid), dim3(RED_THREADS), 0, ctx.stream,
@@ -126,7 +132,6 @@ void diff_bispec_backward(Context& ctx, const trvg_binning& kb, double norm,
     for (size_t i = 0; i < d.bins.size(); i++) {
       const int b = d.bins[i];
       const double n = double(ss.nmodes[b]);
-      if (grad_bk[b] == 0. || ss.nmodes[b] == 0) continue;
       a[i] = grad_bk[b] * norm * d.g.vol_cell / (n * n);
       slot[b] = int(i);
     }
