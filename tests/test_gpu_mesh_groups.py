@@ -149,3 +149,49 @@ def test_bins_without_a_cotangent_are_left_out(prec):
     got, want = grad(b, [0., 0., 0., 2., 0.], x), grad(one, [2.], x)
     tol = 1e-12 if prec == 'fp64' else 1e-6   # pruning: rounding of empty modes
     assert (got - want).abs().max() < tol * want.abs().max()
+
+
+def test_gradient_memory_does_not_grow_with_bins():
+    """42 bins up to the Nyquist wavenumber of 256^3 FP64 (256 MiB a complex
+    mesh): values and gradient add up from calls on 6 bins each, which take
+    their shells in one slab, and the engine holds less than 3 GiB (all shells at
+    once: 21 meshes, 5.3 GiB, beside the spectrum, G and the gradient)."""
+    import torch
+    from triumvirate_amd import _lib
+    from triumvirate_amd.autodiff import DifferentiableBispectrum
+    from triumvirate_amd.dataobjs import Binning
+    print("gradient memory", flush=True)
+    lib, ng, box = _lib.load(), [256] * 3, [1000.] * 3
+    kf = 2 * np.pi / 1000.
+    edges = np.linspace(1.1 * kf, 127.1 * kf, 43)
+    g = torch.Generator(device='cuda').manual_seed(4)
+    mesh = torch.randn(ng, generator=g, dtype=torch.float64, device='cuda')
+    c = torch.randn(42, generator=g, dtype=torch.float64, device='cuda')
+
+    def call(lo, hi):
+        b = Binning('fourier', 'lin')
+        b.set_custom_bins(edges[lo:hi + 1])
+        x = mesh.clone().requires_grad_(True)
+        bk = DifferentiableBispectrum(box, ng, b, 'cic', 'fp64').from_mesh(x)
+        bk.backward(c[lo:hi])
+        return bk.detach(), x.grad
+
+    call(0, 1)                                   # what stays for the process
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    assert lib.trvg_release_workspace() == 0
+    free, own = torch.cuda.mem_get_info()[0], torch.cuda.memory_reserved()
+    bk, grad = call(0, 42)
+    torch.cuda.synchronize()
+    held = free - torch.cuda.mem_get_info()[0] - (torch.cuda.memory_reserved() - own)
+    print(f"  {held / 2 ** 30:.2f} GiB", flush=True)
+    assert held < 3 << 30
+    want_g, want = torch.zeros_like(grad), []
+    for lo in range(0, 42, 6):
+        v, d = call(lo, lo + 6)
+        want.append(v)
+        want_g += d
+    want = torch.cat(want)
+    assert (bk - want).abs().max() < 1e-12 * want.abs().max()
+    assert (grad - want_g).abs().max() < 1e-12 * want_g.abs().max()
+    assert lib.trvg_release_workspace() == 0

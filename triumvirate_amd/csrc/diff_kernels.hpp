@@ -219,11 +219,12 @@ k_f2g_packed(const c2<T>* __restrict__ F, const c2<T>* __restrict__ G, long long
 }
 
 // Cotangents of the shell fields and of G: mesh p of the packed slab F
-// becomes 2 (a_2p F_2p + i a_2p+1 F_2p+1) G, and mesh nt sum_b a_b F_b^2.
+// becomes 2 (a_2p F_2p + i a_2p+1 F_2p+1) G; sum_b a_b F_b^2 goes to the complex
+// mesh gk if there is one, else is added to the real mesh gG.
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
 k_cotangents(c2<T>* __restrict__ F, const c2<T>* __restrict__ G, long long n, int nt,
-             const double* __restrict__ a) {
+             const double* __restrict__ a, c2<T>* __restrict__ gk, T* __restrict__ gG) {
   for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < n;
        c += (long long)gridDim.x * blockDim.x) {
     const double g = double(G[c].x);
@@ -234,20 +235,22 @@ k_cotangents(c2<T>* __restrict__ F, const c2<T>* __restrict__ G, long long n, in
       s += a0 * x * x + a1 * y * y;
       F[(long long)p * n + c] = mk<T>(T(2. * a0 * x * g), T(2. * a1 * y * g));
     }
-    F[(long long)nt * n + c] = mk<T>(T(s), T(0));
+    if (gk) gk[c] = mk<T>(T(s), T(0));
+    else gG[c] = T(double(gG[c]) + s);
   }
 }
 
 // acc(k) += [the spectrum of the cotangent of the bin holding k, + scale
-// times that of G's cotangent] / W(k), from the transformed slab of
-// k_cotangents on the mesh `c` to the full mesh `g` (window tables of g).
-// Bin b of the group is real field slot[b] of the slab (-1: not in it):
+// times that of G's cotangent, gk (may be null)] / W(k), from the transformed
+// slab of k_cotangents on the mesh `c` to the full mesh `g` (window tables of
+// g).  Bin b of the batch is real field slot[b] of the slab (-1: not in it):
 // with P = FFT[u + i v], u(k) = (P(k) + P(-k)^*) / 2 and v(k) = (P(k) -
 // P(-k)^*) / 2i.  Each cell of c is one cell of g, so the update is
 // race-free.
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
-k_adj_acc(c2<T>* __restrict__ acc, const c2<T>* __restrict__ P, int nt, Geom g, Geom c,
+k_adj_acc(c2<T>* __restrict__ acc, const c2<T>* __restrict__ P,
+          const c2<T>* __restrict__ gk, Geom g, Geom c,
           AxisTables tab, const double* __restrict__ edge, int nb,
           const int* __restrict__ slot, double scale) {
   for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < c.nmesh;
@@ -266,8 +269,12 @@ k_adj_acc(c2<T>* __restrict__ acc, const c2<T>* __restrict__ P, int nt, Geom g, 
       k[a] = grid_coord(ix[a], c.n[a], c.dk[a]);
     }
     if (edge_mode) continue;   // beyond the products of any bin
-    const c2<T> t = P[(long long)nt * c.nmesh + q];
-    double re = scale * double(t.x), im = scale * double(t.y);
+    double re = 0., im = 0.;
+    if (gk) {
+      const c2<T> t = gk[q];
+      re = scale * double(t.x);
+      im = scale * double(t.y);
+    }
     const int b = find_bin(edge, nb, mag2_exact(k[0], k[1], k[2]));
     const int s = b < 0 ? -1 : slot[b];
     if (s >= 0) {
