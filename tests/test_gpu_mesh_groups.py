@@ -195,3 +195,48 @@ def test_gradient_memory_does_not_grow_with_bins():
     assert (bk - want).abs().max() < 1e-12 * want.abs().max()
     assert (grad - want_g).abs().max() < 1e-12 * want_g.abs().max()
     assert lib.trvg_release_workspace() == 0
+
+
+def test_mixed_forms_share_bounded_slabs():
+    """Multipoles of several forms in one call, where diagonal and row pairs go
+    to smaller meshes: each equals its own call, in both precisions, and the
+    slabs kept stay those of the full mesh, three of 20 complex fields
+    (128^3 FP64: 1.9 GiB; the (2, m) of all terms together are four and a
+    half), whatever the number of meshes."""
+    import torch
+    from triumvirate_amd import _lib
+    from triumvirate_amd.dataobjs import Binning
+    from triumvirate_amd.threept import (compute_bispec_in_gpp_box,
+                                         compute_bispec_multipoles)
+    print("mixed forms", flush=True)
+    lib = _lib.load()
+    kf = 2 * np.pi / 1000.
+    b = Binning('fourier', 'lin', bin_min=1.1 * kf, bin_max=60. * kf, num_bins=20)
+    ps = cf.make_test_paramset(assignment='cic', ngrid=dict.fromkeys('xyz', 128),
+                               boxsize=dict.fromkeys('xyz', 1000.))
+    mps = [((2, 2, 0), 'full'), ((0, 0, 0), 'diag'), ((2, 0, 2), 'row', 3),
+           ((1, 1, 0), 'off-diag', 2)]
+
+    def data():
+        return P.uniform_box_catalogue(20000, 1000., seed=5, weights=False)
+
+    for prec, tol in (('fp64', 1e-12), ('fp32', 1e-5)):
+        torch.cuda.synchronize()
+        assert lib.trvg_release_workspace() == 0
+        free = torch.cuda.mem_get_info()[0]
+        got = compute_bispec_multipoles(data(), multipoles=mps[:2], binning=b,
+                                        paramset=ps, precision=prec)
+        held = (free - torch.cuda.mem_get_info()[0]) / 2 ** 30
+        print(f"  {prec} {held:.2f} GiB", flush=True)
+        if prec == 'fp64':
+            assert held < 2.8
+        got = compute_bispec_multipoles(data(), multipoles=mps, binning=b,
+                                        paramset=ps, precision=prec)
+        for mp, res in zip(mps, got):
+            one = compute_bispec_in_gpp_box(
+                data(), degrees=mp[0], form=mp[1], idx_bin=mp[2] if len(mp) > 2 else None,
+                binning=b, paramset=ps, precision=prec)
+            for key in ('bk_raw', 'bk_shot'):
+                err = np.max(np.abs(res[key] - one[key])) / np.max(np.abs(one[key]))
+                assert err < tol, (mp, key, err)
+    assert lib.trvg_release_workspace() == 0

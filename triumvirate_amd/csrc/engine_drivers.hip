@@ -1158,15 +1158,21 @@ struct ShellSlab {
   }
 };
 
+// At most `per_mesh` slabs of one mesh are kept, and cells_max complex cells
+// over all meshes (the slabs of the pair under way are always held): the smaller
+// meshes of some multipoles share the memory that per_mesh slabs of the full
+// mesh took.
 template <typename T>
 class SlabCache {
  public:
-  explicit SlabCache(size_t capacity = 2) : cap_(capacity < 2 ? 2 : capacity) {}
+  explicit SlabCache(size_t per_mesh = 2, size_t cells_max = SIZE_MAX)
+      : per_mesh_(per_mesh), cells_max_(cells_max) {}
 
   // Returns a slab of (l, m) covering `bins`, building it with
   // make(slab_base, bins) if needed (field q of the slab at
   // slab_base + q * nmesh, or component q % 2 of mesh q / 2 when packed);
-  // evicts the least recently used slab other than `keep` when full.
+  // evicts the least recently used slabs other than `keep` where room is
+  // needed.
   template <class Make>
   ShellSlab<T>* get(Context& ctx, int l, int m, const std::vector<int>& bins,
                     int nb, const ShellSlab<T>* keep, bool packed, Make&& make) {
@@ -1177,22 +1183,39 @@ class SlabCache {
         entries_.push_back(std::move(e));
         return entries_.back().get();
       }
-    if (entries_.size() >= cap_) {
-      for (size_t i = 0; i < entries_.size(); i++)
-        if (entries_[i].get() != keep) {
-          entries_.erase(entries_.begin() + i);
-          break;
-        }
-    }
+    const size_t cells =
+        size_t(ctx.g.nmesh) * (packed ? (bins.size() + 1) / 2 : bins.size());
     auto e = std::make_unique<ShellSlab<T>>();
+    auto here = [&](const ShellSlab<T>& q) {
+      return q.n[0] == ctx.g.n[0] && q.n[1] == ctx.g.n[1] && q.n[2] == ctx.g.n[2];
+    };
+    size_t same = 0, held = cells;
+    for (const auto& q : entries_) {
+      same += here(*q);
+      held += q->data.size();
+    }
+    for (size_t i = 0; i < entries_.size();) {
+      ShellSlab<T>& q = *entries_[i];
+      const bool full = same >= per_mesh_ && here(q);
+      if (&q == keep || !(full || held > cells_max_)) {
+        i++;
+        continue;
+      }
+      same -= here(q);
+      held -= q.data.size();
+      // The kernels that read it are still queued: the new slab takes its place
+      // in stream order, or it goes back to the shared pool once they are done.
+      if (!e->data.get() && q.data.size() == cells) e->data = std::move(q.data);
+      else TRVG_HIP(hipStreamSynchronize(ctx.stream));
+      entries_.erase(entries_.begin() + i);
+    }
     e->ell = l;
     e->m = m;
     for (int a = 0; a < 3; a++) e->n[a] = ctx.g.n[a];
     e->index.assign(nb, -1);
     e->nfields = int(bins.size());
     e->packed = packed;
-    const long long nm = ctx.g.nmesh;
-    e->data.reset((size_t)nm * (packed ? (bins.size() + 1) / 2 : bins.size()));
+    if (!e->data.get()) e->data.reset(cells);
     make(e->data.get(), bins);
     for (size_t q = 0; q < bins.size(); q++) e->index[bins[q]] = int(q);
     entries_.push_back(std::move(e));
@@ -1200,7 +1223,7 @@ class SlabCache {
   }
 
  private:
-  size_t cap_;
+  size_t per_mesh_, cells_max_;
   std::vector<std::unique_ptr<ShellSlab<T>>> entries_;
 };
 
@@ -1298,20 +1321,29 @@ std::vector<Result> run_bispec_multi(Context& ctx, const DeviceCatalogue& d,
   cplx t_sbar(0., 0.);
   // Meshes of each multipole's pair sums, and dn00(k) / W(k) on them.
   std::vector<std::vector<MeshGroup>> plans;
-  size_t ngroups = 1;
   long long nm_coarse = 0;
+  size_t slab_max = 0;   // cells of the largest slab that the full mesh would take
   for (const Multipole& mp : mps) {
     std::vector<int> ra, cb;
     pair_bins(mp.shape, nb, mp.idx_bin, ra, cb);
     const bool split = mp.shape != TRVG_SHAPE_FULL && mp.shape != TRVG_SHAPE_TRIU;
     plans.push_back(plan_mesh_groups(g, kb, ra, cb, split, sizeof(c2<T>)));
-    ngroups = std::max(ngroups, plans.back().size());
     for (const MeshGroup& gr : plans.back())
       if (gr.coarse) nm_coarse = std::max(nm_coarse, mesh_of(g, gr.n).nmesh);
+    trvg_params p = ctx.p;
+    p.ell1 = mp.ell1; p.ell2 = mp.ell2; p.ELL = mp.ELL;
+    auto cells = [&](int l, int m, size_t fields) {
+      return size_t(nm) * (real_shells(l, m) ? (fields + 1) / 2 : fields);
+    };
+    for (const Term& tm : enumerate_terms(p, survey)) {
+      slab_max = std::max(slab_max, cells(p.ell1, tm.m1, distinct(ra).size()));
+      slab_max = std::max(slab_max, cells(p.ell2, tm.m2, distinct(cb).size()));
+    }
   }
   std::map<std::vector<int>, DevArray<double2>> coarse00;
   DevArray<double2> coarseLM;
-  SlabCache<T> slabs((mps.size() > 1 ? 3 : 2) * ngroups);
+  const size_t per_mesh = mps.size() > 1 ? 3 : 2;
+  SlabCache<T> slabs(per_mesh, per_mesh * slab_max);
   auto make_shell = [&](const double2* src, int l, int mm) {
     return [&, src, l, mm](c2<T>* base, const std::vector<int>& bins) {
       shell_slab_ifft<T, double>(ctx, base, src, kb, bins, ss.nmodes, l, mm, real_shells(l, mm));
