@@ -268,10 +268,11 @@ def test_equal_terms_sum_in_catalogue_order(n, term):
     assert be.norm_particles(CatalogueView(*cat.columns()), 1.) == 1. / want
 
 
-def test_host_sums_and_forked_process():
-    """Normalisation sums over worker threads against numpy (rounding of 7e4
-    terms: 1e-12), and the same sums in a forked process, which has no
-    worker threads."""
+@pytest.mark.parametrize('n', [70001, 3 * 65536, 1000003])
+def test_host_sums_and_forked_process(n):
+    """Normalisation sums over worker threads against numpy (rounding of 1e6
+    terms: 1e-12), and the same value bit by bit in a forked process, which
+    has no worker threads."""
     import multiprocessing as mp
     from triumvirate_amd import _lib
     from triumvirate_amd import threept as T
@@ -279,7 +280,6 @@ def test_host_sums_and_forked_process():
     from triumvirate_amd._abi import CatalogueView
     be = T.CLibBackend(_lib.load())
     rng = np.random.default_rng(5)
-    n = 70001
     nz, ws, wc = rng.uniform(0.5, 1.5, (3, n))
     cat = ParticleCatalogue(*rng.uniform(0., 100., (3, n)), nz=nz, ws=ws, wc=wc)
 
@@ -294,4 +294,4 @@ def test_host_sums_and_forked_process():
     p.start()
     p.join(60)
     assert p.exitcode == 0
-    assert abs(q.get() / want - 1.) < 1e-12
+    assert q.get() == norm()

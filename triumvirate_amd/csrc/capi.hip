@@ -211,10 +211,13 @@ double repeated_sum(double t, long long n) {
   return s;
 }
 
-// sum_p f(ws_p, wc_p, nz_p) over a host catalogue: one partial sum per
-// worker thread, added in their order.  Equal terms (uniform density, unit
-// weights), whose rounding errors add up instead of cancelling, give the sum
-// in catalogue order.
+// sum_p f(ws_p, wc_p, nz_p) over a host catalogue: one partial sum per SUM_PART
+// particles, added in their order, so that the value does not depend on the
+// number of worker threads.  Equal terms (uniform density, unit weights),
+// whose rounding errors add up instead of cancelling, give the sum in
+// catalogue order.
+constexpr long long SUM_PART = 1 << 16;
+
 template <class F>
 double particle_sum(const trvg_catalogue* c, F f) {
   if (c == nullptr || c->x == nullptr)
@@ -226,18 +229,23 @@ double particle_sum(const trvg_catalogue* c, F f) {
   };
   if (c->ntotal < 1) return 0.;
   const double t0 = term(0);
-  std::vector<double> part(host_threads(), 0.);
-  std::vector<char> equal(host_threads(), 1);
-  host_ranges(c->ntotal, [&](long long b, long long e, int t) {
-    double s = 0.;
-    bool eq = true;
-    for (long long i = b; i < e; i++) {
-      const double v = term(i);
-      s += v;
-      eq &= v == t0;
+  const long long parts = (c->ntotal + SUM_PART - 1) / SUM_PART;
+  std::vector<double> part(parts, 0.);
+  std::vector<char> equal(parts, 1);
+  host_ranges(c->ntotal, [&](long long b, long long e, int) {
+    // The parts that begin in [b, e).
+    for (long long q = (b + SUM_PART - 1) / SUM_PART; q * SUM_PART < e; q++) {
+      double s = 0.;
+      bool eq = true;
+      const long long end = std::min(c->ntotal, (q + 1) * SUM_PART);
+      for (long long i = q * SUM_PART; i < end; i++) {
+        const double v = term(i);
+        s += v;
+        eq &= v == t0;
+      }
+      part[q] = s;
+      equal[q] = eq;
     }
-    part[t] = s;
-    equal[t] = eq;
   });
   if (std::count(equal.begin(), equal.end(), 0) == 0 && t0 > 0. && std::isnormal(t0) &&
       t0 < 1e300)
