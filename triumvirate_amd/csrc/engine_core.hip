@@ -297,8 +297,16 @@ const double* ones_table(int dev) {
 bool pow2(int n) { return (n & (n - 1)) == 0; }
 
 // Cost of a pass along an axis relative to one of power-of-two length (FP64
-// strided passes, 200^3 against 256^3: 8.6 against 5.1 ps per cell).
-double axis_cost(int n) { return pow2(n) && n <= 1024 ? 1. : 1.7; }
+// strided passes, ps per cell: 256^3 5.1, 200^3 8.5, and 208^3, whose factor 13
+// takes the direct form, 23).  FP32 passes of 200^3 and 208^3 stand at 3 and 5,
+// but their own weights choose no better: the 144x120x180 row splits over two
+// meshes, 1.04 -> 1.10 ms of kernels.
+double axis_cost(int n) {
+  if (pow2(n) && n <= 1024) return 1.;
+  for (int q : {2, 3, 5, 7})
+    while (n % q == 0) n /= q;
+  return n == 1 ? 1.7 : 4.5;
+}
 
 // The cheapest mesh with m >= 2 K + 2 per axis (none longer than the full
 // mesh's): per axis the next power of two, the next even length with no
