@@ -211,41 +211,46 @@ double repeated_sum(double t, long long n) {
   return s;
 }
 
+// sum f(ws, wc, nz) over particles [b, e) of a catalogue; equal: whether every
+// term is t0.  A loop of its own, which the compiler splits by absent columns
+// (inside the loop over parts it did not: 8e6 unit weights 2.4 -> 15 ms).
+template <class F>
+double part_sum(const trvg_catalogue& c, F f, long long b, long long e, double t0, char& equal) {
+  const double *ws = c.ws, *wc = c.wc, *nz = c.nz;
+  const long long st = c.stride > 0 ? c.stride : 1;
+  double s = 0.;
+  bool eq = true;
+  for (long long i = b; i < e; i++) {
+    const double v = f(ws ? ws[i * st] : 1., wc ? wc[i * st] : 1., nz ? nz[i * st] : 0.);
+    s += v;
+    eq &= v == t0;
+  }
+  equal = eq;
+  return s;
+}
+
 // sum_p f(ws_p, wc_p, nz_p) over a host catalogue: one partial sum per SUM_PART
 // particles, added in their order, so that the value does not depend on the
 // number of worker threads.  Equal terms (uniform density, unit weights),
 // whose rounding errors add up instead of cancelling, give the sum in
 // catalogue order.
-constexpr long long SUM_PART = 1 << 16;
+constexpr long long SUM_PART = 1 << 12;
 
 template <class F>
 double particle_sum(const trvg_catalogue* c, F f) {
   if (c == nullptr || c->x == nullptr)
     throw Error(TRVG_ERR_DATA, "Particle data are uninitialised.");
-  const long long st = c->stride > 0 ? c->stride : 1;
-  auto term = [&](long long i) {
-    return f(c->ws ? c->ws[i * st] : 1., c->wc ? c->wc[i * st] : 1.,
-             c->nz ? c->nz[i * st] : 0.);
-  };
   if (c->ntotal < 1) return 0.;
-  const double t0 = term(0);
+  char first;
+  const double t0 = part_sum(*c, f, 0, 1, 0., first);
   const long long parts = (c->ntotal + SUM_PART - 1) / SUM_PART;
   std::vector<double> part(parts, 0.);
   std::vector<char> equal(parts, 1);
   host_ranges(c->ntotal, [&](long long b, long long e, int) {
     // The parts that begin in [b, e).
-    for (long long q = (b + SUM_PART - 1) / SUM_PART; q * SUM_PART < e; q++) {
-      double s = 0.;
-      bool eq = true;
-      const long long end = std::min(c->ntotal, (q + 1) * SUM_PART);
-      for (long long i = q * SUM_PART; i < end; i++) {
-        const double v = term(i);
-        s += v;
-        eq &= v == t0;
-      }
-      part[q] = s;
-      equal[q] = eq;
-    }
+    for (long long q = (b + SUM_PART - 1) / SUM_PART; q * SUM_PART < e; q++)
+      part[q] = part_sum(*c, f, q * SUM_PART, std::min(c->ntotal, (q + 1) * SUM_PART), t0,
+                         equal[q]);
   });
   if (std::count(equal.begin(), equal.end(), 0) == 0 && t0 > 0. && std::isnormal(t0) &&
       t0 < 1e300)

@@ -169,7 +169,7 @@ __device__ __forceinline__ void dft_reg(c2<T>* v, T sgn) {
 // Against radix-4 stages with the line in LDS throughout, a transform
 // crosses LDS 6 times instead of 10 (N = 256), starts from the loads
 // themselves and ends in the stores, and masked rows are loaded together
-// instead of one after the other.  Radix 4 (47 registers in FP32, 72 in
+// instead of one after the other.  Radix 4 (51 registers in FP32, 72 in
 // FP64 for N = 256: eight and seven waves per SIMD) beats radix 8 (90 and
 // 126), whose fewer exchanges do not make up for the waves.  Measured,
 // before and after, in us: strided pass of 256^3 FP32 63 -> 48, FP64 103 ->
@@ -183,7 +183,8 @@ __device__ __forceinline__ void dft_reg(c2<T>* v, T sgn) {
 constexpr int FFT_LR = 2;
 
 // LDS position of element n: one element of padding per eight, which spreads
-// the writes of the first stage (stride 8) over all banks.
+// the writes of the first stage (stride 4, or 8 of radix-8 stages) over all
+// banks.
 __host__ __device__ __forceinline__ constexpr int fft_pad(int n) { return n + n / 8; }
 
 // LDS elements between the lines of a workgroup: nl lanes in a row belong to

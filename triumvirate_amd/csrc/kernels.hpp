@@ -1442,7 +1442,7 @@ __device__ __forceinline__ long long tile_cell(const Geom& g, const int o0[3], i
 // CPLX: complex weights (a second LDS block); SHADOW: the half-cell-shifted
 // pass of interlacing (stencils reach one cell further: a 12^3 block).  The
 // shadow pass used to go straight to the mesh, ORDER^3 global atomics per
-// particle (PCS on 256^3: 15 ms per 2e6 particles, 67 ms of the 111 ms of an
+// particle (PCS on 256^3: 4.46 ms per 2e6 particles, 67 ms of the 111 ms of an
 // interlaced quadrupole); binned like the main pass it takes 0.23 ms.
 template <typename T, int ORDER, bool CPLX, bool SHADOW>
 __global__ void __launch_bounds__(256)
